@@ -204,28 +204,69 @@ __global__ __launch_bounds__(256) void attn_mask_ranges_kernel(const uint8_t* __
         }
       }
     }
-  } else if (b < nqb) {
-    const int r0 = b * kAttnRangeBlock, nr = min(kAttnRangeBlock, L - r0);
-    for (int r = 0; r < nr; ++r) {
-      const uint8_t* row = mask + static_cast<int64_t>(r0 + r) * S;
-#pragma unroll 8
-      for (int col = threadIdx.x; col < S; col += 256) {
-        if (row[col] != 0) {
-          lo = min(lo, col);
-          hi = max(hi, col);
+  } else {
+    // Rows at any byte. Row r's part of a block (the whole row of a query block, 64 columns of a
+    // key block) lies in the aligned 16-byte chunks that overlap it; a chunk's bytes outside the
+    // part are cleared, and a chunk not wholly inside the mask (at its ends) is read by bytes. The
+    // threads take the (row, chunk) pairs of the block in order, kU loads in flight each, none of
+    // them under a branch. Byte reads of one row after another, a round trip each, took 59 us for
+    // four 1000 x 1000 masks; this takes 12 us (MI355X).
+    constexpr int kU = 4;
+    const bool keys = b >= nqb;
+    const int c0 = keys ? (b - nqb) * kAttnRangeBlock : 0, n = keys ? min(kAttnRangeBlock, S - c0) : S;
+    const int r0 = keys ? 0 : b * kAttnRangeBlock, rows = keys ? L : min(kAttnRangeBlock, L - r0);
+    const int cpr = (n + 15) / 16 + 1;   // at most this many chunks overlap a part
+    const int64_t bytes = static_cast<int64_t>(L) * S;
+    const int mis = static_cast<int>(reinterpret_cast<uintptr_t>(mask) & 15u);
+    const int64_t first_in = (16 - mis) & 15, last_in = (bytes + mis) / 16 * 16 - mis - 16;   // chunks wholly inside
+    int64_t r = threadIdx.x / cpr;
+    int ch = threadIdx.x % cpr;
+    const int step_r = 256 / cpr, step_ch = 256 % cpr;
+    while (r < rows) {
+      uint4 w[kU];
+      int64_t at[kU], part[kU];
+      int row[kU];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        row[u] = static_cast<int>(min(r, static_cast<int64_t>(rows - 1)));
+        part[u] = static_cast<int64_t>(r0 + row[u]) * S + c0;
+        at[u] = r < rows ? (part[u] + mis) / 16 * 16 - mis + 16 * static_cast<int64_t>(ch) : bytes;
+        w[u] = make_uint4(0, 0, 0, 0);
+        if (last_in >= first_in)   // uniform
+          w[u] = *reinterpret_cast<const uint4*>(mask + min(max(at[u], first_in), last_in));
+        ch += step_ch;
+        r += step_r;
+        if (ch >= cpr) {
+          ch -= cpr;
+          ++r;
         }
       }
-    }
-  } else {
-    const int c0 = (b - nqb) * kAttnRangeBlock, nc = min(kAttnRangeBlock, S - c0);
-    const int col = threadIdx.x % kAttnRangeBlock;
-    if (col < nc) {
-#pragma unroll 8
-      for (int r = threadIdx.x / kAttnRangeBlock; r < L; r += 256 / kAttnRangeBlock) {
-        if (mask[static_cast<int64_t>(r) * S + c0 + col] != 0) {
-          lo = min(lo, r);
-          hi = max(hi, r);
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        const int from = static_cast<int>(max(part[u] - at[u], int64_t{0}));             // bytes of the chunk inside
+        const int to = static_cast<int>(min(part[u] + n - at[u], int64_t{16}));          // the part: from .. to - 1
+        if (to <= from) continue;
+        uint32_t v[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+        if (at[u] < first_in || at[u] > last_in) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            v[i] = 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (4 * i + e >= from && 4 * i + e < to) v[i] |= static_cast<uint32_t>(mask[at[u] + 4 * i + e]) << (8 * e);
+          }
         }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {   // of word i, bytes f .. t - 1 are inside
+          const int f = min(max(from - 4 * i, 0), 4), t = min(max(to - 4 * i, 0), 4);
+          v[i] &= (f == 4 ? 0u : 0xffffffffu << (8 * f)) & (t == 4 ? 0xffffffffu : (1u << (8 * t)) - 1u);
+        }
+        int first, last;
+        chunk_bounds(make_uint4(v[0], v[1], v[2], v[3]), first, last);
+        if (last < 0) continue;
+        const int col = static_cast<int>(at[u] - part[u]);
+        lo = min(lo, keys ? row[u] : col + first);
+        hi = max(hi, keys ? row[u] : col + last);
       }
     }
   }

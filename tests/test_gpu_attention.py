@@ -330,6 +330,21 @@ def test_mask_ranges_kernel(L, S):
     assert got.cpu().tolist()[:len(_ranges_reference(mask))] == _ranges_reference(mask)
 
 
+# Masks whose rows start at any byte (S not a multiple of 16, a mask at an offset in its buffer):
+# the first and last admissible byte of a block in partly covered 16-byte chunks, at the mask's ends
+# and in masks smaller than a chunk.
+@pytest.mark.parametrize("offset", [0, 1, 7, 15])
+@pytest.mark.parametrize("L,S", [(1, 3), (3, 5), (2, 17), (65, 15), (5, 1000), (200, 129), (128, 64), (1030, 1)])
+def test_mask_ranges_kernel_at_any_byte(L, S, offset):
+    g = torch.Generator().manual_seed(17 * L + S + offset)
+    for keep in (1.0, 0.02, 0.0):
+        mask = torch.rand(L, S, generator=g) < keep
+        buffer = torch.ones(L * S + offset + 33, dtype=torch.bool)   # admissible bytes around the mask
+        buffer[offset:offset + L * S] = mask.flatten()
+        got = _ops._mask_ranges(buffer.cuda()[offset:offset + L * S].view(L, S), L, S)
+        assert got.cpu().tolist()[:len(_ranges_reference(mask))] == _ranges_reference(mask), keep
+
+
 # Sliding windows much narrower than the sequence: the kernels skip the key blocks outside each
 # query block's range (and, in the pipelined kernel, keep one fully masked block for a query block
 # with no admissible key).
