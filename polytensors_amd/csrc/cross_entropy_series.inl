@@ -22,6 +22,15 @@ namespace pt {
 
 constexpr int kCeThreads = 256;
 
+// Elements before the first 16-byte boundary at or after p, at most n: the vectors of a row start
+// there.
+template <typename T>
+__device__ __forceinline__ int64_t ce_head(const T* p, int64_t n) {
+  const int64_t head = static_cast<int64_t>((16u - static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p) & 15u)) & 15u) /
+                       static_cast<int64_t>(sizeof(T));
+  return head < n ? head : n;
+}
+
 template <typename A, int K>
 __device__ __forceinline__ void accumulate_element(A x0, const A (&xk)[K + 1], A m, A (&S)[K + 1]) {
   const A p = exp_fast(x0 - m);
@@ -52,11 +61,16 @@ __device__ __forceinline__ void rescale(A& m, A new_m, A (&S)[K + 1]) {
 // One block of THREADS threads per row. Logits are read with non-temporal
 // 16-byte loads (each byte is read once; streaming them past the caches lifts
 // the kernel from about 74% to 86% of HBM peak on MI355X), two vectors per
-// order in flight per thread and iteration. With CAP every logit series is
-// first replaced by its softcap cap * tanh(z / cap) (series_math.h), on the fly.
+// order in flight per thread and iteration. A row may start at any element
+// (a class count or row stride that is no multiple of a vector): its vectors
+// start at order 0's first 16-byte boundary, and the loads take the other
+// orders at any element. 4096 x 32001 bfloat16 logits at degree 3 (1.05 GB):
+// 352 us by elements, 218 us by unaligned vectors from the row's start, 173 us
+// (6.1 TB/s) from the boundary. With CAP every logit series is first replaced
+// by its softcap cap * tanh(z / cap) (series_math.h), on the fly.
 template <typename T, int K, int THREADS, bool CAP>
 __global__ __launch_bounds__(THREADS) void cross_entropy_series_row_kernel(
-    CPtrs<T> z, int64_t rows, int64_t classes, int64_t row_stride, bool vec_ok,
+    CPtrs<T> z, int64_t rows, int64_t classes, int64_t row_stride,
     const int64_t* __restrict__ target, int64_t ignore_index, MPtrs<typename AccOf<T>::type> loss,
     MPtrs<typename AccOf<T>::type> lse, typename AccOf<T>::type cap, typename AccOf<T>::type inv_cap) {
   using A = typename AccOf<T>::type;
@@ -72,58 +86,55 @@ __global__ __launch_bounds__(THREADS) void cross_entropy_series_row_kernel(
 #pragma unroll
   for (int k = 0; k <= K; ++k) S[k] = A(0);
 
-  int64_t scalar_from = 0;
-  if (vec_ok) {
-    constexpr int U = 2;
-    const int64_t nvec = classes / V;
-    int64_t j = threadIdx.x;
-    for (; j + (U - 1) * THREADS < nvec; j += U * THREADS) {
-      Vec<T, V> a[U][K + 1];
+  constexpr int U = 2;
+  const int64_t head = ce_head(z.p[0] + base, classes), nvec = (classes - head) / V;
+  int64_t j = threadIdx.x;
+  for (; j + (U - 1) * THREADS < nvec; j += U * THREADS) {
+    Vec<T, V> a[U][K + 1];
 #pragma unroll
-      for (int u = 0; u < U; ++u)
+    for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int k = 0; k <= K; ++k) a[u][k] = load_vec_nt<T, V>(z.p[k] + base + (j + u * THREADS) * V);
-      A x[U][V][K + 1];
-      A hi = kNegInf;
+      for (int k = 0; k <= K; ++k) a[u][k] = load_vec_nt_any<T, V>(z.p[k] + base + head + (j + u * THREADS) * V);
+    A x[U][V][K + 1];
+    A hi = kNegInf;
 #pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int e = 0; e < V; ++e) {
-#pragma unroll
-          for (int k = 0; k <= K; ++k) x[u][e][k] = to_acc(a[u][k].v[e]);
-          if constexpr (CAP) softcap_series<A, K>(x[u][e], cap, inv_cap);
-          hi = fmax(hi, x[u][e][0]);
-        }
-      rescale<A, K>(m, hi, S);
-      if (m != kNegInf) {
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-          for (int e = 0; e < V; ++e) accumulate_element<A, K>(x[u][e][0], x[u][e], m, S);
-      }
-    }
-    for (; j < nvec; j += THREADS) {
-      Vec<T, V> a[K + 1];
-#pragma unroll
-      for (int k = 0; k <= K; ++k) a[k] = load_vec_nt<T, V>(z.p[k] + base + j * V);
-      A x[V][K + 1];
-      A hi = kNegInf;
+    for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int e = 0; e < V; ++e) {
 #pragma unroll
-        for (int k = 0; k <= K; ++k) x[e][k] = to_acc(a[k].v[e]);
-        if constexpr (CAP) softcap_series<A, K>(x[e], cap, inv_cap);
-        hi = fmax(hi, x[e][0]);
+        for (int k = 0; k <= K; ++k) x[u][e][k] = to_acc(a[u][k].v[e]);
+        if constexpr (CAP) softcap_series<A, K>(x[u][e], cap, inv_cap);
+        hi = fmax(hi, x[u][e][0]);
       }
-      rescale<A, K>(m, hi, S);
-      if (m != kNegInf) {
+    rescale<A, K>(m, hi, S);
+    if (m != kNegInf) {
 #pragma unroll
-        for (int e = 0; e < V; ++e) accumulate_element<A, K>(x[e][0], x[e], m, S);
-      }
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < V; ++e) accumulate_element<A, K>(x[u][e][0], x[u][e], m, S);
     }
-    scalar_from = nvec * V;
   }
-  for (int64_t col = scalar_from + threadIdx.x; col < classes; col += THREADS) {
+  for (; j < nvec; j += THREADS) {
+    Vec<T, V> a[K + 1];
+#pragma unroll
+    for (int k = 0; k <= K; ++k) a[k] = load_vec_nt_any<T, V>(z.p[k] + base + head + j * V);
+    A x[V][K + 1];
+    A hi = kNegInf;
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+#pragma unroll
+      for (int k = 0; k <= K; ++k) x[e][k] = to_acc(a[k].v[e]);
+      if constexpr (CAP) softcap_series<A, K>(x[e], cap, inv_cap);
+      hi = fmax(hi, x[e][0]);
+    }
+    rescale<A, K>(m, hi, S);
+    if (m != kNegInf) {
+#pragma unroll
+      for (int e = 0; e < V; ++e) accumulate_element<A, K>(x[e][0], x[e], m, S);
+    }
+  }
+  for (int64_t i = threadIdx.x; i < classes - nvec * V; i += THREADS) {   // the elements around the vectors
+    const int64_t col = i < head ? i : i + nvec * V;
     A x[K + 1];
 #pragma unroll
     for (int k = 0; k <= K; ++k) x[k] = to_acc(z.p[k][base + col]);
@@ -235,10 +246,8 @@ static int launch_ce_k(const CeArgs& a) {
   constexpr int V = VecWidth<T>::value;
   CPtrs<T> z{};
   MPtrs<A> loss{}, lse{};
-  bool vec_ok = (a.row_stride * static_cast<int64_t>(sizeof(T))) % 16 == 0;
   for (int k = 0; k <= K; ++k) {
     z.p[k] = static_cast<const T*>(a.z[k]);
-    vec_ok = vec_ok && pt_host::aligned16(a.z[k]);
     if (a.lse != nullptr) lse.p[k] = static_cast<A*>(a.lse[k]);
   }
   A* per_row = static_cast<A*>(a.workspace);
@@ -250,7 +259,7 @@ static int launch_ce_k(const CeArgs& a) {
   const A inv_cap = A(1) / capv;
 #define PT_CE_LAUNCH(TH, CP)                                                                   \
   cross_entropy_series_row_kernel<T, K, TH, CP><<<dim3(a.rows), dim3(TH), 0, a.stream>>>(     \
-      z, a.rows, a.classes, a.row_stride, vec_ok, a.target, a.ignore_index, loss, lse, capv, inv_cap)
+      z, a.rows, a.classes, a.row_stride, a.target, a.ignore_index, loss, lse, capv, inv_cap)
   if (a.classes >= 4096 * static_cast<int64_t>(V)) {
     if (cap) PT_CE_LAUNCH(512, true);
     else PT_CE_LAUNCH(512, false);
@@ -315,13 +324,17 @@ __device__ __forceinline__ void ce_bwd_element(const A (&x)[K + 1], bool is_targ
   }
 }
 
+// As in the forward, rows start at any element; the vectors start at a 16-byte
+// boundary of the output, as partly written 16-byte stores cost more than such
+// loads (4096 x 32001 bfloat16, degree 3, 2.1 GB: 576 us by elements, 515 us by
+// unaligned vectors, 481 us from the boundary).
 // Two vectors per order in flight per thread (91 VGPRs, 5 waves per SIMD) measure
 // about 1% faster than one (59 VGPRs, 8 waves) on the 8192 x 32000 fp32 rows.
 constexpr int kCeBwdUnroll = 2;
 
 template <typename T, int K, int THREADS, bool CAP>
 __global__ __launch_bounds__(THREADS) void cross_entropy_series_bwd_kernel(
-    CPtrs<T> z, int64_t classes, int64_t row_stride, bool vec_ok, const int64_t* __restrict__ target,
+    CPtrs<T> z, int64_t classes, int64_t row_stride, const int64_t* __restrict__ target,
     int64_t ignore_index, CPtrs<typename AccOf<T>::type> lse_p, CPtrs<typename AccOf<T>::type> cot_p,
     MPtrs<T> dz, typename AccOf<T>::type cap, typename AccOf<T>::type inv_cap) {
   using A = typename AccOf<T>::type;
@@ -336,6 +349,7 @@ __global__ __launch_bounds__(THREADS) void cross_entropy_series_bwd_kernel(
     lse[k] = lse_p.p[k][row];
     c[k] = ignored ? A(0) : cot_p.p[k][row];
   }
+  const int64_t head = ce_head(dz.p[0] + out, classes), nvec = (classes - head) / V;
   // U vectors per order in flight per thread and iteration, as in the forward.
   auto vec_step = [&](Vec<T, V> (&a)[K + 1], int64_t j) {
 #pragma unroll
@@ -346,37 +360,33 @@ __global__ __launch_bounds__(THREADS) void cross_entropy_series_bwd_kernel(
         A x[K + 1];
 #pragma unroll
         for (int k = 0; k <= K; ++k) x[k] = vec_get(a[k], e + h);
-        ce_bwd_element<A, K, CAP>(x, j * V + e + h == y, lse, c, cap, inv_cap, r[h]);
+        ce_bwd_element<A, K, CAP>(x, head + j * V + e + h == y, lse, c, cap, inv_cap, r[h]);
       }
 #pragma unroll
       for (int k = 0; k <= K; ++k) vec_put2(a[k], e, r[0][k], r[1][k]);
     }
 #pragma unroll
-    for (int k = 0; k <= K; ++k) store_vec_nt<T, V>(dz.p[k] + out + j * V, a[k]);
+    for (int k = 0; k <= K; ++k) store_vec_nt_any<T, V>(dz.p[k] + out + head + j * V, a[k]);
   };
-  int64_t scalar_from = 0;
-  if (vec_ok) {
-    constexpr int U = kCeBwdUnroll;
-    const int64_t nvec = classes / V;
-    int64_t j = threadIdx.x;
-    for (; j + (U - 1) * THREADS < nvec; j += U * THREADS) {
-      Vec<T, V> a[U][K + 1];
+  constexpr int U = kCeBwdUnroll;
+  int64_t j = threadIdx.x;
+  for (; j + (U - 1) * THREADS < nvec; j += U * THREADS) {
+    Vec<T, V> a[U][K + 1];
 #pragma unroll
-      for (int u = 0; u < U; ++u)
+    for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int k = 0; k <= K; ++k) a[u][k] = load_vec_nt<T, V>(z.p[k] + base + (j + u * THREADS) * V);
+      for (int k = 0; k <= K; ++k) a[u][k] = load_vec_nt_any<T, V>(z.p[k] + base + head + (j + u * THREADS) * V);
 #pragma unroll
-      for (int u = 0; u < U; ++u) vec_step(a[u], j + u * THREADS);
-    }
-    for (; j < nvec; j += THREADS) {
-      Vec<T, V> a[K + 1];
-#pragma unroll
-      for (int k = 0; k <= K; ++k) a[k] = load_vec_nt<T, V>(z.p[k] + base + j * V);
-      vec_step(a, j);
-    }
-    scalar_from = nvec * V;
+    for (int u = 0; u < U; ++u) vec_step(a[u], j + u * THREADS);
   }
-  for (int64_t col = scalar_from + threadIdx.x; col < classes; col += THREADS) {
+  for (; j < nvec; j += THREADS) {
+    Vec<T, V> a[K + 1];
+#pragma unroll
+    for (int k = 0; k <= K; ++k) a[k] = load_vec_nt_any<T, V>(z.p[k] + base + head + j * V);
+    vec_step(a, j);
+  }
+  for (int64_t i = threadIdx.x; i < classes - nvec * V; i += THREADS) {   // the elements around the vectors
+    const int64_t col = i < head ? i : i + nvec * V;
     A x[K + 1], r[K + 1];
 #pragma unroll
     for (int k = 0; k <= K; ++k) x[k] = to_acc(z.p[k][base + col]);
@@ -393,21 +403,18 @@ static int launch_ce_bwd_k(const CeBwdArgs& a) {
   CPtrs<T> z{};
   CPtrs<A> lse{}, cot{};
   MPtrs<T> dz{};
-  bool vec_ok = (a.row_stride * static_cast<int64_t>(sizeof(T))) % 16 == 0 &&
-                (a.classes * static_cast<int64_t>(sizeof(T))) % 16 == 0;
   for (int k = 0; k <= K; ++k) {
     z.p[k] = static_cast<const T*>(a.z[k]);
     lse.p[k] = static_cast<const A*>(a.lse[k]);
     cot.p[k] = static_cast<const A*>(a.cot[k]);
     dz.p[k] = static_cast<T*>(a.dz[k]);
-    vec_ok = vec_ok && pt_host::aligned16(a.z[k]) && pt_host::aligned16(a.dz[k]);
   }
   const bool cap = a.softcap > 0.0;
   const A capv = cap ? static_cast<A>(a.softcap) : A(1);
   const A inv_cap = A(1) / capv;
 #define PT_CE_BWD_LAUNCH(TH, CP)                                                                     \
   cross_entropy_series_bwd_kernel<T, K, TH, CP><<<dim3(a.rows), dim3(TH), 0, a.stream>>>(           \
-      z, a.classes, a.row_stride, vec_ok, a.target, a.ignore_index, lse, cot, dz, capv, inv_cap)
+      z, a.classes, a.row_stride, a.target, a.ignore_index, lse, cot, dz, capv, inv_cap)
   if (a.classes >= 4096 * static_cast<int64_t>(V)) {
     if (cap) PT_CE_BWD_LAUNCH(512, true);
     else PT_CE_BWD_LAUNCH(512, false);

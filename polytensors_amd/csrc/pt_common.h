@@ -108,6 +108,22 @@ __device__ __forceinline__ void store_vec_nt(T* p, const Vec<T, V>& v) {
   __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, v), reinterpret_cast<u32x4_t*>(p));
 }
 
+// The same at any element's address (a row of odd length, an order of a stacked buffer of odd
+// size): gfx950 takes 16-byte global accesses at any byte, so these are the same instructions as the
+// aligned ones and cost the same where the address is aligned.
+typedef u32x4_t u32x4_any_t __attribute__((aligned(2)));
+template <typename T, int V>
+__device__ __forceinline__ Vec<T, V> load_vec_nt_any(const T* p) {
+  static_assert(sizeof(Vec<T, V>) == 16, "16-byte vectors only");
+  const u32x4_t w = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any_t*>(p));
+  return __builtin_bit_cast(Vec<T, V>, w);
+}
+template <typename T, int V>
+__device__ __forceinline__ void store_vec_nt_any(T* p, const Vec<T, V>& v) {
+  static_assert(sizeof(Vec<T, V>) == 16, "16-byte vectors only");
+  __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, v), reinterpret_cast<u32x4_any_t*>(p));
+}
+
 // Storage vector <-> arithmetic values. bfloat16 pairs are unpacked from
 // 32-bit words with one shift or mask each and packed with one conversion
 // instruction per pair.

@@ -273,3 +273,26 @@ def test_weights_and_label_smoothing_gradient_series(weighted, smoothing):
         out.backward()
     _check(out.coeffs, taylor(loss, [Z], degree), torch.float64)
     _check(x.grad.coeffs, taylor(lambda z: torch.func.grad(loss)(z), [Z], degree), torch.float64)
+
+
+# Rows that start at any element: odd class counts around whole vectors and unrolled pairs of them,
+# a view one column into rows of odd length. Loss and gradient series against the oracle.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32, torch.float64])
+@pytest.mark.parametrize("C", [1, 7, 9, 2047, 2049, 4097, 33001])
+def test_rows_at_any_element(dtype, C):
+    degree, N = 3, 5
+    full, y = _logits(N, C, degree, seed=C, dtype=dtype, pad=2)
+    Z = [c[:, 1:C + 1].contiguous() for c in full]
+    views = [c.cuda()[:, 1:C + 1] for c in full]
+    cot = [c.sum(1) for c in _logits(N, 3, degree, seed=5, dtype=torch.float64)[0]]
+    with PolyTensor.plain_range():
+        logits = PolyTensor(tuple(views), requires_grad=True)
+        loss = PolyTensor.cross_entropy(logits, y.cuda(), reduction="none")
+        loss.backward(PolyTensor(tuple(c.to(loss.dtype).cuda() for c in cot)))
+    Zd = [c.double() for c in Z]
+    _check([c.detach() for c in loss.coeffs], oracle.cross_entropy(Zd, y, reduction="none"), dtype, inputs=Z)
+    want = oracle.cross_entropy_backward(Zd, y, cot)
+    for k, (a, b) in enumerate(zip(logits.grad.coeffs, want)):
+        # (one class: p - e_y is zero and the kernel's value the rounding of the cotangent's)
+        scale = max(b.abs().max().item(), 1e-3)
+        assert (a.cpu().double() - b).abs().max().item() / scale <= TOL[dtype], k
