@@ -46,6 +46,7 @@
 
 #include "cauchy_matmul.h"
 #include "mfma.h"
+#include "order_gemm.inl"
 
 namespace pt {
 
@@ -334,20 +335,29 @@ static int launch_cauchy_k(const CauchyArgs& a) {
   for (int o = 0; o <= K; ++o) C.p[o] = static_cast<T*>(a.c[o]);
   vec = vec && a.k % V == 0 && a.a_bs % V == 0 && a.b_bs % V == 0 && (a.trans_b || a.n % V == 0);
   const bool a_series = a.a_orders > 1, b_series = a.b_orders > 1;
+  auto zero_higher = [&](int st) -> int {   // two ordinary operands: C_0 = A_0 B_0, zero higher orders
+    if (st != PT_OK || K == 0) return st;
+    const int64_t count = a.batch * a.m * a.n;
+    const int64_t blocks = std::min<int64_t>((count + 255) / 256, 4096);
+    cauchy_zero_orders_kernel<T><<<dim3(blocks), dim3(256), 0, a.stream>>>(C, K, count);
+    PT_LAUNCH_CHECK();
+    return PT_OK;
+  };
+  if constexpr (sizeof(T) == 4) {
+    // float32 with an ordinary operand: order by order, where the DMA can read the operands (the
+    // kernel below reads any row length and alignment, at 114 against 137 TFLOP/s: order_gemm.inl)
+    if (!(a_series && b_series) && order_gemm_takes<T>(a)) {
+      const int orders = std::max(a.a_orders, a.b_orders), st = launch_by_order<T>(a, orders);
+      return orders == K + 1 ? st : zero_higher(st);
+    }
+  }
   if constexpr (K == 0) {
     return launch_cauchy_orders<T, 0, 1, 1>(a, A, B, C, vec);
   } else {
     if (a_series && b_series) return launch_cauchy_orders<T, K, K + 1, K + 1>(a, A, B, C, vec);
     if (a_series) return launch_cauchy_orders<T, K, K + 1, 1>(a, A, B, C, vec);
     if (b_series) return launch_cauchy_orders<T, K, 1, K + 1>(a, A, B, C, vec);
-    // Two ordinary operands: C_0 = A_0 B_0 and zero higher orders.
-    int st = launch_cauchy_orders<T, 0, 1, 1>(a, A, B, C, vec);
-    if (st != PT_OK) return st;
-    const int64_t count = a.batch * a.m * a.n;
-    const int64_t blocks = std::min<int64_t>((count + 255) / 256, 4096);
-    cauchy_zero_orders_kernel<T><<<dim3(blocks), dim3(256), 0, a.stream>>>(C, K, count);
-    PT_LAUNCH_CHECK();
-    return PT_OK;
+    return zero_higher(launch_cauchy_orders<T, 0, 1, 1>(a, A, B, C, vec));
   }
 }
 

@@ -38,9 +38,12 @@
 
 #include "cauchy_matmul.h"
 #include "half_mfma.h"
+#include "order_gemm.inl"
 
 namespace pt {
 
+// Both operands are series (an ordinary one: order_gemm.inl).
+//
 // Workgroup tile: WMW x WNW waves, each owning FM x FN MFMA blocks of 16 x 16 of every C_k. The
 // narrow tile (64 x 64, 4 waves of 32 x 32) leaves LDS for two workgroups per CU; the wide tile
 // (128 x 128, 8 waves of 64 x 32) reads a third fewer LDS bytes per MFMA and half the HBM
@@ -268,21 +271,23 @@ static int launch_cauchy_half_k(const CauchyArgs& a) {
   for (int o = 0; o < a.a_orders; ++o) A.p[o] = static_cast<const T*>(a.a[o]);
   for (int o = 0; o < a.b_orders; ++o) B.p[o] = static_cast<const T*>(a.b[o]);
   for (int o = 0; o <= K; ++o) C.p[o] = static_cast<T*>(a.c[o]);
-  const bool a_series = a.a_orders > 1, b_series = a.b_orders > 1;
-  if constexpr (K == 0) {
-    return launch_cauchy_half_orders<T, 0, 1, 1>(a, A, B, C);
-  } else {
-    if (a_series && b_series) return launch_cauchy_half_orders<T, K, K + 1, K + 1>(a, A, B, C);
-    if (a_series) return launch_cauchy_half_orders<T, K, K + 1, 1>(a, A, B, C);
-    if (b_series) return launch_cauchy_half_orders<T, K, 1, K + 1>(a, A, B, C);
-    const int st = launch_cauchy_half_orders<T, 0, 1, 1>(a, A, B, C);
-    if (st != PT_OK) return st;
-    const int64_t count = a.batch * a.m * a.n;
-    const int64_t blocks = std::min<int64_t>((count + 255) / 256, 4096);
-    cauchy_half_zero_orders_kernel<T><<<dim3(blocks), dim3(256), 0, a.stream>>>(C, K, count);
-    PT_LAUNCH_CHECK();
-    return PT_OK;
-  }
+  return launch_cauchy_half_orders<T, K, K + 1, K + 1>(a, A, B, C);
+}
+
+// A product with an ordinary operand: every order by itself; two ordinary operands give order 0,
+// and zero higher orders.
+template <typename T>
+static int launch_cauchy_half_ordinary(const CauchyArgs& a) {
+  const int orders = std::max(a.a_orders, a.b_orders);
+  const int st = launch_by_order<T>(a, orders);
+  if (st != PT_OK || orders > a.degree) return st;
+  MPtrs<T> C{};
+  for (int o = 0; o <= a.degree; ++o) C.p[o] = static_cast<T*>(a.c[o]);
+  const int64_t count = a.batch * a.m * a.n;
+  const int64_t blocks = std::min<int64_t>((count + 255) / 256, 4096);
+  cauchy_half_zero_orders_kernel<T><<<dim3(blocks), dim3(256), 0, a.stream>>>(C, a.degree, count);
+  PT_LAUNCH_CHECK();
+  return PT_OK;
 }
 
 template <typename T>
@@ -300,8 +305,14 @@ int launch_cauchy_half(const CauchyArgs& a) {
         "16-byte aligned operands and batch strides, and each matrix below 1 GiB");
     return PT_UNSUPPORTED;
   }
+  if (a.a_orders == 1 || a.b_orders == 1) {
+    if (!order_gemm_takes<T>(a)) {
+      pt_host::set_error("Cauchy matmul (16-bit): more output tiles than a launch holds");
+      return PT_UNSUPPORTED;
+    }
+    return launch_cauchy_half_ordinary<T>(a);
+  }
   switch (a.degree) {
-    case 0: return launch_cauchy_half_k<T, 0>(a);
     case 1: return launch_cauchy_half_k<T, 1>(a);
     case 2: return launch_cauchy_half_k<T, 2>(a);
     case 3: return launch_cauchy_half_k<T, 3>(a);

@@ -1,0 +1,405 @@
+// Products of a series with an ordinary matrix, C_o = A_o B (or A B_o), o = 0..K, as one matrix
+// product in which the orders are further rows (columns) of C. float32, and bfloat16 / float16 with
+// float32 accumulation. An ordinary operand mixes no orders, so the k-diagonals share nothing as
+// they do in the series-by-series kernels (cauchy_matmul*.inl, which ran these products before):
+// what bounds it is how fast one tile's contraction streams from memory to the MFMAs. With K = 3,
+// the forward products and the input gradients of a 1024 -> 4096 -> 1024 bfloat16 layer pair on 4096
+// rows took 232 and 222 us each (600 TFLOP/s) and take 137 and 129 (1000-1070); 8192 rows of float32,
+// 768 -> 3072, 1356 us (114 TFLOP/s) and 1281 (121).
+//
+// * Chunks of 64 bytes of contraction (32 halves, 16 floats) are moved into LDS by LDS DMA
+//   (half_mfma.h) in a ring of kRing buffers. The DMA of chunk c + kRing is issued when chunk c's
+//   operands are in registers, and waited for by a count (vmcnt) three chunks later, so a tile has
+//   three chunks of memory latency in flight where the two-buffer kernels have one.
+// * Operands are read from LDS one chunk ahead into a second register set, so the LDS reads issue
+//   between the MFMAs of the chunk before: one barrier per chunk.
+// * B may be stored [n][k] or [k][n]; the latter is read through transpose reads (halves) or
+//   element reads (floats).
+#pragma once
+
+#include <algorithm>
+
+#include "cauchy_matmul.h"
+#include "half_mfma.h"
+#include "mfma.h"
+
+namespace pt {
+
+// One MFMA block of a chunk: its operand registers per lane, and how they are read from a tile.
+// Tiles with the contraction along rows: [row][64 bytes], 16-byte chunk ch of row r stored at
+// ch ^ F((r / 4) % 4) with F = (0, 2, 3, 1); along columns: [k][width], chunk ^ kSwz(k).
+template <typename T>
+struct OrderBlock;
+
+__host__ __device__ __forceinline__ int order_swz_rows(int r, int ch) { return ch ^ ((0x78 >> (2 * ((r >> 2) & 3))) & 3); }
+
+template <typename T>
+struct OrderBlockHalf {
+  static constexpr int S = 16, ACC = 4, STEPS = 1;   // block side, accumulator registers, MFMAs per chunk
+  using frag_t = u32x4;
+  using acc_t = floatx4;
+  // rows along n of the block are consecutive in a lane: C^T = B^T A^T
+  __host__ __device__ __forceinline__ static int swz_k(int k, int ch) {   // rows of at least 256 bytes
+    return ch ^ (2 * ((k & 3) | (((k >> 3) & 1) << 2)));
+  }
+  __device__ __forceinline__ static frag_t read_rows(const T* tile, int row0, int lane) {
+    const int row = row0 + lane % 16;
+    return *reinterpret_cast<const u32x4*>(&tile[row * 32 + order_swz_rows(row, lane / 16) * 8]);
+  }
+  template <int W>
+  __device__ __forceinline__ static frag_t read_cols(const T* tile, int col0, int lane) {
+    const int g = lane / 16, j = (lane % 16) / 4, a = lane % 4;
+    const int k1 = 8 * g + j, k2 = 8 * g + 4 + j;
+    const int ch = col0 / 8 + a / 2, e = 4 * (a % 2);
+    return lds_read_tr16x2(&tile[k1 * W + swz_k(k1, ch) * 8 + e], &tile[k2 * W + swz_k(k2, ch) * 8 + e]);
+  }
+  __device__ __forceinline__ static acc_t zero() { return acc_t{0.f, 0.f, 0.f, 0.f}; }
+  __device__ __forceinline__ static acc_t mma(const frag_t& a, const frag_t& b, int, acc_t c) {
+    return HalfMfma<T>::mma(b, a, c);
+  }
+};
+template <>
+struct OrderBlock<bf16> : OrderBlockHalf<bf16> {};
+template <>
+struct OrderBlock<_Float16> : OrderBlockHalf<_Float16> {};
+
+template <>
+struct OrderBlock<float> {
+  static constexpr int S = 32, ACC = 16, STEPS = 8;
+  struct frag_t {
+    float v[8];   // contraction elements 8 (lane / 32) .. + 7 of row lane % 32
+  };
+  using acc_t = floatx16;
+  __host__ __device__ __forceinline__ static int swz_k(int k, int ch) { return ch ^ (8 * ((k >> 3) & 1)); }
+  __device__ __forceinline__ static frag_t read_rows(const float* tile, int row0, int lane) {
+    const int row = row0 + lane % 32, h = lane / 32;
+    frag_t f;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const Vec<float, 4> x = load_vec<float, 4>(&tile[row * 16 + order_swz_rows(row, 2 * h + q) * 4]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f.v[4 * q + e] = x.v[e];
+    }
+    return f;
+  }
+  template <int W>
+  __device__ __forceinline__ static frag_t read_cols(const float* tile, int col0, int lane) {
+    const int col = col0 + lane % 32, h = lane / 32;
+    frag_t f;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) f.v[s] = tile[(8 * h + s) * W + swz_k(8 * h + s, col / 4) * 4 + col % 4];
+    return f;
+  }
+  __device__ __forceinline__ static acc_t zero() { return Mfma<float>::zero(); }
+  __device__ __forceinline__ static acc_t mma(const frag_t& a, const frag_t& b, int s, acc_t c) {
+    return Mfma<float>::mma(b.v[s], a.v[s], c);
+  }
+};
+
+template <typename T>
+struct OrderGemmParams {
+  CPtrs<T> a, b;
+  MPtrs<T> c;
+  int m, n, k;                  // of one order; k a whole number of 16-byte vectors where it runs along rows
+  int lda, ldb;                 // row strides in elements
+  int a_bytes, b_bytes;         // extent of one matrix
+  int64_t a_bs, b_bs, c_bs;     // batch strides in elements
+  int a_step, b_step;           // 1 where the operand's pointer changes by order
+  int orders;                   // by order: orders of C; summed: terms of the sum
+  int tiles_m, tiles_n;         // of one order
+};
+
+constexpr int kOrderRing = 4;
+
+template <typename T, int WMW, int WNW, int FM, int FN>
+struct OrderTile {
+  using B = OrderBlock<T>;
+  static constexpr int BM = WMW * FM * B::S, BN = WNW * FN * B::S, BK = 64 / static_cast<int>(sizeof(T));
+  static constexpr int kWaves = WMW * WNW, kThreads = kWaves * kWave;
+  static constexpr int SA = BM / 16 / kWaves, SB = BN / 16 / kWaves;   // 1 KB DMA segments per wave and chunk
+  static constexpr size_t LDS = static_cast<size_t>(kOrderRing) * (BM + BN) * 64;
+  static_assert(SA * 16 * kWaves == BM && SB * 16 * kWaves == BN, "whole DMA segments per wave");
+};
+
+template <int N>
+__device__ __forceinline__ void order_wait_barrier() {   // at most N of this wave's vector loads in flight
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+template <typename T, int WMW, int WNW, int FM, int FN, bool A_COLS, bool B_COLS, bool SUM, int MIN_WAVES>
+__global__ __launch_bounds__(WMW* WNW* kWave) __attribute__((amdgpu_waves_per_eu(MIN_WAVES)))
+void order_gemm_kernel(OrderGemmParams<T> p) {
+  using Tile = OrderTile<T, WMW, WNW, FM, FN>;
+  using Blk = OrderBlock<T>;
+  constexpr int BM = Tile::BM, BN = Tile::BN, BK = Tile::BK, V = 16 / static_cast<int>(sizeof(T));
+  constexpr int SA = Tile::SA, SB = Tile::SB, R = kOrderRing;
+  constexpr int CPA = A_COLS ? BM / V : 4, CPB = B_COLS ? BN / V : 4;   // 16-byte chunks per tile row
+  __shared__ __attribute__((aligned(16))) T As[R][BM * BK];
+  __shared__ __attribute__((aligned(16))) T Bs[R][BN * BK];
+
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int wm = wave / WNW, wn = wave % WNW;
+
+  // Workgroup -> tile: consecutive ids go round robin over the 8 XCDs, so each XCD takes a
+  // contiguous range of tiles; within it kGroup tile rows are walked column by column.
+  constexpr int kXcd = 8, kGroup = 8;
+  int t = blockIdx.x;
+  {
+    const int total = gridDim.x, per = total / kXcd;
+    if (t < per * kXcd) t = (t % kXcd) * per + t / kXcd;
+  }
+  const int rows = p.tiles_m * (SUM || p.a_step == 0 ? 1 : p.orders);   // tile rows: every order's of A
+  const int cols = p.tiles_n * (SUM || p.a_step != 0 || p.b_step == 0 ? 1 : p.orders);
+  const int per_batch = rows * cols;
+  const int64_t batch = t / per_batch;
+  t %= per_batch;
+  const int group = t / (kGroup * cols), first = group * kGroup, high = min(kGroup, rows - first);
+  const int tr = first + (t % (kGroup * cols)) % high, tc = (t % (kGroup * cols)) / high;
+  const int oa = tr / p.tiles_m, ob = tc / p.tiles_n;   // (one of them is 0)
+  const int tile_m = (tr % p.tiles_m) * BM, tile_n = (tc % p.tiles_n) * BN;
+  const int order = SUM ? 0 : oa + ob;
+
+  // this wave's DMA segments: each lane's byte offset in the matrix and contraction position in
+  // the chunk (past every chunk's end for rows and columns outside the matrix)
+  int va[SA], vb[SB], ka[SA], kb[SB];
+#pragma unroll
+  for (int s = 0; s < SA; ++s) {
+    const int slot = (wave * SA + s) * 64 + lane, r = slot / CPA, ch = slot % CPA;
+    if constexpr (A_COLS) {
+      const int lch = Blk::swz_k(r, ch), g = tile_m + lch * V;
+      va[s] = (r * p.lda + g) * static_cast<int>(sizeof(T));
+      ka[s] = g < p.m ? r : INT32_MAX;
+    } else {
+      const int lch = order_swz_rows(r, ch), g = tile_m + r;
+      va[s] = (g * p.lda + lch * V) * static_cast<int>(sizeof(T));
+      ka[s] = g < p.m ? lch * V : INT32_MAX;
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < SB; ++s) {
+    const int slot = (wave * SB + s) * 64 + lane, r = slot / CPB, ch = slot % CPB;
+    if constexpr (B_COLS) {
+      const int lch = Blk::swz_k(r, ch), g = tile_n + lch * V;
+      vb[s] = (r * p.ldb + g) * static_cast<int>(sizeof(T));
+      kb[s] = g < p.n ? r : INT32_MAX;
+    } else {
+      const int lch = order_swz_rows(r, ch), g = tile_n + r;
+      vb[s] = (g * p.ldb + lch * V) * static_cast<int>(sizeof(T));
+      kb[s] = g < p.n ? lch * V : INT32_MAX;
+    }
+  }
+  const int step_a = (A_COLS ? BK * p.lda : BK) * static_cast<int>(sizeof(T));
+  const int step_b = (B_COLS ? BK * p.ldb : BK) * static_cast<int>(sizeof(T));
+  const int per_order = (p.k + BK - 1) / BK;
+  const int chunks = SUM ? per_order * p.orders : per_order;
+
+  // the chunk to issue next: its term of the sum, its position, its buffer. Past the last chunk
+  // every lane is out of range (zeros nobody reads), so each chunk counts the same loads.
+  int is = 0, ik = 0, ibuf = 0, left = p.k;
+  BufferRsrc ra, rb;
+  auto point = [&]() {   // the operands of term is (of order oa, ob)
+    const int term = min(is, p.orders - 1);
+    const int sa = SUM ? term * p.a_step : oa, sb = SUM ? (p.orders - 1 - term) * p.b_step : ob;
+    ra = buffer_rsrc(p.a.p[sa] + batch * p.a_bs, p.a_bytes);
+    rb = buffer_rsrc(p.b.p[sb] + batch * p.b_bs, p.b_bytes);
+  };
+  point();
+  auto issue_segment = [&](int s) {   // segment s of the chunk: A's SA, then B's SB
+    if (s < SA) {
+      lds_dma16(&As[ibuf][(wave * SA + s) * (1024 / static_cast<int>(sizeof(T)))], ra,
+                ka[s] < left ? va[s] : kBufferOutOfRange);
+      va[s] += step_a;
+    } else {
+      const int u = s - SA;
+      lds_dma16(&Bs[ibuf][(wave * SB + u) * (1024 / static_cast<int>(sizeof(T)))], rb,
+                kb[u] < left ? vb[u] : kBufferOutOfRange);
+      vb[u] += step_b;
+    }
+  };
+  auto issued = [&]() {
+    ibuf = ibuf + 1 == R ? 0 : ibuf + 1;
+    left -= BK;
+    if (++ik == per_order) {
+      ik = 0;
+      ++is;
+      left = SUM && is < p.orders ? p.k : 0;
+      if constexpr (SUM) {
+#pragma unroll
+        for (int s = 0; s < SA; ++s) va[s] -= per_order * step_a;
+#pragma unroll
+        for (int s = 0; s < SB; ++s) vb[s] -= per_order * step_b;
+        point();
+      }
+    }
+  };
+
+  typename Blk::acc_t acc[FM][FN];
+#pragma unroll
+  for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+    for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = Blk::zero();
+
+  typename Blk::frag_t fa[2][FM], fb[2][FN];
+  auto read_operand = [&](int buf, int set, int i) {   // operand i of a chunk: B's FN, then A's FM
+    if (i < FN) {
+      const int at = (wn * FN + i) * Blk::S;
+      if constexpr (B_COLS) fb[set][i] = Blk::template read_cols<BN>(Bs[buf], at, lane);
+      else fb[set][i] = Blk::read_rows(Bs[buf], at, lane);
+    } else {
+      const int at = (wm * FM + i - FN) * Blk::S;
+      if constexpr (A_COLS) fa[set][i - FN] = Blk::template read_cols<BM>(As[buf], at, lane);
+      else fa[set][i - FN] = Blk::read_rows(As[buf], at, lane);
+    }
+  };
+  auto multiply_row = [&](int set, int fm) {
+#pragma unroll
+    for (int s = 0; s < Blk::STEPS; ++s)   // (no MFMA waits for the one before it)
+#pragma unroll
+      for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = Blk::mma(fa[set][fm], fb[set][fn], s, acc[fm][fn]);
+  };
+
+  for (int i = 0; i < R; ++i) {
+#pragma unroll
+    for (int s = 0; s < SA + SB; ++s) issue_segment(s);
+    issued();
+  }
+  order_wait_barrier<(R - 1) * (SA + SB)>();   // chunk 0 has landed, for every wave
+#pragma unroll
+  for (int i = 0; i < FM + FN; ++i) read_operand(0, 0, i);
+  int buf = 1;
+  // Chunk c is in register set c % 2; chunks c + 1 .. c + R - 1 are in flight or landed. The
+  // operand reads of chunk c + 1 and the DMA of chunk c + R are spread between the MFMA rows of
+  // chunk c (fixed by the scheduling barriers), so the MFMAs start right after the barrier.
+  auto step = [&](int set) {
+    order_wait_barrier<(R - 2) * (SA + SB)>();   // chunk c + 1 has landed; chunk c's buffer has been read
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm) {
+      multiply_row(set, fm);
+#pragma unroll
+      for (int i = fm * (FM + FN) / FM; i < (fm + 1) * (FM + FN) / FM; ++i) read_operand(buf, set ^ 1, i);
+#pragma unroll
+      for (int s = fm * (SA + SB) / FM; s < (fm + 1) * (SA + SB) / FM; ++s) issue_segment(s);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    issued();
+    buf = buf + 1 == R ? 0 : buf + 1;
+  };
+  int c = 0;
+  for (; c + 1 < chunks; c += 2) {
+    step(0);
+    step(1);
+  }
+  if (c < chunks) {
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm) multiply_row(0, fm);
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // no DMA outlives the workgroup's LDS
+
+  // ---- epilogue: a lane's registers are runs of four columns of one row of C ----
+  T* base = p.c.p[order] + batch * p.c_bs;
+#pragma unroll
+  for (int fm = 0; fm < FM; ++fm) {
+    const int row = tile_m + (wm * FM + fm) * Blk::S + lane % Blk::S;
+    if (row >= p.m) continue;
+#pragma unroll
+    for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+      for (int q = 0; q < Blk::ACC / 4; ++q) {
+        const int col = tile_n + (wn * FN + fn) * Blk::S + 8 * q + 4 * (lane / Blk::S);
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[fm][fn][4 * q + e];
+        T* dst = base + static_cast<int64_t>(row) * p.n + col;
+        if (col + 3 < p.n) {
+          Vec<T, 4> w;
+#pragma unroll
+          for (int e = 0; e < 4; e += 2) vec_put2(w, e, v[e], v[e + 1]);
+          __builtin_memcpy(dst, &w, sizeof(w));   // at any element: one 8- or 16-byte store
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (col + e < p.n) dst[e] = from_acc<T>(v[e]);
+        }
+      }
+  }
+}
+
+// Whether the DMA can read the operands: whole, aligned 16-byte vectors along rows, 32-bit offsets.
+template <typename T>
+static bool order_gemm_takes(const CauchyArgs& a) {
+  constexpr int64_t V = 16 / static_cast<int64_t>(sizeof(T)), kLimit = (int64_t{1} << 30) / static_cast<int64_t>(sizeof(T));
+  bool ok = a.k % V == 0 && (a.trans_b || a.n % V == 0) && a.a_bs % V == 0 && a.b_bs % V == 0 &&
+            a.m * a.k < kLimit && a.k * a.n < kLimit &&
+            ((a.m + 63) / 64) * ((a.n + 63) / 64) * std::max(a.a_orders, a.b_orders) * a.batch <= INT32_MAX;
+  for (int o = 0; o < a.a_orders; ++o) ok = ok && pt_host::aligned16(a.a[o]);
+  for (int o = 0; o < a.b_orders; ++o) ok = ok && pt_host::aligned16(a.b[o]);
+  return ok;
+}
+
+template <typename T, int WMW, int WNW, int FM, int FN, bool A_COLS, bool B_COLS, bool SUM>
+static int launch_order_tile(OrderGemmParams<T> p, int64_t batch, hipStream_t stream) {
+  using Tile = OrderTile<T, WMW, WNW, FM, FN>;
+  p.tiles_m = (p.m + Tile::BM - 1) / Tile::BM;
+  p.tiles_n = (p.n + Tile::BN - 1) / Tile::BN;
+  const int64_t tiles = static_cast<int64_t>(p.tiles_m) * p.tiles_n * (SUM ? 1 : p.orders) * batch;
+  order_gemm_kernel<T, WMW, WNW, FM, FN, A_COLS, B_COLS, SUM, 2>
+      <<<dim3(static_cast<unsigned>(tiles)), dim3(Tile::kThreads), 0, stream>>>(p);
+  PT_LAUNCH_CHECK();
+  return PT_OK;
+}
+
+// The tile: the one with the least estimated time per chunk of contraction over the launch.
+// * Halves: 256 x 256 (one workgroup of 8 waves a CU) takes 0.80 us a chunk with every CU busy, and
+//   128 x 128 (up to two workgroups of 4 waves a CU) 0.57 us with two and 0.35 with one (from 8192^3
+//   at 809 and 1173 us, and 512 chunks of 256 small tiles at 178 us): four small tiles cost 1.4
+//   times a large one where both fill the chip, less where the large ones leave CUs idle.
+// * Floats: 128 x 128, 128 x 64 and 64 x 64 (two, three and five workgroups a CU); MFMA-bound, so the
+//   busiest CU's tiles count, at 137, 133 and 128 TFLOP/s (8192 x 768 x 3072, degree 3).
+template <typename T, bool A_COLS, bool B_COLS, bool SUM>
+static int launch_order_gemm(const OrderGemmParams<T>& p, int64_t batch, hipStream_t stream) {
+  auto tiles = [&](int64_t bm, int64_t bn) {
+    return (p.m + bm - 1) / bm * ((p.n + bn - 1) / bn) * (SUM ? 1 : p.orders) * batch;
+  };
+  if constexpr (sizeof(T) == 2) {
+    const int64_t large = tiles(256, 256), small = tiles(128, 128), rest = small % 512;
+    const double t_large = 0.80 * static_cast<double>((large + 255) / 256);
+    const double t_small = 0.57 * static_cast<double>(small / 512) + (rest == 0 ? 0.0 : rest <= 256 ? 0.35 : 0.57);
+    if (t_large < t_small) return launch_order_tile<T, 2, 4, 8, 4, A_COLS, B_COLS, SUM>(p, batch, stream);
+    return launch_order_tile<T, 2, 2, 4, 4, A_COLS, B_COLS, SUM>(p, batch, stream);
+  } else {
+    auto cost = [&](int64_t bm, int64_t bn, double rate) {
+      return static_cast<double>((tiles(bm, bn) + 255) / 256 * bm * bn) / rate;
+    };
+    const double c0 = cost(128, 128, 137), c1 = cost(128, 64, 133), c2 = cost(64, 64, 128);
+    if (c0 <= c1 && c0 <= c2) return launch_order_tile<T, 2, 2, 2, 2, A_COLS, B_COLS, SUM>(p, batch, stream);
+    if (c1 <= c2) return launch_order_tile<T, 2, 2, 2, 1, A_COLS, B_COLS, SUM>(p, batch, stream);
+    return launch_order_tile<T, 2, 2, 1, 1, A_COLS, B_COLS, SUM>(p, batch, stream);
+  }
+}
+
+// C_o = A_o B or A B_o for `orders` orders (operands with one order are shared by all).
+template <typename T>
+static int launch_by_order(const CauchyArgs& a, int orders) {
+  OrderGemmParams<T> p{};
+  for (int o = 0; o < a.a_orders; ++o) p.a.p[o] = static_cast<const T*>(a.a[o]);
+  for (int o = 0; o < a.b_orders; ++o) p.b.p[o] = static_cast<const T*>(a.b[o]);
+  for (int o = 0; o < orders; ++o) p.c.p[o] = static_cast<T*>(a.c[o]);
+  p.m = static_cast<int>(a.m);
+  p.n = static_cast<int>(a.n);
+  p.k = static_cast<int>(a.k);
+  p.lda = p.k;
+  p.ldb = a.trans_b ? p.k : p.n;
+  p.a_bytes = static_cast<int>(a.m * a.k * static_cast<int64_t>(sizeof(T)));
+  p.b_bytes = static_cast<int>(a.n * a.k * static_cast<int64_t>(sizeof(T)));
+  p.a_bs = a.a_bs;
+  p.b_bs = a.b_bs;
+  p.c_bs = a.m * a.n;
+  p.a_step = a.a_orders > 1;
+  p.b_step = a.b_orders > 1;
+  p.orders = orders;
+  if (a.trans_b) return launch_order_gemm<T, false, false, false>(p, a.batch, a.stream);
+  return launch_order_gemm<T, false, true, false>(p, a.batch, a.stream);
+}
+
+}  // namespace pt

@@ -154,3 +154,30 @@ def test_full_size_config_sampled_rows():
     rhs = C + _ops.cauchy_matmul(A2, B, degree, False)
     for k in range(degree + 1):
         assert rel_err(lhs[k].cpu(), rhs[k].cpu()) <= 1e-5
+
+
+# An ordinary operand on either side: the order-by-order products, at the edges of their tiles (64, 128
+# and 256 rows or columns), contractions around its chunks (16 floats, 32 halves) and its four-chunk
+# ring, single rows, batches, and row lengths the 16-byte loads do not take.
+# Tolerance: each order against float64 of the stored inputs, relative to its largest value: one
+# rounding of the result in the storage type, and float32 sums of k terms (below 1e-5 here).
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -11 + 1e-5)])
+@pytest.mark.parametrize("m,k,n,batch,degree", [
+    (1, 8, 8, (), 1), (64, 16, 64, (), 2), (65, 72, 136, (), 3), (128, 128, 128, (), 8), (129, 160, 264, (), 2),
+    (257, 64, 256, (3,), 1), (255, 1000, 513, (), 2), (40, 15, 33, (2,), 2), (520, 256, 3000, (), 4), (2, 4104, 72, (), 3)])
+def test_ordinary_operand_products(dtype, tol, m, k, n, batch, degree):
+    g = torch.Generator().manual_seed(m + k + n)
+    A = [torch.randn(*batch, m, k, generator=g).to(dtype) for _ in range(degree + 1)]
+    W = (torch.randn(n, k, generator=g) / k ** 0.5).to(dtype)
+    B = [torch.randn(*batch, k, n, generator=g).to(dtype) for _ in range(degree + 1)]
+    L = (torch.randn(m, k, generator=g) / k ** 0.5).to(dtype)
+    with torch.no_grad(), PolyTensor.plain_range():
+        x, y = (PolyTensor(tuple(c.cuda() for c in s)) for s in (A, B))
+        got = {"x @ W^T": x @ W.cuda().t(), "x @ W": x @ W.cuda().t().contiguous(), "L @ y": L.cuda() @ y,
+               "linear": torch.nn.functional.linear(x, W.cuda())}
+    right, left = W.double().t(), L.double()
+    for name, out in got.items():
+        for o in range(degree + 1):
+            want = left @ B[o].double() if name == "L @ y" else A[o].double() @ right
+            err = (out.coeffs[o].cpu().double() - want).abs().max() / want.abs().max()
+            assert err <= tol, (name, o, err)
