@@ -227,6 +227,25 @@ int pt_cauchy_matmul(int dtype, int degree, const void* const* a, int a_orders,
                      int trans_b, void* stream);
 
 /*
+ * One order of a product of series: the sum C = sum_s op(A_s) @ op(B_s) over `terms` (1..9) pairs
+ * of matrices, the gradient of an ordinary operand of pt_cauchy_matmul (the cotangent of its one
+ * order, /root/reference/src/polytensors/_plain.py:118-128 read in reverse), in one launch.
+ * a: `terms` pointers, each [batch, m, k], or [batch, k, m] if trans_a; row stride lda elements.
+ * b: `terms` pointers, each [batch, k, n], or [batch, n, k] if trans_b; row stride ldb elements.
+ * Batch strides in elements; 0 broadcasts one matrix over the batch.
+ * c: [batch, m, n] contiguous.
+ * dtype: PT_FLOAT32, PT_BFLOAT16 or PT_FLOAT16 (fp32 accumulation, each element rounded once).
+ * Rows are read in 16-byte vectors: operands 16-byte aligned, row and batch strides multiples of 16
+ * bytes, and so k where an operand's rows run along it (a unless trans_a, b if trans_b; the vectors
+ * past m or n of an operand whose rows run along those are read inside the row stride, and take no
+ * part); each matrix below 1 GiB, else PT_UNSUPPORTED. trans_a needs trans_b = 0.
+ */
+int pt_matmul_order_sum(int dtype, int terms, const void* const* a, const void* const* b, void* c,
+                        int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,
+                        int64_t a_batch_stride, int64_t b_batch_stride, int trans_a, int trans_b,
+                        void* stream);
+
+/*
  * Flash-style attention forward of degree-K series:
  *   S(t) = scale * Q(t) K(t)^T (masked), P(t) = softmax(S(t)), O(t) = P(t) V(t).
  * q: q_orders pointers (1 or K+1), each [bh, lq, d];

@@ -30,6 +30,7 @@ SCHEMAS = {
     "cross_entropy_series_backward": ("(Tensor[] z, Tensor target, int ignore_index, float softcap, Tensor lse, "
                                       "Tensor[] cot) -> Tensor"),
     "cauchy_matmul": "(Tensor[] a, Tensor[] b, int degree, bool trans_b) -> Tensor",
+    "matmul_order_sum": "(Tensor[] a, Tensor[] b, bool trans_a, bool trans_b) -> Tensor",
     "taylor_attention_fwd": ("(Tensor[] q, Tensor[] k, Tensor[] v, Tensor? mask, bool causal, float scale, "
                              "int degree, int[]? mask_map=None) -> (Tensor, Tensor)"),
     "taylor_attention_bwd": ("(Tensor[] q, Tensor[] k, Tensor[] v, Tensor out, Tensor lse, Tensor[] grad, "
@@ -127,6 +128,18 @@ def _(a, b, degree, trans_b):
     bb = b[0].shape[0]
     n = b[0].shape[1] if trans_b else b[0].shape[2]
     return a[0].new_empty((degree + 1, max(ba, bb), m, n))
+
+
+# sum_s op(a_s) @ op(b_s): the gradient of an ordinary operand (no gradient of its own: a graph of
+# the gradient is formed from cauchy_matmul)
+matmul_order_sum = _op("matmul_order_sum")
+
+
+@torch.library.register_fake(f"{NAMESPACE}::matmul_order_sum")
+def _(a, b, trans_a, trans_b):
+    m = a[0].shape[2 if trans_a else 1]
+    n = b[0].shape[1 if trans_b else 2]
+    return a[0].new_empty((max(a[0].shape[0], b[0].shape[0]), m, n))
 
 
 # ---------------------------------------------------------------------------
@@ -405,6 +418,14 @@ def _mm_setup(ctx, inputs, output):
     ctx.n_inputs = len(inputs)
 
 
+def _sums(*operands):
+    """Whether matmul_order_sum takes these matrices: no graph of the gradient is asked for, a type
+    it has, each (row-padded) matrix below 1 GiB."""
+    if torch.is_grad_enabled() or operands[0].dtype == torch.float64:
+        return False
+    return all((x.shape[-2] + 8) * (x.shape[-1] + 8) * x.element_size() < 1 << 30 for x in operands)
+
+
 def _mm_backward(ctx, grad):
     na, nb, degree, trans_b, need_a, need_b = ctx.meta
     saved = ctx.saved_tensors
@@ -413,12 +434,18 @@ def _mm_backward(ctx, grad):
     batch = grad.shape[1]
     ga = gb = None
     if need_a:   # dA = C (*) B^T
-        da = cauchy_matmul(c, b, degree, not trans_b)
+        if na == 1 and degree > 0 and _sums(c[0], b[0]):   # an ordinary A: coefficient K alone, sum_s C_{K-s} B_s^T
+            da = matmul_order_sum(c[::-1][:nb], b, False, not trans_b)[None]
+        else:
+            da = cauchy_matmul(c, b, degree, not trans_b)
         if a[0].shape[0] == 1 and batch > 1:
             da = da.sum(1, keepdim=True)
         ga = _read_back(da, na)
     if need_b:   # dB = A^T (*) C, or its transpose for a [batch, n, k] operand
-        if trans_b:
+        if nb == 1 and _sums(a[0], c[0]):   # an ordinary B: sum_s A_s^T C_{K-s}
+            gs = c[::-1][:na]
+            db = matmul_order_sum(*((gs, a) if trans_b else (a, gs)), True, False)[None]
+        elif trans_b:
             db = cauchy_matmul([x.transpose(-1, -2).contiguous() for x in c], a, degree, False)
         else:
             db = cauchy_matmul([x.transpose(-1, -2).contiguous() for x in a], c, degree, False)

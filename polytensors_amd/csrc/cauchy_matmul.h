@@ -21,6 +21,20 @@ struct CauchyArgs {
 template <typename T>
 int launch_cauchy(const CauchyArgs& a);
 
+// C = sum_s op(A_s) op(B_s) over `terms` pairs (order_gemm.inl).
+struct OrderSumArgs {
+  int terms;
+  const void* const* a;
+  const void* const* b;
+  void* c;
+  int64_t batch, m, n, k, lda, ldb, a_bs, b_bs;
+  bool trans_a, trans_b;
+  hipStream_t stream;
+};
+
+template <typename T>
+int launch_order_sum(const OrderSumArgs& a);   // float, bf16, _Float16
+
 // bfloat16 / float16 operands on the 16x16x32 MFMAs (cauchy_matmul_half.inl); T = bf16 or _Float16.
 template <typename T>
 int launch_cauchy_half(const CauchyArgs& a);

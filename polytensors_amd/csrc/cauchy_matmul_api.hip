@@ -42,4 +42,30 @@ int pt_cauchy_matmul(int dtype, int degree, const void* const* a, int a_orders,
   }
 }
 
+int pt_matmul_order_sum(int dtype, int terms, const void* const* a, const void* const* b, void* c, int64_t batch,
+                        int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, int64_t a_batch_stride,
+                        int64_t b_batch_stride, int trans_a, int trans_b, void* stream) {
+  pt_host::clear_error();
+  PT_REQUIRE(terms >= 1 && terms <= PT_MAX_DEGREE + 1, PT_INVALID_ARGUMENT, "matmul order sum: terms must be in 1..9");
+  PT_REQUIRE(dtype == PT_FLOAT32 || dtype == PT_BFLOAT16 || dtype == PT_FLOAT16, PT_UNSUPPORTED,
+             "matmul order sum: float32, bfloat16 or float16");
+  PT_REQUIRE(!(trans_a && trans_b), PT_UNSUPPORTED, "matmul order sum: trans_a needs trans_b = 0");
+  PT_REQUIRE(batch >= 0 && m >= 0 && n >= 0 && k >= 0 && a_batch_stride >= 0 && b_batch_stride >= 0, PT_INVALID_ARGUMENT,
+             "matmul order sum: negative size or batch stride");
+  PT_REQUIRE(lda >= (trans_a ? m : k) && ldb >= (trans_b ? k : n), PT_INVALID_ARGUMENT,
+             "matmul order sum: a row stride below the row length");
+  if (batch == 0 || m == 0 || n == 0) return PT_OK;
+  PT_REQUIRE(a != nullptr && b != nullptr && c != nullptr, PT_INVALID_ARGUMENT,
+             "matmul order sum: a, b and c are required");
+  for (int s = 0; s < terms; ++s)
+    PT_REQUIRE((a[s] != nullptr && b[s] != nullptr) || k == 0, PT_INVALID_ARGUMENT, "matmul order sum: null operand");
+  pt::OrderSumArgs args{terms, a, b, c, batch, m, n, k, lda, ldb, a_batch_stride, b_batch_stride,
+                        trans_a != 0, trans_b != 0, static_cast<hipStream_t>(stream)};
+  switch (dtype) {
+    case PT_FLOAT32: return pt::launch_order_sum<float>(args);
+    case PT_BFLOAT16: return pt::launch_order_sum<pt::bf16>(args);
+    default: return pt::launch_order_sum<_Float16>(args);
+  }
+}
+
 }  // extern "C"

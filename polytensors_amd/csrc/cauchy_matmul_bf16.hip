@@ -3,4 +3,5 @@
 
 namespace pt {
 template int launch_cauchy_half<bf16>(const CauchyArgs&);
+template int launch_order_sum<bf16>(const OrderSumArgs&);
 }  // namespace pt

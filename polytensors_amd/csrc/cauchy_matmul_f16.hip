@@ -3,4 +3,5 @@
 
 namespace pt {
 template int launch_cauchy_half<_Float16>(const CauchyArgs&);
+template int launch_order_sum<_Float16>(const OrderSumArgs&);
 }  // namespace pt

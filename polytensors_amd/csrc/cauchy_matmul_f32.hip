@@ -3,4 +3,5 @@
 
 namespace pt {
 template int launch_cauchy<float>(const CauchyArgs&);
+template int launch_order_sum<float>(const OrderSumArgs&);
 }  // namespace pt

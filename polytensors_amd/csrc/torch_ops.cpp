@@ -294,6 +294,46 @@ Tensor cauchy_matmul(const TensorList& a_in, const TensorList& b_in, int64_t deg
   return out.narrow(-1, 0, n_out).contiguous();
 }
 
+// sum_s op(a_s) op(b_s) over pairs of [batch, rows, cols] matrices (float32, bfloat16, float16).
+Tensor matmul_order_sum(const TensorList& a_in, const TensorList& b_in, bool trans_a, bool trans_b) {
+  check_abi();
+  for (const auto& [name, s] : {std::pair<const char*, const TensorList*>{"a", &a_in}, {"b", &b_in}}) {
+    check_series(std::string("matmul_order_sum ") + name, *s);
+    TORCH_CHECK_VALUE((*s)[0].dim() == 3, "matmul_order_sum: ", name, " must be 3-D [batch, rows, cols]");
+  }
+  const Tensor &a0 = a_in[0], &b0 = b_in[0];
+  TORCH_CHECK_VALUE(a_in.size() == b_in.size(), "matmul_order_sum: a and b need the same number of matrices");
+  TORCH_CHECK_VALUE(b0.scalar_type() == a0.scalar_type() && b0.device() == a0.device(),
+                    "matmul_order_sum: operand dtype/device differ");
+  const int64_t ba = a0.size(0), bb = b0.size(0);
+  const int64_t m = a0.size(trans_a ? 2 : 1), n = b0.size(trans_b ? 1 : 2);
+  int64_t k = a0.size(trans_a ? 1 : 2);
+  TORCH_CHECK_VALUE(b0.size(trans_b ? 2 : 1) == k, "matmul_order_sum: inner dimensions differ");
+  TORCH_CHECK_VALUE(ba == bb || ba == 1 || bb == 1, "matmul_order_sum: batch dimensions do not broadcast");
+  const int64_t batch = std::max(ba, bb);
+  c10::DeviceGuard guard(a0.device());
+  // rows of whole 16-byte vectors (zeros past a contraction leave the sum unchanged; columns past m
+  // or n take no part)
+  const int64_t vec = 16 / static_cast<int64_t>(a0.element_size());
+  TensorList a = a_in, b = b_in;
+  for (Tensor& t : a) t = aligned16(pad_dim(t, -1, vec));
+  for (Tensor& t : b) t = aligned16(pad_dim(t, -1, vec));
+  const int64_t lda = a[0].size(2), ldb = b[0].size(2);
+  if (!trans_a && trans_b) k = lda;   // both padded along the contraction
+  if (!trans_a && !trans_b && lda != k) {   // a's padding needs as many rows of b
+    for (Tensor& t : b) t = pad_dim(t, -2, vec);
+    k = lda;
+  }
+  Tensor out = at::empty({batch, m, n}, a0.options());
+  auto as = cptrs(a), bs = cptrs(b);
+  const int status = pt_matmul_order_sum(
+      dtype_code(a0.scalar_type()), static_cast<int>(a.size()), as.data(), bs.data(), out.data_ptr(), batch, m, n, k, lda,
+      ldb, ba == 1 ? 0 : a[0].size(1) * lda, bb == 1 ? 0 : b[0].size(1) * ldb, trans_a ? 1 : 0, trans_b ? 1 : 0,
+      stream_of(a0));
+  check_status(status, "matmul_order_sum");
+  return out;
+}
+
 // ---- Taylor attention --------------------------------------------------------
 
 // An attention mask as the kernels take it: the boolean mask of the admissible entries (a
@@ -623,6 +663,7 @@ TORCH_LIBRARY(polytensors_amd, m) {
   m.def("cross_entropy_series_backward(Tensor[] z, Tensor target, int ignore_index, float softcap, Tensor lse, "
         "Tensor[] cot) -> Tensor");
   m.def("cauchy_matmul(Tensor[] a, Tensor[] b, int degree, bool trans_b) -> Tensor");
+  m.def("matmul_order_sum(Tensor[] a, Tensor[] b, bool trans_a, bool trans_b) -> Tensor");
   m.def("taylor_attention_fwd(Tensor[] q, Tensor[] k, Tensor[] v, Tensor? mask, bool causal, float scale, "
         "int degree, int[]? mask_map=None) -> (Tensor, Tensor)");
   m.def("taylor_attention_bwd(Tensor[] q, Tensor[] k, Tensor[] v, Tensor out, Tensor lse, Tensor[] grad, "
@@ -640,6 +681,7 @@ TORCH_LIBRARY_IMPL(polytensors_amd, CUDA, m) {
   m.impl("cross_entropy_series", &cross_entropy_series);
   m.impl("cross_entropy_series_backward", &cross_entropy_series_backward);
   m.impl("cauchy_matmul", &cauchy_matmul);
+  m.impl("matmul_order_sum", &matmul_order_sum);
   m.impl("taylor_attention_fwd", &taylor_attention_fwd);
   m.impl("taylor_attention_bwd", &taylor_attention_bwd);
   m.impl("complex_to_real", &complex_to_real);

@@ -271,3 +271,31 @@ def test_float32_attention_and_cross_entropy_pipeline():
         return oracle.cross_entropy(logits, y)
 
     _compare(dev, cpu, qkv, seed=95, tol=1e-4)
+
+
+# The gradient of an ordinary matrix operand (one order of a series product, matmul_order_sum) at the
+# edges of its tiles (64, 128, 256), contractions around its chunks (16 floats, 32 halves), rows no
+# 16-byte vector divides, a batch it is shared over, on either side of the product.
+# Tolerance: one rounding of a float32 sum of (K + 1) m products (below 1e-5 of the largest value here).
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -11 + 1e-5)])
+@pytest.mark.parametrize("m,k,n,batch,degree", [
+    (1, 8, 16, (), 1), (33, 64, 64, (), 3), (128, 128, 256, (), 2), (65, 129, 31, (), 4), (300, 257, 136, (), 8),
+    (40, 24, 72, (3,), 2), (2000, 512, 520, (), 3), (17, 5, 3, (2,), 0)])
+def test_gradient_of_an_ordinary_matrix(dtype, tol, m, k, n, batch, degree):
+    g = torch.Generator().manual_seed(m + 3 * k + n)
+    make = lambda *shape: torch.randn(*shape, generator=g, dtype=torch.float64).to(dtype)   # noqa: E731
+    X, Y = ([make(*batch, *shape) for _ in range(degree + 1)] for shape in ((m, k), (k, n)))
+    C = [make(*batch, m, n) for _ in range(degree + 1)]
+    cases = {"x @ W": (lambda x, w: x @ w, X, make(k, n), lambda a, w: a @ w),
+             "linear": (lambda x, w: torch.nn.functional.linear(x, w), X, make(n, k), lambda a, w: a @ w.transpose(-1, -2)),
+             "W @ y": (lambda y, w: w @ y, Y, make(m, k), lambda b, w: w @ b)}
+    for name, (call, series, W, plain) in cases.items():
+        w = W.cuda().requires_grad_()
+        with PolyTensor.plain_range(), PolyTensor.coefficient_autograd():
+            out = call(PolyTensor(tuple(c.cuda() for c in series)), w)
+        (got,) = torch.autograd.grad(out.coeffs, w, [c.cuda() for c in C])
+        wd = W.double().requires_grad_()
+        (want,) = torch.autograd.grad([plain(c.double(), wd) for c in series], wd, [c.double() for c in C])
+        # (a batch's gradients are rounded before they are summed)
+        err = (got.cpu().double() - want).abs().max() / want.abs().max()
+        assert err <= tol * (2 if batch else 1), (name, err)
