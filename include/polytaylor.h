@@ -227,6 +227,26 @@ int pt_cauchy_matmul(int dtype, int degree, const void* const* a, int a_orders,
                      int trans_b, void* stream);
 
 /*
+ * pt_cauchy_matmul of operands with row strides: rows of a lda elements apart, of b ldb (both at
+ * least the row length). Where lda (ldb) is a multiple of a 16-byte vector and the rows of a (of b
+ * if trans_b) run along k, the values from k to the next multiple of a vector must be zero; b's
+ * values past n (not trans_b) take no part. So 16-bit operands of any k and n run with padded rows
+ * (pt_pack_rows): here the 16-bit kernels need lda and ldb, not k and n, to be multiples of 8.
+ */
+int pt_cauchy_matmul_strided(int dtype, int degree, const void* const* a, int a_orders,
+                             const void* const* b, int b_orders, void* const* c,
+                             int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,
+                             int64_t a_batch_stride, int64_t b_batch_stride, int trans_b, void* stream);
+
+/*
+ * Copies `count` (1..9) contiguous [rows, cols] matrices of 2-, 4- or 8-byte elements, at any
+ * element's address, into [rows, dst_cols] ones (dst_cols >= cols, 16-byte aligned, rows of whole
+ * 16-byte vectors) with zeros past cols, in one launch.
+ */
+int pt_pack_rows(int elem_bytes, int count, const void* const* src, void* const* dst, int64_t rows,
+                 int64_t cols, int64_t dst_cols, void* stream);
+
+/*
  * One order of a product of series: the sum C = sum_s op(A_s) @ op(B_s) over `terms` (1..9) pairs
  * of matrices, the gradient of an ordinary operand of pt_cauchy_matmul (the cotangent of its one
  * order, /root/reference/src/polytensors/_plain.py:118-128 read in reverse), in one launch.
@@ -236,9 +256,9 @@ int pt_cauchy_matmul(int dtype, int degree, const void* const* a, int a_orders,
  * c: [batch, m, n] contiguous.
  * dtype: PT_FLOAT32, PT_BFLOAT16 or PT_FLOAT16 (fp32 accumulation, each element rounded once).
  * Rows are read in 16-byte vectors: operands 16-byte aligned, row and batch strides multiples of 16
- * bytes, and so k where an operand's rows run along it (a unless trans_a, b if trans_b; the vectors
- * past m or n of an operand whose rows run along those are read inside the row stride, and take no
- * part); each matrix below 1 GiB, else PT_UNSUPPORTED. trans_a needs trans_b = 0.
+ * bytes, each matrix (its rows times the row stride) below 1 GiB, else PT_UNSUPPORTED. The values of a
+ * row from its length to the next multiple of a vector are zeros where it runs along k, and take no
+ * part where it runs along m or n. trans_a needs trans_b = 0.
  */
 int pt_matmul_order_sum(int dtype, int terms, const void* const* a, const void* const* b, void* c,
                         int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,

@@ -55,6 +55,9 @@ SIGNATURES = {
     "pt_cross_entropy_series_noalloc_max_bytes": (ctypes.c_size_t, []),
     "pt_cauchy_matmul": (_c_int, [_c_int, _c_int, _c_vpp, _c_int, _c_vpp, _c_int, _c_vpp,
                                   _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_vp]),
+    "pt_cauchy_matmul_strided": (_c_int, [_c_int, _c_int, _c_vpp, _c_int, _c_vpp, _c_int, _c_vpp, _c_i64, _c_i64, _c_i64,
+                                          _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_vp]),
+    "pt_pack_rows": (_c_int, [_c_int, _c_int, _c_vpp, _c_vpp, _c_i64, _c_i64, _c_i64, _c_vp]),
     "pt_matmul_order_sum": (_c_int, [_c_int, _c_int, _c_vpp, _c_vpp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
                                      _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_vp]),
     "pt_taylor_attention_fwd": (_c_int, [_c_int, _c_int, _c_vpp, _c_int, _c_vpp, _c_int, _c_vpp, _c_int,

@@ -13,9 +13,12 @@ struct CauchyArgs {
   int b_orders;
   void* const* c;
   int64_t batch, m, n, k;
+  int64_t lda, ldb;   // row strides; zeros from k to the next 16-byte vector where rows run along k
   int64_t a_bs, b_bs;
   bool trans_b;
   hipStream_t stream;
+  int64_t rows_b() const { return trans_b ? n : k; }
+  int64_t width_b() const { return trans_b ? k : n; }
 };
 
 template <typename T>
@@ -31,6 +34,10 @@ struct OrderSumArgs {
   bool trans_a, trans_b;
   hipStream_t stream;
 };
+
+// Copies of `count` [rows, cols] matrices with rows padded by zeros to dst_cols (cauchy_matmul_api.hip).
+int launch_pack_rows(int elem_bytes, int count, const void* const* src, void* const* dst, int64_t rows, int64_t cols,
+                     int64_t dst_cols, hipStream_t stream);
 
 template <typename T>
 int launch_order_sum(const OrderSumArgs& a);   // float, bf16, _Float16

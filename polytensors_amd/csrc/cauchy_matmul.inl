@@ -73,7 +73,7 @@ template <typename T, int K, int AO, int BO, int BM, int BN, int BK, int WAVES_M
           int MIN_WAVES, bool TRANS_B, bool VEC>
 __global__ __launch_bounds__(WAVES_M * WAVES_N * kWave) __attribute__((amdgpu_waves_per_eu(MIN_WAVES)))
 void cauchy_matmul_kernel(
-    CPtrs<T> A, CPtrs<T> B, MPtrs<T> C, int M, int N, int Kd, int64_t a_bs, int64_t b_bs) {
+    CPtrs<T> A, CPtrs<T> B, MPtrs<T> C, int M, int N, int Kd, int lda, int ldb, int64_t a_bs, int64_t b_bs) {
   using MF = Mfma<T>;
   using acc_t = typename MF::acc_t;
   constexpr int THREADS = WAVES_M * WAVES_N * kWave;
@@ -118,8 +118,8 @@ void cauchy_matmul_kernel(
       for (int it = 0; it < NA; ++it) {
         const int v = it * THREADS + threadIdx.x;
         const int gr = tile_m + v / (BK / V), gk = k0 + (v % (BK / V)) * V;
-        const T* p = a_base[o] + static_cast<int64_t>(gr) * Kd + gk;
-        if constexpr (VEC) {   // Kd % V == 0: a vector is wholly inside or outside
+        const T* p = a_base[o] + static_cast<int64_t>(gr) * lda + gk;
+        if constexpr (VEC) {   // a vector that starts inside is whole: lda % V == 0, zeros past Kd
           if (gr < M && gk < Kd) {
             ra[o][it] = load_vec<T, V>(p);
           } else {
@@ -138,7 +138,7 @@ void cauchy_matmul_kernel(
         const int v = it * THREADS + threadIdx.x;
         if constexpr (TRANS_B) {   // B stored [N][Kd]
           const int gn = tile_n + v / (BK / V), gk = k0 + (v % (BK / V)) * V;
-          const T* p = b_base[o] + static_cast<int64_t>(gn) * Kd + gk;
+          const T* p = b_base[o] + static_cast<int64_t>(gn) * ldb + gk;
           if constexpr (VEC) {
             if (gn < N && gk < Kd) {
               rb[o][it] = load_vec<T, V>(p);
@@ -152,8 +152,8 @@ void cauchy_matmul_kernel(
           }
         } else {                   // B stored [Kd][N]: a vector runs along n
           const int gk = k0 + v / (BN / V), gn = tile_n + (v % (BN / V)) * V;
-          const T* p = b_base[o] + static_cast<int64_t>(gk) * N + gn;
-          if constexpr (VEC) {     // N % V == 0
+          const T* p = b_base[o] + static_cast<int64_t>(gk) * ldb + gn;
+          if constexpr (VEC) {     // ldb % V == 0 (columns past N are not stored)
             if (gk < Kd && gn < N) {
               rb[o][it] = load_vec<T, V>(p);
             } else {
@@ -303,9 +303,10 @@ static int launch_cauchy_orders(const CauchyArgs& a, const CPtrs<T>& A, const CP
   const dim3 grid((a.n + Tile::BN - 1) / Tile::BN, (a.m + Tile::BM - 1) / Tile::BM, a.batch);
   const dim3 block(Tile::WAVES_M * Tile::WAVES_N * kWave);
   const int M = static_cast<int>(a.m), N = static_cast<int>(a.n), Kd = static_cast<int>(a.k);
+  const int lda = static_cast<int>(a.lda), ldb = static_cast<int>(a.ldb);
 #define PT_CAUCHY_LAUNCH(TB, VV)                                                                   \
   cauchy_matmul_kernel<T, K, AO, BO, Tile::BM, Tile::BN, Tile::BK, Tile::WAVES_M, Tile::WAVES_N, \
-                       Tile::MIN_WAVES, TB, VV><<<grid, block, 0, a.stream>>>(A, B, C, M, N, Kd, a.a_bs, a.b_bs)
+                       Tile::MIN_WAVES, TB, VV><<<grid, block, 0, a.stream>>>(A, B, C, M, N, Kd, lda, ldb, a.a_bs, a.b_bs)
   if (a.trans_b) {
     if (vec) PT_CAUCHY_LAUNCH(true, true);
     else PT_CAUCHY_LAUNCH(true, false);
@@ -333,7 +334,7 @@ static int launch_cauchy_k(const CauchyArgs& a) {
     vec = vec && pt_host::aligned16(a.b[o]);
   }
   for (int o = 0; o <= K; ++o) C.p[o] = static_cast<T*>(a.c[o]);
-  vec = vec && a.k % V == 0 && a.a_bs % V == 0 && a.b_bs % V == 0 && (a.trans_b || a.n % V == 0);
+  vec = vec && a.lda % V == 0 && a.ldb % V == 0 && a.a_bs % V == 0 && a.b_bs % V == 0;
   const bool a_series = a.a_orders > 1, b_series = a.b_orders > 1;
   auto zero_higher = [&](int st) -> int {   // two ordinary operands: C_0 = A_0 B_0, zero higher orders
     if (st != PT_OK || K == 0) return st;

@@ -30,8 +30,10 @@
 //   column n per lane) is two ds_read_b64_tr_b16 transpose reads, lane 4j + a
 //   of group g addressing row 8g + j (then 8g + 4 + j), columns n0 + 4a .. + 3.
 // Rows past M / N and contraction chunks past Kd are out of the DMA's range and
-// load as zeros (the launcher requires Kd and, for B stored [k][n], N to be
-// multiples of 8, so a 16-byte chunk is wholly inside or outside).
+// load as zeros. Row strides are multiples of 8 elements, and rows along the
+// contraction hold zeros from Kd to the next multiple, so a chunk is whole
+// wherever it starts inside; columns of B past N (row stride past it) reach
+// only elements of C that are not stored.
 #pragma once
 
 #include <algorithm>
@@ -69,7 +71,7 @@ __host__ __device__ __forceinline__ int cauchy_swz_k(int k, int ch) {
 
 template <typename T, int K, int AO, int BO, bool TRANS_B, bool WIDE>
 __global__ __launch_bounds__((CauchyHalfTile<AO, BO, WIDE>::kThreads)) void cauchy_matmul_half_kernel(
-    CPtrs<T> A, CPtrs<T> B, MPtrs<T> C, int M, int N, int Kd, int64_t a_bs, int64_t b_bs, int c_vec) {
+    CPtrs<T> A, CPtrs<T> B, MPtrs<T> C, int M, int N, int Kd, int lda, int ldb, int64_t a_bs, int64_t b_bs) {
   using Tile = CauchyHalfTile<AO, BO, WIDE>;
   using MM = HalfMfma<T>;
   constexpr int BM = Tile::BM, BN = Tile::BN, BK = Tile::BK, FM = Tile::FM, FN = Tile::FN;
@@ -86,8 +88,8 @@ __global__ __launch_bounds__((CauchyHalfTile<AO, BO, WIDE>::kThreads)) void cauc
   const int wm = wave / Tile::WNW, wn = wave % Tile::WNW;
   const int tile_m = blockIdx.y * BM, tile_n = blockIdx.x * BN;
   const int64_t batch = blockIdx.z;
-  const int a_bytes = M * Kd * static_cast<int>(sizeof(T));
-  const int b_bytes = Kd * N * static_cast<int>(sizeof(T));
+  const int a_bytes = M * lda * static_cast<int>(sizeof(T));
+  const int b_bytes = (TRANS_B ? N : Kd) * ldb * static_cast<int>(sizeof(T));
 
   // DMA of chunk k0 into buffer buf: this wave moves segment `wave` (1 KB) of every order tile
   auto issue = [&](int buf, int k0) {
@@ -95,7 +97,7 @@ __global__ __launch_bounds__((CauchyHalfTile<AO, BO, WIDE>::kThreads)) void cauc
       const int row = 16 * wave + lane / 4;
       const int lch = cauchy_swz_rows(row, lane % 4);
       const int gm = tile_m + row, gk = k0 + 8 * lch;
-      const int voff = (gm < M && gk < Kd) ? (gm * Kd + gk) * static_cast<int>(sizeof(T)) : kBufferOutOfRange;
+      const int voff = (gm < M && gk < Kd) ? (gm * lda + gk) * static_cast<int>(sizeof(T)) : kBufferOutOfRange;
 #pragma unroll
       for (int o = 0; o < AO; ++o)
         lds_dma16(&As[buf][o][512 * wave], buffer_rsrc(A.p[o] + batch * a_bs, a_bytes), voff);
@@ -105,12 +107,12 @@ __global__ __launch_bounds__((CauchyHalfTile<AO, BO, WIDE>::kThreads)) void cauc
       const int row = 16 * wave + lane / 4;
       const int lch = cauchy_swz_rows(row, lane % 4);
       const int gn = tile_n + row, gk = k0 + 8 * lch;
-      voff = (gn < N && gk < Kd) ? (gn * Kd + gk) * static_cast<int>(sizeof(T)) : kBufferOutOfRange;
+      voff = (gn < N && gk < Kd) ? (gn * ldb + gk) * static_cast<int>(sizeof(T)) : kBufferOutOfRange;
     } else {                   // B stored [Kd][N]: k rows (64 / CPR) wave + lane / CPR, physical chunk lane % CPR
       const int kr = (64 / CPR) * wave + lane / CPR;
       const int lch = cauchy_swz_k<WIDE>(kr, lane % CPR);
       const int gk = k0 + kr, gn = tile_n + 8 * lch;
-      voff = (gk < Kd && gn < N) ? (gk * N + gn) * static_cast<int>(sizeof(T)) : kBufferOutOfRange;
+      voff = (gk < Kd && gn < N) ? (gk * ldb + gn) * static_cast<int>(sizeof(T)) : kBufferOutOfRange;
     }
 #pragma unroll
     for (int o = 0; o < BO; ++o)
@@ -200,7 +202,6 @@ __global__ __launch_bounds__((CauchyHalfTile<AO, BO, WIDE>::kThreads)) void cauc
   __builtin_amdgcn_s_waitcnt(0);
 
   // ---- epilogue: lane (c, g) holds C[m0 + c][n0 + 4g .. + 3] of each block ----
-  const bool vec = c_vec != 0;   // N % 4 == 0 and every C_k 8-byte aligned: 8-byte stores
 #pragma unroll
   for (int o = 0; o <= K; ++o) {
     T* base = C.p[o] + batch * static_cast<int64_t>(M) * N;
@@ -213,11 +214,12 @@ __global__ __launch_bounds__((CauchyHalfTile<AO, BO, WIDE>::kThreads)) void cauc
         if (row >= M) continue;
         const floatx4 v = acc[o][fm][fn];
         T* p = base + static_cast<int64_t>(row) * N + col;
-        if (vec && col + 3 < N) {
-          *reinterpret_cast<uint2*>(p) = make_uint2(MM::pack2(v[0], v[1]), MM::pack2(v[2], v[3]));
+        const uint32_t w01 = MM::pack2(v[0], v[1]), w23 = MM::pack2(v[2], v[3]);
+        if (col + 3 < N) {   // at any element: one 8-byte store
+          const uint2 w = make_uint2(w01, w23);
+          __builtin_memcpy(p, &w, sizeof(w));
         } else {
           uint16_t* q = reinterpret_cast<uint16_t*>(p);
-          const uint32_t w01 = MM::pack2(v[0], v[1]), w23 = MM::pack2(v[2], v[3]);
           if (col < N) q[0] = static_cast<uint16_t>(w01);
           if (col + 1 < N) q[1] = static_cast<uint16_t>(w01 >> 16);
           if (col + 2 < N) q[2] = static_cast<uint16_t>(w23);
@@ -242,14 +244,13 @@ static int launch_cauchy_half_tile(const CauchyArgs& a, const CPtrs<T>& A, const
   const dim3 grid((a.n + Tile::BN - 1) / Tile::BN, (a.m + Tile::BM - 1) / Tile::BM, a.batch);
   const dim3 block(Tile::kThreads);
   const int M = static_cast<int>(a.m), N = static_cast<int>(a.n), Kd = static_cast<int>(a.k);
-  int c_vec = N % 4 == 0;
-  for (int o = 0; o <= K; ++o) c_vec = c_vec && reinterpret_cast<uintptr_t>(C.p[o]) % 8 == 0;
+  const int lda = static_cast<int>(a.lda), ldb = static_cast<int>(a.ldb);
   if (a.trans_b)
     cauchy_matmul_half_kernel<T, K, AO, BO, true, WIDE>
-        <<<grid, block, 0, a.stream>>>(A, B, C, M, N, Kd, a.a_bs, a.b_bs, c_vec);
+        <<<grid, block, 0, a.stream>>>(A, B, C, M, N, Kd, lda, ldb, a.a_bs, a.b_bs);
   else
     cauchy_matmul_half_kernel<T, K, AO, BO, false, WIDE>
-        <<<grid, block, 0, a.stream>>>(A, B, C, M, N, Kd, a.a_bs, a.b_bs, c_vec);
+        <<<grid, block, 0, a.stream>>>(A, B, C, M, N, Kd, lda, ldb, a.a_bs, a.b_bs);
   PT_LAUNCH_CHECK();
   return PT_OK;
 }
@@ -292,17 +293,17 @@ static int launch_cauchy_half_ordinary(const CauchyArgs& a) {
 
 template <typename T>
 int launch_cauchy_half(const CauchyArgs& a) {
-  // 16-byte DMA chunks: whole chunks of the contraction (and of N for B stored [k][n]), aligned
-  // operands and batch strides, and each batch's matrix addressable with 32-bit offsets
+  // 16-byte DMA chunks: rows and batch strides of whole chunks, aligned operands, and each batch's
+  // matrix addressable with 32-bit offsets
   constexpr int64_t kLimit = int64_t{1} << 30;
-  bool ok = a.k % 8 == 0 && (a.trans_b || a.n % 8 == 0) && a.a_bs % 8 == 0 && a.b_bs % 8 == 0 &&
-            a.m * a.k * 2 < kLimit && a.k * a.n * 2 < kLimit;
+  bool ok = a.lda % 8 == 0 && a.ldb % 8 == 0 && a.a_bs % 8 == 0 && a.b_bs % 8 == 0 && a.lda < kLimit && a.ldb < kLimit &&
+            a.m * a.lda * 2 < kLimit && a.rows_b() * a.ldb * 2 < kLimit;
   for (int o = 0; o < a.a_orders; ++o) ok = ok && pt_host::aligned16(a.a[o]);
   for (int o = 0; o < a.b_orders; ++o) ok = ok && pt_host::aligned16(a.b[o]);
   if (!ok) {
     pt_host::set_error(
-        "Cauchy matmul (16-bit): needs the contraction size (and n unless trans_b) to be multiples of 8, "
-        "16-byte aligned operands and batch strides, and each matrix below 1 GiB");
+        "Cauchy matmul (16-bit): needs row strides (k, and n unless trans_b, without strides given) and batch strides "
+        "to be multiples of 8, 16-byte aligned operands, and each matrix below 1 GiB");
     return PT_UNSUPPORTED;
   }
   if (a.a_orders == 1 || a.b_orders == 1) {

@@ -105,7 +105,7 @@ template <typename T>
 struct OrderGemmParams {
   CPtrs<T> a, b;
   MPtrs<T> c;
-  int m, n, k;                  // of one order; k a whole number of 16-byte vectors where it runs along rows
+  int m, n, k;                  // of one order; zeros from k to the next 16-byte vector where it runs along rows
   int lda, ldb;                 // row strides in elements
   int a_bytes, b_bytes;         // extent of one matrix
   int64_t a_bs, b_bs, c_bs;     // batch strides in elements
@@ -334,8 +334,8 @@ void order_gemm_kernel(OrderGemmParams<T> p) {
 template <typename T>
 static bool order_gemm_takes(const CauchyArgs& a) {
   constexpr int64_t V = 16 / static_cast<int64_t>(sizeof(T)), kLimit = (int64_t{1} << 30) / static_cast<int64_t>(sizeof(T));
-  bool ok = a.k % V == 0 && (a.trans_b || a.n % V == 0) && a.a_bs % V == 0 && a.b_bs % V == 0 &&
-            a.m * a.k < kLimit && a.k * a.n < kLimit &&
+  bool ok = a.lda % V == 0 && a.ldb % V == 0 && a.a_bs % V == 0 && a.b_bs % V == 0 && a.lda < kLimit && a.ldb < kLimit &&
+            a.m * a.lda < kLimit && a.rows_b() * a.ldb < kLimit &&
             ((a.m + 63) / 64) * ((a.n + 63) / 64) * std::max(a.a_orders, a.b_orders) * a.batch <= INT32_MAX;
   for (int o = 0; o < a.a_orders; ++o) ok = ok && pt_host::aligned16(a.a[o]);
   for (int o = 0; o < a.b_orders; ++o) ok = ok && pt_host::aligned16(a.b[o]);
@@ -393,10 +393,10 @@ static int launch_by_order(const CauchyArgs& a, int orders) {
   p.m = static_cast<int>(a.m);
   p.n = static_cast<int>(a.n);
   p.k = static_cast<int>(a.k);
-  p.lda = p.k;
-  p.ldb = a.trans_b ? p.k : p.n;
-  p.a_bytes = static_cast<int>(a.m * a.k * static_cast<int64_t>(sizeof(T)));
-  p.b_bytes = static_cast<int>(a.n * a.k * static_cast<int64_t>(sizeof(T)));
+  p.lda = static_cast<int>(a.lda);
+  p.ldb = static_cast<int>(a.ldb);
+  p.a_bytes = static_cast<int>(a.m * a.lda * static_cast<int64_t>(sizeof(T)));
+  p.b_bytes = static_cast<int>(a.rows_b() * a.ldb * static_cast<int64_t>(sizeof(T)));
   p.a_bs = a.a_bs;
   p.b_bs = a.b_bs;
   p.c_bs = a.m * a.n;
@@ -412,13 +412,13 @@ int launch_order_sum(const OrderSumArgs& a) {
   constexpr int64_t V = 16 / static_cast<int64_t>(sizeof(T)), kLimit = (int64_t{1} << 30) / static_cast<int64_t>(sizeof(T));
   const int64_t rows_a = a.trans_a ? a.k : a.m, rows_b = a.trans_b ? a.n : a.k;
   bool ok = a.lda % V == 0 && a.ldb % V == 0 && a.a_bs % V == 0 && a.b_bs % V == 0 &&
-            (a.k % V == 0 || (a.trans_a && !a.trans_b)) && a.m <= INT32_MAX && a.n <= INT32_MAX && a.k <= INT32_MAX &&
+            a.m <= INT32_MAX && a.n <= INT32_MAX && a.k <= INT32_MAX &&
             a.lda < kLimit && a.ldb < kLimit && rows_a * a.lda < kLimit && rows_b * a.ldb < kLimit &&
             ((a.m + 63) / 64) * ((a.n + 63) / 64) * a.batch <= INT32_MAX;
   for (int s = 0; s < a.terms; ++s) ok = ok && pt_host::aligned16(a.a[s]) && pt_host::aligned16(a.b[s]);
   if (!ok) {
-    pt_host::set_error("matmul order sum: needs 16-byte aligned operands, row and batch strides (and k where rows run "
-                       "along it) of whole 16-byte vectors, and each matrix below 1 GiB");
+    pt_host::set_error("matmul order sum: needs 16-byte aligned operands, row and batch strides of whole 16-byte "
+                       "vectors, and each matrix below 1 GiB");
     return PT_UNSUPPORTED;
   }
   OrderGemmParams<T> p{};

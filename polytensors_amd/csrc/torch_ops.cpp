@@ -233,19 +233,34 @@ Tensor cross_entropy_series_backward(const TensorList& z, const Tensor& target, 
 
 // ---- Cauchy-product matmul ---------------------------------------------------
 
-// x zero-padded at the end of dim to a multiple of `multiple` (x itself if it is one).
-Tensor pad_dim(const Tensor& x, int64_t dim, int64_t multiple) {
-  const int64_t size = x.size(dim);
-  const int64_t extra = (multiple - size % multiple) % multiple;
-  if (extra == 0) return x;
-  std::vector<int64_t> pad(2 * (x.dim() - 1 - ((dim % x.dim() + x.dim()) % x.dim())), 0);
-  pad.push_back(0);
-  pad.push_back(extra);
-  return at::constant_pad_nd(x, pad, 0);
-}
+// Matrices as the 16-byte loads of the matmul kernels take them: rows `stride` elements apart.
+struct Rows {
+  TensorList matrices;
+  int64_t stride;
+};
 
-Tensor aligned16(const Tensor& x) {
-  return reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 ? x : x.clone();
+// Contiguous [batch, rows, cols] matrices with aligned rows: as they are, or, where a row is no whole
+// number of 16-byte vectors or a matrix is not aligned, copied with rows padded by zeros (all orders in
+// one launch). The 16-bit kernels read nothing else; float32 gains by it (4 x 511 x 1023 x 769, degree 4:
+// 704 -> 519 us; 300 x 301 x 1001 by an ordinary matrix, degree 3: 44 -> 26); float64, bound by its
+// MFMAs, does not (1006 -> 973 us there, 57 -> 61 here), and is left to the kernel's element loads.
+Rows packed_rows(const TensorList& in) {
+  const Tensor& first = in[0];
+  const int64_t cols = first.size(2), rows = first.size(0) * first.size(1);
+  const int64_t vec = 16 / static_cast<int64_t>(first.element_size());
+  bool whole = cols % vec == 0 || first.scalar_type() == at::kDouble;
+  for (const Tensor& t : in)
+    whole = whole && (reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 || first.scalar_type() == at::kDouble);
+  if (whole) return {in, cols};
+  const int64_t stride = (cols + vec - 1) / vec * vec;
+  Tensor buffer = at::empty({static_cast<int64_t>(in.size()), first.size(0), first.size(1), stride}, first.options());
+  TensorList out = buffer.unbind(0);
+  auto from = cptrs(in);
+  auto to = slices(buffer);
+  check_status(pt_pack_rows(static_cast<int>(first.element_size()), static_cast<int>(in.size()), from.data(), to.data(),
+                            rows, cols, stride, stream_of(first)),
+               "pack_rows");
+  return {std::move(out), stride};
 }
 
 Tensor cauchy_matmul(const TensorList& a_in, const TensorList& b_in, int64_t degree, bool trans_b) {
@@ -260,38 +275,24 @@ Tensor cauchy_matmul(const TensorList& a_in, const TensorList& b_in, int64_t deg
   TORCH_CHECK_VALUE(b_in[0].scalar_type() == dtype && b_in[0].device() == a_in[0].device(),
                     "cauchy_matmul: operand dtype/device differ");
   const int64_t ba = a_in[0].size(0), m = a_in[0].size(1);
-  int64_t kd = a_in[0].size(2);
+  const int64_t kd = a_in[0].size(2);
   const int64_t bb = b_in[0].size(0);
-  int64_t n = trans_b ? b_in[0].size(1) : b_in[0].size(2);
+  const int64_t n = trans_b ? b_in[0].size(1) : b_in[0].size(2);
   const int64_t kb = trans_b ? b_in[0].size(2) : b_in[0].size(1);
   TORCH_CHECK_VALUE(kb == kd, "cauchy_matmul: inner dimensions differ");
   TORCH_CHECK_VALUE(ba == bb || ba == 1 || bb == 1, "cauchy_matmul: batch dimensions do not broadcast");
   const int64_t batch = std::max(ba, bb);
-  const int64_t n_out = n;
   c10::DeviceGuard guard(a_in[0].device());
-  TensorList a = a_in, b = b_in;
-  if (dtype == at::kBFloat16 || dtype == at::kHalf) {
-    // the 16-bit kernel moves 16-byte chunks: zero-pad the contraction (which leaves every product
-    // unchanged) and, for B stored [k, n], the columns to multiples of 8, and give it 16-byte
-    // aligned operands
-    for (Tensor& t : a) t = aligned16(pad_dim(t, -1, 8));
-    for (Tensor& t : b) t = aligned16(pad_dim(t, trans_b ? -1 : -2, 8));
-    if (!trans_b) {
-      for (Tensor& t : b) t = pad_dim(t, -1, 8);
-      n = b[0].size(2);
-    }
-    kd = a[0].size(2);
-  }
-  Tensor out = at::empty({degree + 1, batch, m, n}, a[0].options());
-  auto as = cptrs(a), bs = cptrs(b);
+  const Rows a = packed_rows(a_in), b = packed_rows(b_in);
+  Tensor out = at::empty({degree + 1, batch, m, n}, a_in[0].options());
+  auto as = cptrs(a.matrices), bs = cptrs(b.matrices);
   auto cs = slices(out);
-  const int status = pt_cauchy_matmul(dtype_code(dtype), static_cast<int>(degree), as.data(),
-                                      static_cast<int>(a.size()), bs.data(), static_cast<int>(b.size()), cs.data(),
-                                      batch, m, n, kd, ba == 1 ? 0 : m * kd, bb == 1 ? 0 : n * kd, trans_b ? 1 : 0,
-                                      stream_of(a[0]));
+  const int status = pt_cauchy_matmul_strided(
+      dtype_code(dtype), static_cast<int>(degree), as.data(), static_cast<int>(a_in.size()), bs.data(),
+      static_cast<int>(b_in.size()), cs.data(), batch, m, n, kd, a.stride, b.stride, ba == 1 ? 0 : m * a.stride,
+      bb == 1 ? 0 : b_in[0].size(1) * b.stride, trans_b ? 1 : 0, stream_of(a_in[0]));
   check_status(status, "cauchy_matmul");
-  if (n == n_out) return out;
-  return out.narrow(-1, 0, n_out).contiguous();
+  return out;
 }
 
 // sum_s op(a_s) op(b_s) over pairs of [batch, rows, cols] matrices (float32, bfloat16, float16).
@@ -307,29 +308,18 @@ Tensor matmul_order_sum(const TensorList& a_in, const TensorList& b_in, bool tra
                     "matmul_order_sum: operand dtype/device differ");
   const int64_t ba = a0.size(0), bb = b0.size(0);
   const int64_t m = a0.size(trans_a ? 2 : 1), n = b0.size(trans_b ? 1 : 2);
-  int64_t k = a0.size(trans_a ? 1 : 2);
+  const int64_t k = a0.size(trans_a ? 1 : 2);
   TORCH_CHECK_VALUE(b0.size(trans_b ? 2 : 1) == k, "matmul_order_sum: inner dimensions differ");
   TORCH_CHECK_VALUE(ba == bb || ba == 1 || bb == 1, "matmul_order_sum: batch dimensions do not broadcast");
   const int64_t batch = std::max(ba, bb);
   c10::DeviceGuard guard(a0.device());
-  // rows of whole 16-byte vectors (zeros past a contraction leave the sum unchanged; columns past m
-  // or n take no part)
-  const int64_t vec = 16 / static_cast<int64_t>(a0.element_size());
-  TensorList a = a_in, b = b_in;
-  for (Tensor& t : a) t = aligned16(pad_dim(t, -1, vec));
-  for (Tensor& t : b) t = aligned16(pad_dim(t, -1, vec));
-  const int64_t lda = a[0].size(2), ldb = b[0].size(2);
-  if (!trans_a && trans_b) k = lda;   // both padded along the contraction
-  if (!trans_a && !trans_b && lda != k) {   // a's padding needs as many rows of b
-    for (Tensor& t : b) t = pad_dim(t, -2, vec);
-    k = lda;
-  }
+  const Rows a = packed_rows(a_in), b = packed_rows(b_in);
   Tensor out = at::empty({batch, m, n}, a0.options());
-  auto as = cptrs(a), bs = cptrs(b);
+  auto as = cptrs(a.matrices), bs = cptrs(b.matrices);
   const int status = pt_matmul_order_sum(
-      dtype_code(a0.scalar_type()), static_cast<int>(a.size()), as.data(), bs.data(), out.data_ptr(), batch, m, n, k, lda,
-      ldb, ba == 1 ? 0 : a[0].size(1) * lda, bb == 1 ? 0 : b[0].size(1) * ldb, trans_a ? 1 : 0, trans_b ? 1 : 0,
-      stream_of(a0));
+      dtype_code(a0.scalar_type()), static_cast<int>(a_in.size()), as.data(), bs.data(), out.data_ptr(), batch, m, n, k,
+      a.stride, b.stride, ba == 1 ? 0 : a0.size(1) * a.stride, bb == 1 ? 0 : b0.size(1) * b.stride, trans_a ? 1 : 0,
+      trans_b ? 1 : 0, stream_of(a0));
   check_status(status, "matmul_order_sum");
   return out;
 }

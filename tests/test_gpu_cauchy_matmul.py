@@ -181,3 +181,28 @@ def test_ordinary_operand_products(dtype, tol, m, k, n, batch, degree):
             want = left @ B[o].double() if name == "L @ y" else A[o].double() @ right
             err = (out.coeffs[o].cpu().double() - want).abs().max() / want.abs().max()
             assert err <= tol, (name, o, err)
+
+
+# Series by series with rows that are no whole 16-byte vectors, or that start at any element: operands
+# copied with padded rows, outputs written at any element, at the edges of the tiles and with operands
+# shared over a batch. Tolerances as above; the sums hold up to (K + 1) k terms.
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.float64, 1e-13), (torch.bfloat16, 2.0 ** -8)])
+@pytest.mark.parametrize("m,k,n,batch_a,batch_b,offset", [
+    (1, 1, 1, (), (), 0), (64, 31, 65, (), (), 1), (257, 33, 259, (2,), (), 0), (300, 65, 511, (), (3,), 3),
+    (65, 128, 64, (), (), 1), (40, 250, 9, (2,), (2,), 0)])
+def test_rows_that_no_vector_divides(dtype, tol, m, k, n, batch_a, batch_b, offset):
+    g, degree = torch.Generator().manual_seed(m + k + n), 3
+    A = [torch.randn(*batch_a, m, k, generator=g, dtype=torch.float64).to(dtype) for _ in range(degree + 1)]
+    B = [torch.randn(*batch_b, k, n, generator=g, dtype=torch.float64).to(dtype) for _ in range(degree + 1)]
+
+    def placed(c):   # on the device, `offset` elements past an aligned address
+        buffer = torch.zeros(c.numel() + offset, dtype=dtype, device="cuda")
+        buffer[offset:] = c.flatten().cuda()
+        return buffer[offset:].view(c.shape)
+
+    with torch.no_grad(), PolyTensor.plain_range():
+        out = PolyTensor(tuple(placed(c) for c in A)) @ PolyTensor(tuple(placed(c) for c in B))
+    want = oracle.matmul([c.double() for c in A], [c.double() for c in B])
+    for o in range(degree + 1):
+        err = (out.coeffs[o].cpu().double() - want[o]).abs().max() / want[o].abs().max()
+        assert err <= tol, (o, err)
