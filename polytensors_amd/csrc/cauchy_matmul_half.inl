@@ -256,11 +256,17 @@ static int launch_cauchy_half_tile(const CauchyArgs& a, const CPtrs<T>& A, const
 }
 
 // The wide tile where its LDS fits, its (K+1) x 32 accumulator registers leave room for the
-// operands within 256 (K <= 4), and both output sides span at least two of its tiles.
+// operands within 256 (K <= 4), and its rounds over the chip take less time: a round of up to 256
+// wide tiles (one a CU) takes 1.56 times one of up to 512 narrow ones (two a CU; 0.60 with one), from
+// 4096^3 at degree 4: 4 rounds of wide tiles 1.367 ms, 8 of narrow ones 1.750 ms.
 template <typename T, int K, int AO, int BO>
 static int launch_cauchy_half_orders(const CauchyArgs& a, const CPtrs<T>& A, const CPtrs<T>& B, const MPtrs<T>& C) {
   if constexpr (K <= 4 && CauchyHalfTile<AO, BO, true>::LDS <= 160 * 1024) {
-    if (a.m >= 256 && a.n >= 256) return launch_cauchy_half_tile<T, K, AO, BO, true>(a, A, B, C);
+    auto tiles = [&](int64_t side) { return (a.m + side - 1) / side * ((a.n + side - 1) / side) * a.batch; };
+    const int64_t rest = tiles(64) % 512;
+    const double wide = 1.56 * static_cast<double>((tiles(128) + 255) / 256);
+    const double narrow = static_cast<double>(tiles(64) / 512) + (rest == 0 ? 0.0 : rest <= 256 ? 0.6 : 1.0);
+    if (wide < narrow) return launch_cauchy_half_tile<T, K, AO, BO, true>(a, A, B, C);
   }
   return launch_cauchy_half_tile<T, K, AO, BO, false>(a, A, B, C);
 }
