@@ -244,6 +244,8 @@ struct Rows {
 // one launch). The 16-bit kernels read nothing else; float32 gains by it (4 x 511 x 1023 x 769, degree 4:
 // 704 -> 519 us; 300 x 301 x 1001 by an ordinary matrix, degree 3: 44 -> 26); float64, bound by its
 // MFMAs, does not (1006 -> 973 us there, 57 -> 61 here), and is left to the kernel's element loads.
+// Rows of 512 bytes and more are padded to whole 128-byte cache lines: a tile's row segments of 64 to
+// 256 bytes otherwise straddle lines (4 x 511 x 1023 x 769 bfloat16, degree 4: 85 -> 77 us).
 Rows packed_rows(const TensorList& in) {
   const Tensor& first = in[0];
   const int64_t cols = first.size(2), rows = first.size(0) * first.size(1);
@@ -252,7 +254,8 @@ Rows packed_rows(const TensorList& in) {
   for (const Tensor& t : in)
     whole = whole && (reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 || first.scalar_type() == at::kDouble);
   if (whole) return {in, cols};
-  const int64_t stride = (cols + vec - 1) / vec * vec;
+  const int64_t unit = cols * static_cast<int64_t>(first.element_size()) >= 512 ? 8 * vec : vec;
+  const int64_t stride = (cols + unit - 1) / unit * unit;
   Tensor buffer = at::empty({static_cast<int64_t>(in.size()), first.size(0), first.size(1), stride}, first.options());
   TensorList out = buffer.unbind(0);
   auto from = cptrs(in);
