@@ -232,11 +232,15 @@ int pt_cauchy_matmul(int dtype, int degree, const void* const* a, int a_orders,
  * if trans_b) run along k, the values from k to the next multiple of a vector must be zero; b's
  * values past n (not trans_b) take no part. So 16-bit operands of any k and n run with padded rows
  * (pt_pack_rows): here the 16-bit kernels need lda and ldb, not k and n, to be multiples of 8.
+ * bias: null, or n values of `dtype` (any alignment) added to every row of C_0 before it is rounded
+ *       (the bias of a linear layer, an ordinary tensor, adds to the constant order:
+ *       /root/reference/src/polytensors/_range_ops.py:109-132).
  */
 int pt_cauchy_matmul_strided(int dtype, int degree, const void* const* a, int a_orders,
                              const void* const* b, int b_orders, void* const* c,
                              int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,
-                             int64_t a_batch_stride, int64_t b_batch_stride, int trans_b, void* stream);
+                             int64_t a_batch_stride, int64_t b_batch_stride, int trans_b, const void* bias,
+                             void* stream);
 
 /*
  * Copies `count` (1..9) contiguous [rows, cols] matrices of 2-, 4- or 8-byte elements, at any

@@ -318,13 +318,24 @@ def complex_quotient(divide, multiply, a, b):
     return _join(divide(nr, denominator), None if ni is None else divide(ni, denominator))
 
 
+def one_product(a, b):
+    """Whether ``bilinear`` of a matrix product runs as one real product: one complex-direction
+    series with a real constant term and one real ordinary tensor, 2K + 1 planes within the
+    kernel's degree."""
+    ac = _is_complex_series(a)
+    x, other = (a, b) if ac else (b, a)
+    return (_is_complex_series(x) and not isinstance(other, PolyTensor) and not has_complex_base(a, b)
+            and 2 * x.degree <= _gate.MAX_DEGREE)
+
+
 def bilinear(fn, what, a, b, *rest, **kwargs):
     """``fn(a, b, ...)`` for an operation bilinear in the series a, b (Cauchy products).
 
-    With one complex-direction series and one ordinary tensor, the imaginary run
-    takes the imaginary planes as a series of degree K-1 (orders shifted down by
-    one: an ordinary operand does not mix orders), so it forms K products, not
-    K+1. Two series operands use the four real runs of the complex product. An
+    An ordinary operand does not mix orders: with one complex-direction series and
+    one ordinary tensor, the 2K + 1 real planes (order 0, the real parts, the
+    imaginary parts) are the orders of one real product (matrix products, to the
+    kernel's degree), or else the imaginary run takes the imaginary planes as a
+    series of degree K-1, so it forms K products, not K+1. Two series operands use the four real runs of the complex product. An
     operand with a complex constant term takes the general split
     (``complex_product``).
     """
@@ -335,6 +346,10 @@ def bilinear(fn, what, a, b, *rest, **kwargs):
     if ac != bc and not isinstance(b if ac else a, PolyTensor):
         x = a if ac else b
         real, imag = _ops.complex_to_real(_planes(x), [1.0, 0.0], [0.0, 1.0]).unbind(0)
+        if what in ("matmul", "linear") and one_product(a, b):
+            planes = PolyTensor((x.coeffs[0],) + tuple(real.unbind(0)) + tuple(imag.unbind(0)))
+            y = (fn(planes, b, *rest, **kwargs) if ac else fn(a, planes, *rest, **kwargs)).coeffs
+            return _combine_parts(PolyTensor(y[:x.degree + 1]), list(y[x.degree + 1:]))
         xr = PolyTensor((x.coeffs[0],) + tuple(real.unbind(0)))
         xi = PolyTensor(tuple(imag.unbind(0)))
         yr = fn(xr, b, *rest, **kwargs) if ac else fn(a, xr, *rest, **kwargs)

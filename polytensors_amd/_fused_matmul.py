@@ -40,9 +40,10 @@ def why_ineligible(a, b, below_autograd=False):
     return None
 
 
-def _cauchy(A, B, degree, trans_b):
+def _cauchy(A, B, degree, trans_b, bias=None):
     """The Cauchy-product kernel's stacked [K+1, batch, m, n] result for operand coefficient lists
-    A (1 or K+1 orders) and B; above the kernel's degree, in blocks of its orders.
+    A (1 or K+1 orders) and B (``bias`` added to the constant order's rows, to the kernel's degree);
+    above it, in blocks of its orders.
 
     With blocks of m = MAX_DEGREE + 1 orders, X = sum_p t^(m p) X^(p) and
     A (*) B = sum_{p,q} t^(m (p+q)) A^(p) (*) B^(q), each block product being the full product of two
@@ -52,6 +53,8 @@ def _cauchy(A, B, degree, trans_b):
     """
     cap = _gate.MAX_DEGREE
     if degree <= cap:
+        if bias is not None:
+            return _ops.cauchy_matmul(A, B, degree, trans_b, bias)
         return _ops.cauchy_matmul(A, B, degree, trans_b)
     m = cap + 1
 
@@ -104,13 +107,15 @@ def _degree(*xs):
     return next(x.degree for x in xs if isinstance(x, PolyTensor))
 
 
-def matmul(a, b, below_autograd=False):
-    """Series of ``torch.matmul(a, b)``."""
+def matmul(a, b, below_autograd=False, bias=None):
+    """Series of ``torch.matmul(a, b)`` (plus ``bias``, one that ``_kernel_bias`` admits)."""
     reason = why_ineligible(a, b, below_autograd)
     if reason is not None:
         raise NotImplementedError(f"matmul: {reason}")
     if _complex.has_complex(a, b) or _complex.has_complex_base(a, b):
-        return _complex.bilinear(matmul, "matmul", a, b, below_autograd=below_autograd)
+        inside = bias is not None and _complex.one_product(a, b)
+        result = _complex.bilinear(matmul, "matmul", a, b, below_autograd=below_autograd, bias=bias if inside else None)
+        return result if bias is None or inside else result + bias
     degree = _degree(a, b)
     A = list(_gate.coefficients(a, degree))
     B = list(_gate.coefficients(b, degree))
@@ -140,9 +145,9 @@ def matmul(a, b, below_autograd=False):
 
     if all(c.ndim == 2 and not c.is_contiguous() and c.t().is_contiguous() for c in B):
         # a transposed [n, k] matrix (a linear layer's weight): the kernel reads it in place
-        out = _cauchy(flat(A, m, kd), [c.t().reshape(1, n, kd) for c in B], degree, True)
+        out = _cauchy(flat(A, m, kd), [c.t().reshape(1, n, kd) for c in B], degree, True, bias)
     else:
-        out = _cauchy(flat(A, m, kd), flat(B, kd, n), degree, False)
+        out = _cauchy(flat(A, m, kd), flat(B, kd, n), degree, False, bias)
     out = out.view(degree + 1, *batch, m, n)
     if squeeze_m:
         out = out.squeeze(-2)
@@ -151,14 +156,28 @@ def matmul(a, b, below_autograd=False):
     return PolyTensor.from_stacked(out)
 
 
+def _kernel_bias(bias, a, b, columns):
+    """Whether the kernel of the product of a and b adds this bias: an ordinary vector of its
+    ``columns``, of the operands' dtype and device, that no graph is recorded for, to the kernel's
+    degree."""
+    if not isinstance(bias, torch.Tensor) or isinstance(bias, PolyTensor) or (torch.is_grad_enabled() and
+                                                                              bias.requires_grad):
+        return False
+    return (bias.dtype == b.dtype and bias.device == b.device and tuple(bias.shape) == (columns,) and
+            bias.is_contiguous() and _degree(a, b) <= _gate.MAX_DEGREE)
+
+
 def linear(x, weight, bias=None):
     """Series of ``torch.nn.functional.linear``: x @ weight^T (+ bias)."""
     reason = why_ineligible(x, weight)
     if reason is not None:
         raise NotImplementedError(f"linear: {reason}")
+    inside = weight.ndim == 2 and _kernel_bias(bias, x, weight, weight.shape[0])
     if _complex.has_complex(x, weight) or _complex.has_complex_base(x, weight):
-        result = _complex.bilinear(linear, "linear", x, weight)
-        return result if bias is None else result + bias
+        # (with an ordinary weight one product, which takes the bias; in general a sum of products)
+        inside = inside and _complex.one_product(x, weight)
+        result = _complex.bilinear(linear, "linear", x, weight, *((bias,) if inside else ()))
+        return result if bias is None or inside else result + bias
     degree = _degree(x, weight, *([bias] if isinstance(bias, PolyTensor) else []))
     X = list(_gate.coefficients(x, degree))
     W = list(_gate.coefficients(weight, degree))
@@ -168,9 +187,9 @@ def linear(x, weight, bias=None):
     lead = X[0].shape[:-1]
     X = [c.reshape(1, -1, in_features).contiguous() for c in X]
     W = [c.reshape(1, out_features, in_features).contiguous() for c in W]
-    out = _cauchy(X, W, degree, True)
+    out = _cauchy(X, W, degree, True, bias if inside else None)
     result = PolyTensor.from_stacked(out.view(degree + 1, *lead, out_features))
-    if bias is not None:
+    if bias is not None and not inside:
         result = result + bias
     return result
 
@@ -182,6 +201,8 @@ def from_dispatch(func, args, kwargs):
     if func is aten.addmm.default:
         bias, a, b = args[:3]
         beta, alpha = kwargs.get("beta", 1), kwargs.get("alpha", 1)
+        if alpha == 1 and beta == 1 and a.ndim == b.ndim == 2 and _kernel_bias(bias, a, b, b.shape[1]):
+            return matmul(a, b, below_autograd=True, bias=bias)
         product = matmul(a, b, below_autograd=True)
         if alpha != 1:
             product = product * alpha

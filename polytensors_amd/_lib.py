@@ -56,7 +56,7 @@ SIGNATURES = {
     "pt_cauchy_matmul": (_c_int, [_c_int, _c_int, _c_vpp, _c_int, _c_vpp, _c_int, _c_vpp,
                                   _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_vp]),
     "pt_cauchy_matmul_strided": (_c_int, [_c_int, _c_int, _c_vpp, _c_int, _c_vpp, _c_int, _c_vpp, _c_i64, _c_i64, _c_i64,
-                                          _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_vp]),
+                                          _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_vp, _c_vp]),
     "pt_pack_rows": (_c_int, [_c_int, _c_int, _c_vpp, _c_vpp, _c_i64, _c_i64, _c_i64, _c_vp]),
     "pt_matmul_order_sum": (_c_int, [_c_int, _c_int, _c_vpp, _c_vpp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
                                      _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_vp]),

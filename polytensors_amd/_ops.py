@@ -29,7 +29,7 @@ SCHEMAS = {
                              "-> (Tensor, Tensor)"),
     "cross_entropy_series_backward": ("(Tensor[] z, Tensor target, int ignore_index, float softcap, Tensor lse, "
                                       "Tensor[] cot) -> Tensor"),
-    "cauchy_matmul": "(Tensor[] a, Tensor[] b, int degree, bool trans_b) -> Tensor",
+    "cauchy_matmul": "(Tensor[] a, Tensor[] b, int degree, bool trans_b, Tensor? bias=None) -> Tensor",
     "matmul_order_sum": "(Tensor[] a, Tensor[] b, bool trans_a, bool trans_b) -> Tensor",
     "taylor_attention_fwd": ("(Tensor[] q, Tensor[] k, Tensor[] v, Tensor? mask, bool causal, float scale, "
                              "int degree, int[]? mask_map=None) -> (Tensor, Tensor)"),
@@ -123,7 +123,7 @@ cauchy_matmul = _op("cauchy_matmul")
 
 
 @torch.library.register_fake(f"{NAMESPACE}::cauchy_matmul")
-def _(a, b, degree, trans_b):
+def _(a, b, degree, trans_b, bias=None):
     ba, m, _ = a[0].shape
     bb = b[0].shape[0]
     n = b[0].shape[1] if trans_b else b[0].shape[2]
@@ -412,7 +412,7 @@ torch.library.register_autograd(f"{NAMESPACE}::cross_entropy_series", _ce_backwa
 
 
 def _mm_setup(ctx, inputs, output):
-    a, b, degree, trans_b = inputs
+    a, b, degree, trans_b = inputs[:4]   # (a bias is an ordinary tensor without grad: _fused_matmul.linear)
     ctx.save_for_backward(*a, *b)
     ctx.meta = (len(a), len(b), degree, trans_b, _grads_flag(a), _grads_flag(b))
     ctx.n_inputs = len(inputs)

@@ -16,6 +16,7 @@ struct CauchyArgs {
   int64_t lda, ldb;   // row strides; zeros from k to the next 16-byte vector where rows run along k
   int64_t a_bs, b_bs;
   bool trans_b;
+  const void* bias;   // null, or n values added to every row of order 0
   hipStream_t stream;
   int64_t rows_b() const { return trans_b ? n : k; }
   int64_t width_b() const { return trans_b ? k : n; }

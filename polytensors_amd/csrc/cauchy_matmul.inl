@@ -73,7 +73,8 @@ template <typename T, int K, int AO, int BO, int BM, int BN, int BK, int WAVES_M
           int MIN_WAVES, bool TRANS_B, bool VEC>
 __global__ __launch_bounds__(WAVES_M * WAVES_N * kWave) __attribute__((amdgpu_waves_per_eu(MIN_WAVES)))
 void cauchy_matmul_kernel(
-    CPtrs<T> A, CPtrs<T> B, MPtrs<T> C, int M, int N, int Kd, int lda, int ldb, int64_t a_bs, int64_t b_bs) {
+    CPtrs<T> A, CPtrs<T> B, MPtrs<T> C, int M, int N, int Kd, int lda, int ldb, int64_t a_bs, int64_t b_bs,
+    const T* __restrict__ bias) {
   using MF = Mfma<T>;
   using acc_t = typename MF::acc_t;
   constexpr int THREADS = WAVES_M * WAVES_N * kWave;
@@ -256,10 +257,11 @@ void cauchy_matmul_kernel(
 #pragma unroll
       for (int fn = 0; fn < FN; ++fn) {
         const int col = tile_n + wn * WN + fn * MF::N + MF::acc_col(lane);
+        const T add = o == 0 && bias != nullptr && col < N ? bias[col] : T(0);
 #pragma unroll
         for (int r = 0; r < MF::ACC; ++r) {
           const int row = tile_m + wm * WM + fm * MF::M + MF::acc_row(lane, r);
-          if (row < M && col < N) c_base[static_cast<int64_t>(row) * N + col] = acc[o][fm][fn][r];
+          if (row < M && col < N) c_base[static_cast<int64_t>(row) * N + col] = o == 0 ? acc[o][fm][fn][r] + add : acc[o][fm][fn][r];
         }
       }
   }
@@ -306,7 +308,8 @@ static int launch_cauchy_orders(const CauchyArgs& a, const CPtrs<T>& A, const CP
   const int lda = static_cast<int>(a.lda), ldb = static_cast<int>(a.ldb);
 #define PT_CAUCHY_LAUNCH(TB, VV)                                                                   \
   cauchy_matmul_kernel<T, K, AO, BO, Tile::BM, Tile::BN, Tile::BK, Tile::WAVES_M, Tile::WAVES_N, \
-                       Tile::MIN_WAVES, TB, VV><<<grid, block, 0, a.stream>>>(A, B, C, M, N, Kd, lda, ldb, a.a_bs, a.b_bs)
+                       Tile::MIN_WAVES, TB, VV><<<grid, block, 0, a.stream>>>(A, B, C, M, N, Kd, lda, ldb, a.a_bs, a.b_bs, \
+                                                static_cast<const T*>(a.bias))
   if (a.trans_b) {
     if (vec) PT_CAUCHY_LAUNCH(true, true);
     else PT_CAUCHY_LAUNCH(true, false);

@@ -71,12 +71,13 @@ int pt_cauchy_matmul(int dtype, int degree, const void* const* a, int a_orders,
                      int64_t n, int64_t k, int64_t a_batch_stride, int64_t b_batch_stride,
                      int trans_b, void* stream) {
   return pt_cauchy_matmul_strided(dtype, degree, a, a_orders, b, b_orders, c, batch, m, n, k, k, trans_b ? k : n,
-                                  a_batch_stride, b_batch_stride, trans_b, stream);
+                                  a_batch_stride, b_batch_stride, trans_b, nullptr, stream);
 }
 
 int pt_cauchy_matmul_strided(int dtype, int degree, const void* const* a, int a_orders, const void* const* b,
                              int b_orders, void* const* c, int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda,
-                             int64_t ldb, int64_t a_batch_stride, int64_t b_batch_stride, int trans_b, void* stream) {
+                             int64_t ldb, int64_t a_batch_stride, int64_t b_batch_stride, int trans_b, const void* bias,
+                             void* stream) {
   pt_host::clear_error();
   PT_REQUIRE(degree >= 0 && degree <= PT_MAX_DEGREE, PT_UNSUPPORTED,
              "Cauchy matmul: degree must be in 0..8");
@@ -105,7 +106,7 @@ int pt_cauchy_matmul_strided(int dtype, int degree, const void* const* a, int a_
     PT_REQUIRE(c[o] != nullptr, PT_INVALID_ARGUMENT, "Cauchy matmul: null C coefficient");
   if (batch == 0 || m == 0 || n == 0) return PT_OK;
   pt::CauchyArgs args{degree, a, a_orders, b, b_orders, c, batch, m, n, k, lda, ldb,
-                      a_batch_stride, b_batch_stride, trans_b != 0, static_cast<hipStream_t>(stream)};
+                      a_batch_stride, b_batch_stride, trans_b != 0, bias, static_cast<hipStream_t>(stream)};
   switch (dtype) {
     case PT_FLOAT32: return pt::launch_cauchy<float>(args);
     case PT_FLOAT64: return pt::launch_cauchy<double>(args);

@@ -71,7 +71,8 @@ __host__ __device__ __forceinline__ int cauchy_swz_k(int k, int ch) {
 
 template <typename T, int K, int AO, int BO, bool TRANS_B, bool WIDE>
 __global__ __launch_bounds__((CauchyHalfTile<AO, BO, WIDE>::kThreads)) void cauchy_matmul_half_kernel(
-    CPtrs<T> A, CPtrs<T> B, MPtrs<T> C, int M, int N, int Kd, int lda, int ldb, int64_t a_bs, int64_t b_bs) {
+    CPtrs<T> A, CPtrs<T> B, MPtrs<T> C, int M, int N, int Kd, int lda, int ldb, int64_t a_bs, int64_t b_bs,
+    const T* __restrict__ bias) {
   using Tile = CauchyHalfTile<AO, BO, WIDE>;
   using MM = HalfMfma<T>;
   constexpr int BM = Tile::BM, BN = Tile::BN, BK = Tile::BK, FM = Tile::FM, FN = Tile::FN;
@@ -212,7 +213,11 @@ __global__ __launch_bounds__((CauchyHalfTile<AO, BO, WIDE>::kThreads)) void cauc
         const int row = tile_m + FM * 16 * wm + 16 * fm + c;
         const int col = tile_n + FN * 16 * wn + 16 * fn + 4 * g;
         if (row >= M) continue;
-        const floatx4 v = acc[o][fm][fn];
+        floatx4 v = acc[o][fm][fn];
+        if (o == 0 && bias != nullptr) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] += col + e < N ? to_acc(bias[col + e]) : 0.f;
+        }
         T* p = base + static_cast<int64_t>(row) * N + col;
         const uint32_t w01 = MM::pack2(v[0], v[1]), w23 = MM::pack2(v[2], v[3]);
         if (col + 3 < N) {   // at any element: one 8-byte store
@@ -247,10 +252,12 @@ static int launch_cauchy_half_tile(const CauchyArgs& a, const CPtrs<T>& A, const
   const int lda = static_cast<int>(a.lda), ldb = static_cast<int>(a.ldb);
   if (a.trans_b)
     cauchy_matmul_half_kernel<T, K, AO, BO, true, WIDE>
-        <<<grid, block, 0, a.stream>>>(A, B, C, M, N, Kd, lda, ldb, a.a_bs, a.b_bs);
+        <<<grid, block, 0, a.stream>>>(A, B, C, M, N, Kd, lda, ldb, a.a_bs, a.b_bs,
+                                         static_cast<const T*>(a.bias));
   else
     cauchy_matmul_half_kernel<T, K, AO, BO, false, WIDE>
-        <<<grid, block, 0, a.stream>>>(A, B, C, M, N, Kd, lda, ldb, a.a_bs, a.b_bs);
+        <<<grid, block, 0, a.stream>>>(A, B, C, M, N, Kd, lda, ldb, a.a_bs, a.b_bs,
+                                         static_cast<const T*>(a.bias));
   PT_LAUNCH_CHECK();
   return PT_OK;
 }

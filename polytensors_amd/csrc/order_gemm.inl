@@ -105,6 +105,7 @@ template <typename T>
 struct OrderGemmParams {
   CPtrs<T> a, b;
   MPtrs<T> c;
+  const T* bias;                // null, or n values added to every row of order 0
   int m, n, k;                  // of one order; zeros from k to the next 16-byte vector where it runs along rows
   int lda, ldb;                 // row strides in elements
   int a_bytes, b_bytes;         // extent of one matrix
@@ -303,6 +304,7 @@ void order_gemm_kernel(OrderGemmParams<T> p) {
 
   // ---- epilogue: a lane's registers are runs of four columns of one row of C ----
   T* base = p.c.p[order] + batch * p.c_bs;
+  const bool add = p.bias != nullptr && order == 0;
 #pragma unroll
   for (int fm = 0; fm < FM; ++fm) {
     const int row = tile_m + (wm * FM + fm) * Blk::S + lane % Blk::S;
@@ -315,6 +317,10 @@ void order_gemm_kernel(OrderGemmParams<T> p) {
         float v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = acc[fm][fn][4 * q + e];
+        if (add) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] += col + e < p.n ? to_acc(p.bias[col + e]) : 0.f;
+        }
         T* dst = base + static_cast<int64_t>(row) * p.n + col;
         if (col + 3 < p.n) {
           Vec<T, 4> w;
@@ -390,6 +396,7 @@ static int launch_by_order(const CauchyArgs& a, int orders) {
   for (int o = 0; o < a.a_orders; ++o) p.a.p[o] = static_cast<const T*>(a.a[o]);
   for (int o = 0; o < a.b_orders; ++o) p.b.p[o] = static_cast<const T*>(a.b[o]);
   for (int o = 0; o < orders; ++o) p.c.p[o] = static_cast<T*>(a.c[o]);
+  p.bias = static_cast<const T*>(a.bias);
   p.m = static_cast<int>(a.m);
   p.n = static_cast<int>(a.n);
   p.k = static_cast<int>(a.k);

@@ -266,7 +266,8 @@ Rows packed_rows(const TensorList& in) {
   return {std::move(out), stride};
 }
 
-Tensor cauchy_matmul(const TensorList& a_in, const TensorList& b_in, int64_t degree, bool trans_b) {
+Tensor cauchy_matmul(const TensorList& a_in, const TensorList& b_in, int64_t degree, bool trans_b,
+                     const c10::optional<Tensor>& bias) {
   check_abi();
   for (const auto& [name, s] : {std::pair<const char*, const TensorList*>{"a", &a_in}, {"b", &b_in}}) {
     const int64_t len = static_cast<int64_t>(s->size());
@@ -284,6 +285,9 @@ Tensor cauchy_matmul(const TensorList& a_in, const TensorList& b_in, int64_t deg
   const int64_t kb = trans_b ? b_in[0].size(2) : b_in[0].size(1);
   TORCH_CHECK_VALUE(kb == kd, "cauchy_matmul: inner dimensions differ");
   TORCH_CHECK_VALUE(ba == bb || ba == 1 || bb == 1, "cauchy_matmul: batch dimensions do not broadcast");
+  TORCH_CHECK_VALUE(!bias || (bias->scalar_type() == dtype && bias->device() == a_in[0].device() && bias->dim() == 1 &&
+                              bias->size(0) == n && bias->is_contiguous()),
+                    "cauchy_matmul: bias must be a contiguous [n] vector of the operands' dtype and device");
   const int64_t batch = std::max(ba, bb);
   c10::DeviceGuard guard(a_in[0].device());
   const Rows a = packed_rows(a_in), b = packed_rows(b_in);
@@ -293,7 +297,8 @@ Tensor cauchy_matmul(const TensorList& a_in, const TensorList& b_in, int64_t deg
   const int status = pt_cauchy_matmul_strided(
       dtype_code(dtype), static_cast<int>(degree), as.data(), static_cast<int>(a_in.size()), bs.data(),
       static_cast<int>(b_in.size()), cs.data(), batch, m, n, kd, a.stride, b.stride, ba == 1 ? 0 : m * a.stride,
-      bb == 1 ? 0 : b_in[0].size(1) * b.stride, trans_b ? 1 : 0, stream_of(a_in[0]));
+      bb == 1 ? 0 : b_in[0].size(1) * b.stride, trans_b ? 1 : 0, bias ? bias->data_ptr() : nullptr,
+      stream_of(a_in[0]));
   check_status(status, "cauchy_matmul");
   return out;
 }
@@ -655,7 +660,7 @@ TORCH_LIBRARY(polytensors_amd, m) {
         "-> (Tensor, Tensor)");
   m.def("cross_entropy_series_backward(Tensor[] z, Tensor target, int ignore_index, float softcap, Tensor lse, "
         "Tensor[] cot) -> Tensor");
-  m.def("cauchy_matmul(Tensor[] a, Tensor[] b, int degree, bool trans_b) -> Tensor");
+  m.def("cauchy_matmul(Tensor[] a, Tensor[] b, int degree, bool trans_b, Tensor? bias=None) -> Tensor");
   m.def("matmul_order_sum(Tensor[] a, Tensor[] b, bool trans_a, bool trans_b) -> Tensor");
   m.def("taylor_attention_fwd(Tensor[] q, Tensor[] k, Tensor[] v, Tensor? mask, bool causal, float scale, "
         "int degree, int[]? mask_map=None) -> (Tensor, Tensor)");

@@ -206,3 +206,39 @@ def test_rows_that_no_vector_divides(dtype, tol, m, k, n, batch_a, batch_b, offs
     for o in range(degree + 1):
         err = (out.coeffs[o].cpu().double() - want[o]).abs().max() / want[o].abs().max()
         assert err <= tol, (o, err)
+
+
+# A linear layer's bias added by the kernel (an ordinary vector without a graph) on each kernel: order by
+# order, series weights, float64; columns the 16-byte stores do not divide; real and complex directions;
+# through addmm under wrapper autograd. A bias the kernel does not take (a series, another dtype) is added after.
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.float64, 1e-13), (torch.bfloat16, 2.0 ** -8)])
+@pytest.mark.parametrize("m,k,n", [(1, 8, 3), (130, 72, 65), (64, 40, 264)])
+@pytest.mark.parametrize("weight", ["plain", "series", "complex"])
+def test_linear_bias(dtype, tol, m, k, n, weight):
+    if weight == "complex" and dtype == torch.bfloat16:
+        pytest.skip("no complex bfloat16")
+    g, degree = torch.Generator().manual_seed(m + n), 3
+    draw = lambda *shape: torch.randn(*shape, generator=g, dtype=torch.float64).to(dtype)   # noqa: E731
+    X, W = [draw(2, m, k) for _ in range(degree + 1)], [draw(n, k) for _ in range(degree + 1)]
+    if weight == "complex":
+        X = X[:1] + [torch.complex(c, draw(2, m, k)) for c in X[1:]]
+    b = draw(n)
+    x = PolyTensor(tuple(c.cuda() for c in X))
+    w = PolyTensor(tuple(c.cuda() for c in W)) if weight == "series" else W[0].cuda()
+    up = lambda cs: [c.to(torch.complex128 if c.is_complex() else torch.float64) for c in cs]   # noqa: E731
+    if weight == "series":
+        want = oracle.matmul(up(X), [c.t() for c in up(W)])
+    else:
+        want = [c @ up(W)[0].t().to(c.dtype) for c in up(X)]
+    want[0] = want[0] + b.double()
+    with PolyTensor.plain_range():
+        with torch.no_grad():
+            outs = [F.linear(x, w, b.cuda()), F.linear(x, w, PolyTensor.constant(b.cuda(), degree))]
+            if weight != "complex":
+                outs.append(F.linear(x, w, b.cuda().double()))   # another dtype: promoted, as torch's add
+        xg = PolyTensor(tuple(c.cuda() for c in X), requires_grad=True)
+        outs.append(F.linear(xg, w, b.cuda()))
+    for out in outs:
+        for o in range(degree + 1):
+            err = (out.coeffs[o].detach().cpu().to(want[o].dtype) - want[o]).abs().max() / want[o].abs().max()
+            assert err <= 2 * tol, (o, err)   # (twice: the separate addition rounds again)
