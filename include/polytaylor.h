@@ -120,6 +120,13 @@ int pt_rms_norm_series_bwd(int dtype, int degree, const void* const* x,
 int pt_layer_norm_series_bwd(int dtype, int degree, const void* const* x,
                              const void* const* g, void* const* dx,
                              int64_t rows, int64_t n, double eps, void* stream);
+/*
+ * The same (LayerNorm if layer, else RMSNorm) for the normalization followed by an ordinary weight:
+ * dx(t) = J(x(t))^T (w g(t)). weight: [n] of `dtype`, or null for none.
+ */
+int pt_norm_series_bwd_weighted(int dtype, int degree, int layer, const void* const* x, const void* const* g,
+                                const void* weight, void* const* dx, int64_t rows, int64_t n, double eps,
+                                void* stream);
 
 /*
  * Cross entropy of a degree-K series of logits z(t) with integer targets.

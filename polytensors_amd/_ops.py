@@ -24,7 +24,7 @@ NAMESPACE = "polytensors_amd"
 # implementation that raises LibraryMissingError, so that every call fails loudly.
 SCHEMAS = {
     "norm_series": "(Tensor[] x, Tensor[] weight, Tensor[] bias, int n, float eps, bool layer) -> Tensor",
-    "norm_series_backward": "(Tensor[] x, Tensor[] grad, int n, float eps, bool layer) -> Tensor",
+    "norm_series_backward": "(Tensor[] x, Tensor[] grad, int n, float eps, bool layer, Tensor? weight=None) -> Tensor",
     "cross_entropy_series": ("(Tensor[] z, Tensor target, int ignore_index, int reduction, float softcap) "
                              "-> (Tensor, Tensor)"),
     "cross_entropy_series_backward": ("(Tensor[] z, Tensor target, int ignore_index, float softcap, Tensor lse, "
@@ -243,7 +243,7 @@ norm_series_backward = _op("norm_series_backward")
 
 
 @torch.library.register_fake(f"{NAMESPACE}::norm_series_backward")
-def _(x, grad, n, eps, layer):
+def _(x, grad, n, eps, layer, weight=None):
     return x[0].new_empty((len(x), *x[0].shape))
 
 

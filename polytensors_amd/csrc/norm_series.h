@@ -22,11 +22,12 @@ struct NormArgs {
 template <typename T, bool LAYER>
 int launch_norm(const NormArgs& a);
 
-// Gradient series of the normalization (no affine terms): dx = J(x(t))^T g(t).
+// Gradient series of the normalization: dx = J(x(t))^T (w g(t)), w an ordinary weight or null.
 struct NormBwdArgs {
   int degree;
   const void* const* x;
   const void* const* g;
+  const void* w;
   void* const* dx;
   int64_t rows;
   int64_t n;

@@ -111,24 +111,24 @@ int pt_layer_norm_series_fwd(int dtype, int degree, const void* const* x,
   return dispatch_norm(dtype, true, a);
 }
 
-int pt_rms_norm_series_bwd(int dtype, int degree, const void* const* x, const void* const* g,
-                           void* const* dx, int64_t rows, int64_t n, double eps, void* stream) {
+int pt_norm_series_bwd_weighted(int dtype, int degree, int layer, const void* const* x, const void* const* g,
+                                const void* weight, void* const* dx, int64_t rows, int64_t n, double eps, void* stream) {
   pt_host::clear_error();
   int st = check_norm_bwd(dtype, degree, x, g, dx, rows, n, eps);
   if (st != PT_OK) return st;
   if (rows == 0) return PT_OK;
-  pt::NormBwdArgs a{degree, x, g, dx, rows, n, eps, static_cast<hipStream_t>(stream)};
-  return dispatch_norm_bwd(dtype, false, a);
+  pt::NormBwdArgs a{degree, x, g, weight, dx, rows, n, eps, static_cast<hipStream_t>(stream)};
+  return dispatch_norm_bwd(dtype, layer != 0, a);
+}
+
+int pt_rms_norm_series_bwd(int dtype, int degree, const void* const* x, const void* const* g,
+                           void* const* dx, int64_t rows, int64_t n, double eps, void* stream) {
+  return pt_norm_series_bwd_weighted(dtype, degree, 0, x, g, nullptr, dx, rows, n, eps, stream);
 }
 
 int pt_layer_norm_series_bwd(int dtype, int degree, const void* const* x, const void* const* g,
                              void* const* dx, int64_t rows, int64_t n, double eps, void* stream) {
-  pt_host::clear_error();
-  int st = check_norm_bwd(dtype, degree, x, g, dx, rows, n, eps);
-  if (st != PT_OK) return st;
-  if (rows == 0) return PT_OK;
-  pt::NormBwdArgs a{degree, x, g, dx, rows, n, eps, static_cast<hipStream_t>(stream)};
-  return dispatch_norm_bwd(dtype, true, a);
+  return pt_norm_series_bwd_weighted(dtype, degree, 1, x, g, nullptr, dx, rows, n, eps, stream);
 }
 
 }  // extern "C"

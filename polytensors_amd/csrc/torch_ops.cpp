@@ -130,7 +130,8 @@ Tensor norm_series(const TensorList& x, const TensorList& weight, const TensorLi
   return out;
 }
 
-Tensor norm_series_backward(const TensorList& x, const TensorList& grad, int64_t n, double eps, bool layer) {
+Tensor norm_series_backward(const TensorList& x, const TensorList& grad, int64_t n, double eps, bool layer,
+                            const c10::optional<Tensor>& weight) {
   check_abi();
   check_series("norm_series_backward x", x);
   check_series("norm_series_backward grad", grad);
@@ -140,13 +141,17 @@ Tensor norm_series_backward(const TensorList& x, const TensorList& grad, int64_t
   const int64_t degree = static_cast<int64_t>(x.size()) - 1;
   const int64_t numel = x[0].numel();
   TORCH_CHECK_VALUE(n >= 1 && numel % n == 0, "norm_series_backward: n must divide the element count");
+  TORCH_CHECK_VALUE(!weight || (weight->scalar_type() == x[0].scalar_type() && weight->device() == x[0].device() &&
+                                weight->numel() == n && weight->is_contiguous()),
+                    "norm_series_backward: weight must be contiguous [n] of the input dtype");
   c10::DeviceGuard guard(x[0].device());
   Tensor out = at::empty(stacked_shape(degree + 1, x[0].sizes()), x[0].options());
   auto xs = cptrs(x), gs = cptrs(grad);
   auto ys = slices(out);
   const int code = dtype_code(x[0].scalar_type());
-  const int status = (layer ? pt_layer_norm_series_bwd : pt_rms_norm_series_bwd)(
-      code, static_cast<int>(degree), xs.data(), gs.data(), ys.data(), numel / n, n, eps, stream_of(x[0]));
+  const int status =
+      pt_norm_series_bwd_weighted(code, static_cast<int>(degree), layer ? 1 : 0, xs.data(), gs.data(),
+                                  weight ? weight->data_ptr() : nullptr, ys.data(), numel / n, n, eps, stream_of(x[0]));
   check_status(status, layer ? "layer_norm_series_bwd" : "rms_norm_series_bwd");
   return out;
 }
@@ -655,7 +660,7 @@ Tensor series_binary(const TensorList& a, const TensorList& b, c10::string_view 
 
 TORCH_LIBRARY(polytensors_amd, m) {
   m.def("norm_series(Tensor[] x, Tensor[] weight, Tensor[] bias, int n, float eps, bool layer) -> Tensor");
-  m.def("norm_series_backward(Tensor[] x, Tensor[] grad, int n, float eps, bool layer) -> Tensor");
+  m.def("norm_series_backward(Tensor[] x, Tensor[] grad, int n, float eps, bool layer, Tensor? weight=None) -> Tensor");
   m.def("cross_entropy_series(Tensor[] z, Tensor target, int ignore_index, int reduction, float softcap) "
         "-> (Tensor, Tensor)");
   m.def("cross_entropy_series_backward(Tensor[] z, Tensor target, int ignore_index, float softcap, Tensor lse, "

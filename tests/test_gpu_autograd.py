@@ -149,6 +149,30 @@ def test_norm_gradient_series(layer, degree, dtype, n):
     _check(dx.coeffs, want_dx, dtype)
 
 
+# An ordinary weight (and bias) without a gradient is applied by the norm's kernels, forward and
+# backward: rows of the register path with lanes past the row, of several chunks, and of the
+# streaming path. One that needs a gradient is a separate operation, as is one of another shape.
+@pytest.mark.parametrize("layer", [False, True])
+@pytest.mark.parametrize("n", [8, 40, 999, 1024, 5000])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32, torch.bfloat16])
+def test_norm_gradient_series_with_an_ordinary_weight(layer, n, dtype):
+    degree = 3
+    X, G, (W, Bias) = ([c.to(dtype) for c in _series(*a)] for a in (((5, n), degree, 31), ((5, n), degree, 32), ((n,), 1, 33)))
+    x = PolyTensor(tuple(c.to(dtype).cuda() for c in X), requires_grad=True)
+    w, b = W.to(dtype).cuda(), Bias.to(dtype).cuda()
+    with PolyTensor.plain_range():
+        y = F.layer_norm(x, (n,), w, b, 1e-5) if layer else F.rms_norm(x, (n,), w, 1e-5)
+        y.backward(PolyTensor(tuple(c.to(dtype).cuda() for c in G)))
+    Wd, Bd = W.double(), Bias.double()
+    Xd, Gw = [c.double() for c in X], [c.double() * Wd for c in G]
+    if layer:
+        want, dx = oracle.layer_norm(Xd, (n,), [Wd], [Bd], eps=1e-5), oracle.layer_norm_backward(Xd, Gw, (n,), eps=1e-5)
+    else:
+        want, dx = oracle.rms_norm(Xd, (n,), [Wd], eps=1e-5), oracle.rms_norm_backward(Xd, Gw, (n,), eps=1e-5)
+    _check([c.detach() for c in y.coeffs], want, dtype)
+    _check(x.grad.coeffs, dx, dtype)
+
+
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 def test_norm_with_series_weight_gradients(dtype):
     # The weight multiplies as a separate series product (as the reference's
