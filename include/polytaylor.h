@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define PT_ABI_VERSION 13
+#define PT_ABI_VERSION 14
 #define PT_MAX_DEGREE 8
 /* Largest degree of the elementwise kernels (pt_activation_series_*, pt_series_binary): their
  * register plans are per element, so they run above PT_MAX_DEGREE. */

@@ -147,8 +147,9 @@ def activation(x, kind):
         return _complex_base(x, kind)
     if _complex.has_complex(x):
         return _complex.at_real_nodes_below_autograd(activation, kind, x, kind)
-    out = _ops.activation_series(_coeffs(x, x.degree), kind)
-    return PolyTensor.from_stacked(out)
+    if _gate.coefficient_graph(x):
+        return PolyTensor._wrap(tuple(_ops.activation_series_orders(_coeffs(x, x.degree), kind)))
+    return PolyTensor.from_stacked(_ops.activation_series(_coeffs(x, x.degree), kind))
 
 
 def backward(grad, saved, kind):

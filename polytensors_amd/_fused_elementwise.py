@@ -51,4 +51,6 @@ def binary(a, b, op):
         coeffs = [c.expand(shape).contiguous() for c in coeffs]
         return coeffs + [torch.zeros_like(coeffs[0]) for _ in range(degree + 1 - len(coeffs))]
 
+    if _gate.coefficient_graph(a, b):
+        return PolyTensor._wrap(tuple(_ops.series_binary_orders(series(a), series(b), op)))
     return PolyTensor.from_stacked(_ops.series_binary(series(a), series(b), op))

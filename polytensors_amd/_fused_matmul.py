@@ -99,6 +99,14 @@ def _cauchy(A, B, degree, trans_b, bias=None):
     return torch.stack(out)
 
 
+def _product(a, b, A, B, degree, trans_b, bias, shape):
+    """The PolyTensor of a @ b, given by their flattened coefficients A and B, in ``shape``; a tensor
+    per order where autograd records the coefficients."""
+    if degree <= _gate.MAX_DEGREE and _gate.coefficient_graph(a, b):
+        return PolyTensor._wrap(tuple(c.view(shape) for c in _ops.cauchy_matmul_orders(A, B, degree, trans_b, bias)))
+    return PolyTensor.from_stacked(_cauchy(A, B, degree, trans_b, bias).view(degree + 1, *shape))
+
+
 def eligible(a, b):
     return why_ineligible(a, b) is None
 
@@ -143,17 +151,11 @@ def matmul(a, b, below_autograd=False, bias=None):
                     for c in coeffs]
         return [c.expand(*batch, rows, cols).reshape(-1, rows, cols).contiguous() for c in coeffs]
 
+    shape = (*batch, *(() if squeeze_m else (m,)), *(() if squeeze_n else (n,)))
     if all(c.ndim == 2 and not c.is_contiguous() and c.t().is_contiguous() for c in B):
         # a transposed [n, k] matrix (a linear layer's weight): the kernel reads it in place
-        out = _cauchy(flat(A, m, kd), [c.t().reshape(1, n, kd) for c in B], degree, True, bias)
-    else:
-        out = _cauchy(flat(A, m, kd), flat(B, kd, n), degree, False, bias)
-    out = out.view(degree + 1, *batch, m, n)
-    if squeeze_m:
-        out = out.squeeze(-2)
-    if squeeze_n:
-        out = out.squeeze(-1)
-    return PolyTensor.from_stacked(out)
+        return _product(a, b, flat(A, m, kd), [c.t().reshape(1, n, kd) for c in B], degree, True, bias, shape)
+    return _product(a, b, flat(A, m, kd), flat(B, kd, n), degree, False, bias, shape)
 
 
 def _kernel_bias(bias, a, b, columns):
@@ -187,8 +189,7 @@ def linear(x, weight, bias=None):
     lead = X[0].shape[:-1]
     X = [c.reshape(1, -1, in_features).contiguous() for c in X]
     W = [c.reshape(1, out_features, in_features).contiguous() for c in W]
-    out = _cauchy(X, W, degree, True, bias if inside else None)
-    result = PolyTensor.from_stacked(out.view(degree + 1, *lead, out_features))
+    result = _product(x, weight, X, W, degree, True, bias if inside else None, (*lead, out_features))
     if bias is not None and not inside:
         result = result + bias
     return result

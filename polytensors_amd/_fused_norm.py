@@ -171,10 +171,13 @@ def _run(input, normalized_shape, weight, bias, eps, layer):
     w = _affine_coeffs(weight, input, shape)
     b = _affine_coeffs(bias, input, shape) if layer else []
     # a coefficient graph differentiates the affine terms as separate series operations
-    fused_affine = w is not None and b is not None and not _gate.coefficient_graph(input, weight, bias)
-    out = _ops.norm_series(x, w if fused_affine else [], b if fused_affine else [], math.prod(shape),
-                           float(eps), layer)
-    result = PolyTensor.from_stacked(out)
+    recorded = _gate.coefficient_graph(input, weight, bias)
+    fused_affine = w is not None and b is not None and not recorded
+    if recorded:
+        result = PolyTensor._wrap(tuple(_ops.norm_series_orders(x, [], [], math.prod(shape), float(eps), layer)))
+    else:
+        result = PolyTensor.from_stacked(_ops.norm_series(x, w if fused_affine else [], b if fused_affine else [],
+                                                          math.prod(shape), float(eps), layer))
     if not fused_affine:
         if weight is not None:
             result = result * weight

@@ -42,6 +42,11 @@ SCHEMAS = {
     "activation_series_backward": "(Tensor[] grad, Tensor[] saved, str kind) -> Tensor",
     "series_binary": "(Tensor[] a, Tensor[] b, str op) -> Tensor",
 }
+# The same results as a tensor per order, for calls whose coefficients autograd records: their
+# cotangents arrive order by order as they are. The slices of a stacked result are differentiated by
+# stacking their cotangents, a copy of the whole series for every operation.
+ORDERS = ("norm_series", "cauchy_matmul", "activation_series", "series_binary")
+SCHEMAS.update({f"{name}_orders": SCHEMAS[name][:-len("Tensor")] + "Tensor[]" for name in ORDERS})
 
 _fallback = []   # the Python library object of the stand-in schemas (kept alive)
 
@@ -255,6 +260,35 @@ def _(z, target, ignore_index, softcap, lse, cot):
     return z[0].new_empty((len(z), *z[0].shape))
 
 
+# The tensor-per-order forms.
+
+norm_series_orders = _op("norm_series_orders")
+cauchy_matmul_orders = _op("cauchy_matmul_orders")
+activation_series_orders = _op("activation_series_orders")
+series_binary_orders = _op("series_binary_orders")
+
+
+@torch.library.register_fake(f"{NAMESPACE}::norm_series_orders")
+def _(x, weight, bias, n, eps, layer):
+    return [x[0].new_empty(x[0].shape) for _ in x]
+
+
+@torch.library.register_fake(f"{NAMESPACE}::cauchy_matmul_orders")
+def _(a, b, degree, trans_b, bias=None):
+    n = b[0].shape[1] if trans_b else b[0].shape[2]
+    return [a[0].new_empty((max(a[0].shape[0], b[0].shape[0]), a[0].shape[1], n)) for _ in range(degree + 1)]
+
+
+@torch.library.register_fake(f"{NAMESPACE}::activation_series_orders")
+def _(x, kind):
+    return [x[0].new_empty(x[0].shape) for _ in x]
+
+
+@torch.library.register_fake(f"{NAMESPACE}::series_binary_orders")
+def _(a, b, op):
+    return [a[0].new_empty(a[0].shape) for _ in a]
+
+
 # ---------------------------------------------------------------------------
 # Coefficient-level autograd (PolyTensor.coefficient_autograd).
 #
@@ -279,8 +313,15 @@ def _(z, target, ignore_index, softcap, lse, cot):
 # series products (``_series_derivative``).
 
 def _reversed(grad):
-    """Cotangents of a stacked [K+1, ...] output in reverse order, as a coefficient list."""
-    return list(grad.flip(0).unbind(0))
+    """Cotangents of an output (stacked [K+1, ...], or a list of orders) in reverse order, as a list
+    of contiguous coefficients at 16-byte aligned places of their storage, as the kernels take them:
+    copied only where they are not."""
+    cots = list(grad.unbind(0)) if isinstance(grad, torch.Tensor) else list(grad)
+    if any(c is None for c in cots):   # an order that takes no part
+        zero = torch.zeros_like(next(c for c in cots if c is not None))
+        cots = [zero if c is None else c for c in cots]
+    return [c if c.is_contiguous() and c.storage_offset() * c.element_size() % 16 == 0
+            else c.clone(memory_format=torch.contiguous_format) for c in reversed(cots)]
 
 
 def _read_back(series, orders):
@@ -363,13 +404,14 @@ def _norm_backward(ctx, grad):
             y = _composed(_poly([c.reshape(-1, n) for c in xs]), (n,), None, None, eps, layer)
             return [c.reshape(xs[0].shape) for c in y.coeffs]
 
-        (dx,) = _regraded([x], list(grad.unbind(0)), compose)
+        (dx,) = _regraded([x], _reversed(grad)[::-1], compose)
         return _returned(ctx, dx, [], [])
     dx = norm_series_backward(x, _reversed(grad), n, eps, layer)
     return _returned(ctx, _read_back(dx, len(x)), [], [])
 
 
 torch.library.register_autograd(f"{NAMESPACE}::norm_series", _norm_backward, setup_context=_norm_setup)
+torch.library.register_autograd(f"{NAMESPACE}::norm_series_orders", _norm_backward, setup_context=_norm_setup)
 
 
 def _ce_setup(ctx, inputs, output):
@@ -431,7 +473,7 @@ def _mm_backward(ctx, grad):
     saved = ctx.saved_tensors
     a, b = list(saved[:na]), list(saved[na:])
     c = _reversed(grad)                     # [batch, m, n] each
-    batch = grad.shape[1]
+    batch = c[0].shape[0]
     ga = gb = None
     if need_a:   # dA = C (*) B^T
         if na == 1 and degree > 0 and _sums(c[0], b[0]):   # an ordinary A: coefficient K alone, sum_s C_{K-s} B_s^T
@@ -456,6 +498,7 @@ def _mm_backward(ctx, grad):
 
 
 torch.library.register_autograd(f"{NAMESPACE}::cauchy_matmul", _mm_backward, setup_context=_mm_setup)
+torch.library.register_autograd(f"{NAMESPACE}::cauchy_matmul_orders", _mm_backward, setup_context=_mm_setup)
 
 
 def _attn_setup(ctx, inputs, output):
@@ -517,10 +560,10 @@ _ACT_PRODUCT_BACKWARD = ("exp", "log", "sin", "cos", "sqrt", "rsqrt")
 
 def _act_setup(ctx, inputs, output):
     x, kind = inputs
-    ctx.kind = kind
+    ctx.kind, ctx.stacked = kind, isinstance(output, torch.Tensor)
     ctx.n_inputs = len(inputs)
     if kind in _ACT_SAVES_OUTPUT:
-        ctx.save_for_backward(output)
+        ctx.save_for_backward(*([output] if isinstance(output, torch.Tensor) else output))
     else:
         ctx.save_for_backward(*x)
 
@@ -569,7 +612,7 @@ def _act_backward(ctx, grad):
     if kind not in _ACT_PRODUCT_BACKWARD and not regraph:
         _once(f"activation_series ({kind})")
     saved = ctx.saved_tensors
-    saved = list(saved[0].unbind(0)) if kind in _ACT_SAVES_OUTPUT else list(saved)
+    saved = list(saved[0].unbind(0)) if kind in _ACT_SAVES_OUTPUT and len(saved) == 1 and ctx.stacked else list(saved)
     g = _reversed(grad)
     if regraph:            # a graph of the gradient: G (*) f' in differentiable series operations
         dx = series_binary(g, _series_derivative(kind, saved), "mul")
@@ -593,6 +636,7 @@ def _act_backward(ctx, grad):
 
 
 torch.library.register_autograd(f"{NAMESPACE}::activation_series", _act_backward, setup_context=_act_setup)
+torch.library.register_autograd(f"{NAMESPACE}::activation_series_orders", _act_backward, setup_context=_act_setup)
 
 
 def _binary_setup(ctx, inputs, output):
@@ -602,7 +646,9 @@ def _binary_setup(ctx, inputs, output):
     ctx.n_inputs = len(inputs)
     # (the quotient's output saved whole: a view of it made here would be saved without its
     # graph, and a second derivative would treat it as a constant)
-    ctx.save_for_backward(*a, *b, *([output] if op == "div" else []))
+    outputs = [output] if isinstance(output, torch.Tensor) else list(output)
+    ctx.stacked = isinstance(output, torch.Tensor)
+    ctx.save_for_backward(*a, *b, *(outputs if op == "div" else []))
 
 
 def _binary_backward(ctx, grad):
@@ -613,13 +659,14 @@ def _binary_backward(ctx, grad):
     if op == "mul":        # d(a b) = b da + a db
         da, db = series_binary(g, b, "mul"), series_binary(g, a, "mul")
     else:                  # d(a / b) = da / b - (a / b) db / b
-        y = list(s[2 * n].unbind(0))
+        y = list(s[2 * n].unbind(0)) if ctx.stacked else list(s[2 * n:])
         da = series_binary(g, b, "div")
         db = -series_binary(list(series_binary(g, y, "mul").unbind(0)), b, "div")
     return _returned(ctx, _read_back(da, n), _read_back(db, n))
 
 
 torch.library.register_autograd(f"{NAMESPACE}::series_binary", _binary_backward, setup_context=_binary_setup)
+torch.library.register_autograd(f"{NAMESPACE}::series_binary_orders", _binary_backward, setup_context=_binary_setup)
 
 
 # The complex-direction plumbing is linear in its inputs. Its gradients follow torch's

@@ -79,6 +79,29 @@ std::vector<int64_t> stacked_shape(int64_t orders, at::IntArrayRef shape) {
   return s;
 }
 
+// A series result: one coefficient-stacked [K+1, ...] tensor, or (the *_orders operators, used where
+// autograd records the coefficients) a tensor per order, whose cotangents autograd then hands back as
+// they are, where those of a stacked result's slices are first copied into one tensor.
+struct SeriesOut {
+  Tensor stacked;
+  TensorList orders;
+  std::vector<void*> ptrs;
+};
+
+SeriesOut series_out(bool separate, int64_t orders, at::IntArrayRef shape, const at::TensorOptions& options) {
+  SeriesOut o;
+  if (!separate) {
+    o.stacked = at::empty(stacked_shape(orders, shape), options);
+    o.ptrs = slices(o.stacked);
+    return o;
+  }
+  for (int64_t k = 0; k < orders; ++k) {
+    o.orders.push_back(at::empty(shape, options));
+    o.ptrs.push_back(o.orders.back().data_ptr());
+  }
+  return o;
+}
+
 void check_series(const std::string& name, const TensorList& c, c10::optional<at::ScalarType> want = c10::nullopt) {
   TORCH_CHECK_VALUE(!c.empty(), name, ": at least one coefficient is required");
   const Tensor& first = c[0];
@@ -95,8 +118,8 @@ void check_series(const std::string& name, const TensorList& c, c10::optional<at
 
 // ---- RMSNorm / LayerNorm series ----------------------------------------------
 
-Tensor norm_series(const TensorList& x, const TensorList& weight, const TensorList& bias, int64_t n, double eps,
-                   bool layer) {
+SeriesOut norm_series_out(bool separate, const TensorList& x, const TensorList& weight, const TensorList& bias, int64_t n,
+                          double eps, bool layer) {
   check_abi();
   check_series("norm_series", x);
   const int64_t degree = static_cast<int64_t>(x.size()) - 1;
@@ -113,9 +136,9 @@ Tensor norm_series(const TensorList& x, const TensorList& weight, const TensorLi
   }
   TORCH_CHECK_VALUE(layer || bias.empty(), "norm_series: bias is a LayerNorm argument");
   c10::DeviceGuard guard(x[0].device());
-  Tensor out = at::empty(stacked_shape(degree + 1, x[0].sizes()), x[0].options());
+  SeriesOut out = series_out(separate, degree + 1, x[0].sizes(), x[0].options());
   auto xs = cptrs(x), ws = cptrs(weight), bs = cptrs(bias);
-  auto ys = slices(out);
+  auto& ys = out.ptrs;
   const int code = dtype_code(x[0].scalar_type());
   int status;
   if (layer) {
@@ -128,6 +151,16 @@ Tensor norm_series(const TensorList& x, const TensorList& weight, const TensorLi
   }
   check_status(status, layer ? "layer_norm_series" : "rms_norm_series");
   return out;
+}
+
+Tensor norm_series(const TensorList& x, const TensorList& weight, const TensorList& bias, int64_t n, double eps,
+                   bool layer) {
+  return norm_series_out(false, x, weight, bias, n, eps, layer).stacked;
+}
+
+TensorList norm_series_orders(const TensorList& x, const TensorList& weight, const TensorList& bias, int64_t n, double eps,
+                              bool layer) {
+  return norm_series_out(true, x, weight, bias, n, eps, layer).orders;
 }
 
 Tensor norm_series_backward(const TensorList& x, const TensorList& grad, int64_t n, double eps, bool layer,
@@ -271,8 +304,8 @@ Rows packed_rows(const TensorList& in) {
   return {std::move(out), stride};
 }
 
-Tensor cauchy_matmul(const TensorList& a_in, const TensorList& b_in, int64_t degree, bool trans_b,
-                     const c10::optional<Tensor>& bias) {
+SeriesOut cauchy_matmul_out(bool separate, const TensorList& a_in, const TensorList& b_in, int64_t degree, bool trans_b,
+                            const c10::optional<Tensor>& bias) {
   check_abi();
   for (const auto& [name, s] : {std::pair<const char*, const TensorList*>{"a", &a_in}, {"b", &b_in}}) {
     const int64_t len = static_cast<int64_t>(s->size());
@@ -296,9 +329,9 @@ Tensor cauchy_matmul(const TensorList& a_in, const TensorList& b_in, int64_t deg
   const int64_t batch = std::max(ba, bb);
   c10::DeviceGuard guard(a_in[0].device());
   const Rows a = packed_rows(a_in), b = packed_rows(b_in);
-  Tensor out = at::empty({degree + 1, batch, m, n}, a_in[0].options());
+  SeriesOut out = series_out(separate, degree + 1, {batch, m, n}, a_in[0].options());
   auto as = cptrs(a.matrices), bs = cptrs(b.matrices);
-  auto cs = slices(out);
+  auto& cs = out.ptrs;
   const int status = pt_cauchy_matmul_strided(
       dtype_code(dtype), static_cast<int>(degree), as.data(), static_cast<int>(a_in.size()), bs.data(),
       static_cast<int>(b_in.size()), cs.data(), batch, m, n, kd, a.stride, b.stride, ba == 1 ? 0 : m * a.stride,
@@ -306,6 +339,16 @@ Tensor cauchy_matmul(const TensorList& a_in, const TensorList& b_in, int64_t deg
       stream_of(a_in[0]));
   check_status(status, "cauchy_matmul");
   return out;
+}
+
+Tensor cauchy_matmul(const TensorList& a, const TensorList& b, int64_t degree, bool trans_b,
+                     const c10::optional<Tensor>& bias) {
+  return cauchy_matmul_out(false, a, b, degree, trans_b, bias).stacked;
+}
+
+TensorList cauchy_matmul_orders(const TensorList& a, const TensorList& b, int64_t degree, bool trans_b,
+                                const c10::optional<Tensor>& bias) {
+  return cauchy_matmul_out(true, a, b, degree, trans_b, bias).orders;
 }
 
 // sum_s op(a_s) op(b_s) over pairs of [batch, rows, cols] matrices (float32, bfloat16, float16).
@@ -598,20 +641,28 @@ int activation_code(const std::string& kind, bool backward, const char* name) {
   TORCH_CHECK_VALUE(false, name, backward ? ": no backward for kind '" : ": unknown kind '", kind, "'");
 }
 
-Tensor activation_series(const TensorList& x, c10::string_view kind) {
+SeriesOut activation_series_out(bool separate, const TensorList& x, c10::string_view kind) {
   check_abi();
   check_series("activation_series", x);
   const std::string k(kind);
   const int code = activation_code(k, false, "activation_series");
   const int64_t degree = static_cast<int64_t>(x.size()) - 1;
   c10::DeviceGuard guard(x[0].device());
-  Tensor out = at::empty(stacked_shape(degree + 1, x[0].sizes()), x[0].options());
+  SeriesOut out = series_out(separate, degree + 1, x[0].sizes(), x[0].options());
   auto xs = cptrs(x);
-  auto ys = slices(out);
+  auto& ys = out.ptrs;
   check_status(pt_activation_series_fwd(dtype_code(x[0].scalar_type()), static_cast<int>(degree), code, xs.data(),
                                         ys.data(), x[0].numel(), stream_of(x[0])),
                "activation_series(" + k + ")");
   return out;
+}
+
+Tensor activation_series(const TensorList& x, c10::string_view kind) {
+  return activation_series_out(false, x, kind).stacked;
+}
+
+TensorList activation_series_orders(const TensorList& x, c10::string_view kind) {
+  return activation_series_out(true, x, kind).orders;
 }
 
 Tensor activation_series_backward(const TensorList& grad, const TensorList& saved, c10::string_view kind) {
@@ -635,7 +686,7 @@ Tensor activation_series_backward(const TensorList& grad, const TensorList& save
   return out;
 }
 
-Tensor series_binary(const TensorList& a, const TensorList& b, c10::string_view op) {
+SeriesOut series_binary_out(bool separate, const TensorList& a, const TensorList& b, c10::string_view op) {
   check_abi();
   check_series("series_binary a", a);
   check_series("series_binary b", b);
@@ -646,14 +697,22 @@ Tensor series_binary(const TensorList& a, const TensorList& b, c10::string_view 
   TORCH_CHECK_VALUE(o == "mul" || o == "div", "series_binary: unknown operation '", o, "'");
   const int64_t degree = static_cast<int64_t>(a.size()) - 1;
   c10::DeviceGuard guard(a[0].device());
-  Tensor out = at::empty(stacked_shape(degree + 1, a[0].sizes()), a[0].options());
+  SeriesOut out = series_out(separate, degree + 1, a[0].sizes(), a[0].options());
   auto as = cptrs(a), bs = cptrs(b);
-  auto ys = slices(out);
+  auto& ys = out.ptrs;
   check_status(pt_series_binary(dtype_code(a[0].scalar_type()), static_cast<int>(degree),
                                 o == "mul" ? PT_BINARY_MUL : PT_BINARY_DIV, as.data(), bs.data(), ys.data(),
                                 a[0].numel(), stream_of(a[0])),
                "series_binary(" + o + ")");
   return out;
+}
+
+Tensor series_binary(const TensorList& a, const TensorList& b, c10::string_view op) {
+  return series_binary_out(false, a, b, op).stacked;
+}
+
+TensorList series_binary_orders(const TensorList& a, const TensorList& b, c10::string_view op) {
+  return series_binary_out(true, a, b, op).orders;
 }
 
 }  // namespace
@@ -676,6 +735,10 @@ TORCH_LIBRARY(polytensors_amd, m) {
   m.def("activation_series(Tensor[] x, str kind) -> Tensor");
   m.def("activation_series_backward(Tensor[] grad, Tensor[] saved, str kind) -> Tensor");
   m.def("series_binary(Tensor[] a, Tensor[] b, str op) -> Tensor");
+  m.def("norm_series_orders(Tensor[] x, Tensor[] weight, Tensor[] bias, int n, float eps, bool layer) -> Tensor[]");
+  m.def("cauchy_matmul_orders(Tensor[] a, Tensor[] b, int degree, bool trans_b, Tensor? bias=None) -> Tensor[]");
+  m.def("activation_series_orders(Tensor[] x, str kind) -> Tensor[]");
+  m.def("series_binary_orders(Tensor[] a, Tensor[] b, str op) -> Tensor[]");
 }
 
 TORCH_LIBRARY_IMPL(polytensors_amd, CUDA, m) {
@@ -692,4 +755,8 @@ TORCH_LIBRARY_IMPL(polytensors_amd, CUDA, m) {
   m.impl("activation_series", &activation_series);
   m.impl("activation_series_backward", &activation_series_backward);
   m.impl("series_binary", &series_binary);
+  m.impl("norm_series_orders", &norm_series_orders);
+  m.impl("cauchy_matmul_orders", &cauchy_matmul_orders);
+  m.impl("activation_series_orders", &activation_series_orders);
+  m.impl("series_binary_orders", &series_binary_orders);
 }

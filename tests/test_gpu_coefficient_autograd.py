@@ -299,3 +299,42 @@ def test_gradient_of_an_ordinary_matrix(dtype, tol, m, k, n, batch, degree):
         # (a batch's gradients are rounded before they are summed)
         err = (got.cpu().double() - want).abs().max() / want.abs().max()
         assert err <= tol * (2 if batch else 1), (name, err)
+
+
+# The recorded operations return a tensor per order: cotangents of some orders alone, non-contiguous
+# and misaligned ones, and an order's gradient from another order's output are what torch's autograd of
+# the same series arithmetic gives (the oracle's, differentiated), for each of the four operations.
+@pytest.mark.parametrize("name", ["linear", "tanh", "product", "quotient", "rms_norm"])
+@pytest.mark.parametrize("wanted", [(0,), (2,), (0, 3), (0, 1, 2, 3)])
+def test_cotangents_of_some_orders(name, wanted):
+    degree, n = 3, 24
+    g = torch.Generator().manual_seed(len(name))
+    X = [torch.randn(5, n, generator=g, dtype=torch.float64) * 0.5 ** k + (2.0 if k == 0 else 0.0) for k in range(degree + 1)]
+    Y = [torch.randn(5, n, generator=g, dtype=torch.float64) * 0.5 ** k + (3.0 if k == 0 else 0.0) for k in range(degree + 1)]
+    W = torch.randn(n, n, generator=g, dtype=torch.float64)
+    calls = {"linear": (lambda x, y: F.linear(x, W.cuda()), lambda x, y: [c @ W.t() for c in x]),
+             "tanh": (lambda x, y: torch.tanh(x), lambda x, y: oracle.activation(x, "tanh")),
+             "product": (lambda x, y: x * y, lambda x, y: oracle.cauchy(x, y)),
+             "quotient": (lambda x, y: x / y, lambda x, y: oracle.quotient(x, y)),
+             "rms_norm": (lambda x, y: F.rms_norm(x, (n,), eps=1e-6), lambda x, y: oracle.rms_norm(x, (n,), eps=1e-6))}
+    call, plain = calls[name]
+    cots = []
+    for k in wanted:   # contiguous, transposed, one element into its buffer
+        c = torch.randn(5, n, generator=g, dtype=torch.float64)
+        d = c.cuda()
+        if k == 2:
+            d = c.t().contiguous().cuda().t()
+        elif k == 3:
+            d = torch.cat([torch.zeros(1, dtype=torch.float64), c.flatten()]).cuda()[1:].view(5, n)
+        cots.append((c, d))
+    leaves = [c.cuda().requires_grad_() for c in X + Y]
+    with PolyTensor.plain_range(), PolyTensor.coefficient_autograd():
+        out = call(PolyTensor(tuple(leaves[:degree + 1])), PolyTensor(tuple(leaves[degree + 1:])))
+    got = torch.autograd.grad([out.coeffs[k] for k in wanted], leaves, [d for _, d in cots], allow_unused=True)
+    ref = [c.clone().requires_grad_() for c in X + Y]
+    want = torch.autograd.grad([plain(ref[:degree + 1], ref[degree + 1:])[k] for k in wanted], ref, [c for c, _ in cots],
+                               allow_unused=True)
+    for i, (a, b) in enumerate(zip(got, want)):
+        a = torch.zeros(5, n, dtype=torch.float64) if a is None else a.cpu()
+        b = torch.zeros(5, n, dtype=torch.float64) if b is None else b
+        assert (a - b).abs().max().item() <= 1e-10 * max(1.0, b.abs().max().item()), (i, a, b)
