@@ -245,6 +245,27 @@ def _nodes(fn, what, args, kwargs, values, recorded):
     return _combine(outputs, weights)
 
 
+def at_stacked_nodes(fn, what, *operands, **kwargs):
+    """``at_real_nodes`` with every node in one call of ``fn``, along a new leading dimension of the
+    operands (series or ordinary tensors), for an operation that treats leading dimensions as a
+    batch and a call that no autograd records. One launch of all nodes' work where a node's alone
+    leaves compute units idle; order 0 is repeated for every node."""
+    _check(operands, what)
+    degree = next(v.degree for v in operands if isinstance(v, PolyTensor))
+    nodes, weights = nodes_and_weights(degree)
+
+    def stacked(x):
+        if _is_complex_series(x):
+            return PolyTensor._wrap(_ops.complex_at_nodes(x.coeffs[0], _planes(x), list(nodes)).unbind(0))
+        repeat = lambda c: c.expand(len(nodes), *c.shape).contiguous()   # noqa: E731
+        return PolyTensor._wrap(tuple(map(repeat, x.coeffs))) if isinstance(x, PolyTensor) else repeat(x)
+
+    y = fn(*map(stacked, operands), **kwargs)
+    src = [c[m] for m in range(len(nodes)) for c in y.coeffs[1:]]
+    planes = _ops.real_to_complex(src, degree, [w.real for w in weights], [w.imag for w in weights])
+    return PolyTensor((y.coeffs[0][0].clone(),) + tuple(planes.unbind(0)))
+
+
 def has_complex_base(*values):
     """Whether any operand is complex in its constant term: a series with a complex order 0, or a
     complex ordinary tensor."""

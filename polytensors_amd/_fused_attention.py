@@ -226,6 +226,17 @@ def _composed(query, key, value, attn_mask, is_causal, scale):
 def attention_checked(query, key, value, attn_mask=None, is_causal=False, scale=None):
     """``attention`` for a call whose eligibility (including dropout and GQA) the caller checked."""
     if _complex.has_complex(query, key, value):
+        # A node's launch has a workgroup per head and 64 queries; with up to 8 a CU their number does
+        # not balance a causal launch, whose workgroups' work differs (24 heads of 512 float32 queries,
+        # d 64, degree 3: 170 us for each of 4 nodes, 337 us for all of them at once), and past it
+        # the repeated order 0 buys nothing.
+        workgroups = math.prod(query.shape[:-2]) * -(-query.shape[-2] // 64)
+        shared = attn_mask is None or attn_mask.numel() == query.shape[-2] * key.shape[-2]   # (no mask per node and head)
+        degree = next(x.degree for x in (query, key, value) if isinstance(x, PolyTensor))
+        if (0 < workgroups < 2048 and shared and degree <= _gate.MAX_DEGREE and not _needs_grad(query, key, value)
+                and not _gate.coefficient_graph(query, key, value)):
+            return _complex.at_stacked_nodes(attention, "scaled_dot_product_attention", query, key, value,
+                                             attn_mask=attn_mask, is_causal=is_causal, scale=scale)
         return _complex.at_real_nodes(attention, "scaled_dot_product_attention", query, key, value,
                                       attn_mask=attn_mask, is_causal=is_causal, scale=scale)
     degree = next(x.degree for x in (query, key, value) if isinstance(x, PolyTensor))

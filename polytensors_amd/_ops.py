@@ -37,6 +37,7 @@ SCHEMAS = {
                              "Tensor? mask, bool causal, float scale, int materialize=-1, int[]? mask_map=None) "
                              "-> (Tensor, Tensor, Tensor)"),
     "complex_to_real": "(Tensor[] src, float[] alpha, float[] beta) -> Tensor",
+    "complex_at_nodes": "(Tensor base, Tensor[] planes, float[] nodes) -> Tensor",
     "real_to_complex": "(Tensor[] src, int orders, float[] wre, float[] wim) -> Tensor",
     "activation_series": "(Tensor[] x, str kind) -> Tensor",
     "activation_series_backward": "(Tensor[] grad, Tensor[] saved, str kind) -> Tensor",
@@ -203,6 +204,15 @@ complex_to_real = _op("complex_to_real")
 @torch.library.register_fake(f"{NAMESPACE}::complex_to_real")
 def _(src, alpha, beta):
     return src[0].new_empty((len(alpha), len(src), *src[0].shape), dtype=_REAL_OF[src[0].dtype])
+
+
+# a series at all its interpolation nodes as one (no autograd: recorded calls run node by node)
+complex_at_nodes = _op("complex_at_nodes")
+
+
+@torch.library.register_fake(f"{NAMESPACE}::complex_at_nodes")
+def _(base, planes, nodes):
+    return base.new_empty((len(planes) + 1, len(nodes), *base.shape))
 
 
 real_to_complex = _op("real_to_complex")

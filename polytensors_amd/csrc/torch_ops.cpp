@@ -604,6 +604,41 @@ Tensor complex_to_real(const TensorList& src, at::ArrayRef<double> alpha, at::Ar
   return out;
 }
 
+// A complex-direction series (real order 0, complex planes 1..K) at real nodes: one real series over
+// a leading dimension of the nodes, [K+1, nodes, ...]; order 0 is the same at every node, order k is
+// Re c_k + node Im c_k.
+Tensor complex_at_nodes(const Tensor& base, const TensorList& planes, at::ArrayRef<double> nodes) {
+  check_abi();
+  TORCH_CHECK_VALUE(!planes.empty() && !nodes.empty(), "complex_at_nodes: planes and nodes required");
+  const Tensor& first = planes[0];
+  TORCH_CHECK_VALUE(first.scalar_type() == at::kComplexFloat || first.scalar_type() == at::kComplexDouble,
+                    "complex_at_nodes: complex64 or complex128 planes");
+  const at::ScalarType real = first.scalar_type() == at::kComplexFloat ? at::kFloat : at::kDouble;
+  TORCH_CHECK_VALUE(base.scalar_type() == real && base.sizes() == first.sizes() && base.device() == first.device(),
+                    "complex_at_nodes: the constant order must be real, of the planes' shape and device");
+  for (const Tensor& c : planes)
+    TORCH_CHECK_VALUE(c.scalar_type() == first.scalar_type() && c.sizes() == first.sizes() &&
+                          c.device() == first.device() && c.is_contiguous(),
+                      "complex_at_nodes: planes must share dtype, shape and device and be contiguous");
+  c10::DeviceGuard guard(first.device());
+  std::vector<int64_t> shape{static_cast<int64_t>(planes.size()) + 1, static_cast<int64_t>(nodes.size())};
+  shape.insert(shape.end(), first.sizes().begin(), first.sizes().end());
+  Tensor out = at::empty(shape, first.options().dtype(real));
+  out.select(0, 0).copy_(base.expand(at::IntArrayRef(shape).slice(1)));
+  const std::vector<double> alpha(nodes.size(), 1.0);
+  std::vector<void*> dst;   // plane (node a, order o) at a * orders + o
+  for (size_t a = 0; a < nodes.size(); ++a)
+    for (size_t o = 0; o < planes.size(); ++o)
+      dst.push_back(static_cast<char*>(out.data_ptr()) +
+                    ((o + 1) * out.stride(0) + a * out.stride(1)) * static_cast<int64_t>(out.element_size()));
+  auto ss = cptrs(planes);
+  const int status = pt_complex_to_real(dtype_code(real), static_cast<int>(planes.size()), ss.data(),
+                                        static_cast<int>(nodes.size()), alpha.data(), nodes.data(), dst.data(),
+                                        first.numel(), stream_of(first));
+  check_status(status, "complex_at_nodes");
+  return out;
+}
+
 Tensor real_to_complex(const TensorList& src, int64_t orders, at::ArrayRef<double> wre, at::ArrayRef<double> wim) {
   check_abi();
   const int64_t variants = static_cast<int64_t>(wre.size());
@@ -731,6 +766,7 @@ TORCH_LIBRARY(polytensors_amd, m) {
   m.def("taylor_attention_bwd(Tensor[] q, Tensor[] k, Tensor[] v, Tensor out, Tensor lse, Tensor[] grad, "
         "Tensor? mask, bool causal, float scale, int materialize=-1, int[]? mask_map=None) -> (Tensor, Tensor, Tensor)");
   m.def("complex_to_real(Tensor[] src, float[] alpha, float[] beta) -> Tensor");
+  m.def("complex_at_nodes(Tensor base, Tensor[] planes, float[] nodes) -> Tensor");
   m.def("real_to_complex(Tensor[] src, int orders, float[] wre, float[] wim) -> Tensor");
   m.def("activation_series(Tensor[] x, str kind) -> Tensor");
   m.def("activation_series_backward(Tensor[] grad, Tensor[] saved, str kind) -> Tensor");
@@ -751,6 +787,7 @@ TORCH_LIBRARY_IMPL(polytensors_amd, CUDA, m) {
   m.impl("taylor_attention_fwd", &taylor_attention_fwd);
   m.impl("taylor_attention_bwd", &taylor_attention_bwd);
   m.impl("complex_to_real", &complex_to_real);
+  m.impl("complex_at_nodes", &complex_at_nodes);
   m.impl("real_to_complex", &real_to_complex);
   m.impl("activation_series", &activation_series);
   m.impl("activation_series_backward", &activation_series_backward);

@@ -164,6 +164,41 @@ def test_attention(dtype, masking):
     _check(got.coeffs, oracle.attention(_up(Q, dtype), _up(K, dtype), _up(V, dtype), **kw), dtype)
 
 
+# All nodes in one launch (a leading dimension of the operands) or one after another (a mask per batch
+# entry, more workgroups than it pays for): ordinary, real and complex operands mixed, three
+# dimensions and four, masks that broadcast, one query.
+@pytest.mark.parametrize("at_once", [True, False])
+@pytest.mark.parametrize("case", ["plain key", "real value", "three dimensions", "shared mask", "batch mask", "one query"])
+def test_attention_nodes(monkeypatch, case, at_once):
+    from polytensors_amd import _complex
+    calls = []
+    original = _complex.at_stacked_nodes
+    monkeypatch.setattr(_complex, "at_stacked_nodes", lambda *a, **k: calls.append(1) or original(*a, **k))
+    dtype, degree, L, d = torch.float64, 3, 37, 16
+    lead = (3,) if case == "three dimensions" else (2, 3)
+    if not at_once:   # heads x query blocks past the limit
+        lead = (2048,) if case == "three dimensions" else (2, 1024)
+        degree, L = 1, 5
+    Q, K, V = (_series((*lead, 1 if case == "one query" and i == 0 else L, d), degree, 17 + i, scale=0.5) for i in range(3))
+    if case == "plain key":
+        K = [K[0]]
+    if case == "real value":
+        V = [c.real if c.is_complex() else c for c in V]
+    g = torch.Generator().manual_seed(3)
+    mask = None
+    if case.endswith("mask"):
+        mask = torch.rand(*((2, 1) if case == "batch mask" else ()), L, L, generator=g) < 0.7
+        mask[..., 0] = True
+    with torch.no_grad(), PolyTensor.plain_range():
+        k = K[0].cuda() if case == "plain key" else _poly(K, dtype)
+        got = F.scaled_dot_product_attention(_poly(Q, dtype), k, _poly(V, dtype),
+                                             attn_mask=None if mask is None else mask.cuda())
+    assert bool(calls) == (at_once and case != "batch mask")
+    zero = [torch.zeros_like(K[0], dtype=torch.complex128)] * degree
+    Kd = _up(K + zero if case == "plain key" else K, dtype)
+    _check(got.coeffs, oracle.attention(_up(Q, dtype), Kd, _up(V, dtype), attn_mask=mask), dtype)
+
+
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 @pytest.mark.parametrize("reduction", ["none", "mean", "sum"])
 def test_cross_entropy(reduction, dtype):
