@@ -9,11 +9,18 @@
 // 768 -> 3072, 1356 us (114 TFLOP/s) and 1281 (121).
 //
 // * Chunks of 64 bytes of contraction (32 halves, 16 floats) are moved into LDS by LDS DMA
-//   (half_mfma.h) in a ring of kRing buffers. The DMA of chunk c + kRing is issued when chunk c's
-//   operands are in registers, and waited for by a count (vmcnt) three chunks later, so a tile has
-//   three chunks of memory latency in flight where the two-buffer kernels have one.
+//   (half_mfma.h) into four buffers, two chunks at a time where an operand's rows run along the
+//   contraction: rows of 128 bytes, whole cache lines. A unit's DMA is issued when the operands of the
+//   unit whose buffers it takes are in registers, and waited for by a count (vmcnt).
+//   The rate a tile's operands arrive at is what bounds the halves: past its L2 a CU reads 64-byte
+//   segments at 56-66 GB/s and 128-byte ones at 85-95 (measured with a DMA-only kernel over 16 MB), and
+//   with single chunks of 64-byte rows the tiles ran at 50-57 GB/s a CU whatever the ring's depth (4, 5 or
+//   8 chunks), waves (4 or 8) and order of issue. Two together: 4096 x 1024 x 4096 at degree 3 130 -> 123 us in
+//   256 x 256 tiles and 177 -> 145 in 128 x 128 ones. With both operands along columns rows are longer
+//   than a line as they are, and single chunks, a deeper ring, are faster (the weight gradient below:
+//   190 us, 230 in pairs).
 // * Operands are read from LDS one chunk ahead into a second register set, so the LDS reads issue
-//   between the MFMAs of the chunk before: one barrier per chunk.
+//   between the MFMAs of the chunk before: one barrier per unit.
 // * Operands may be stored with the contraction along rows (A [m][k], B [n][k]) or along columns
 //   (A [k][m], B [k][n]), the latter read through transpose reads (halves) or element reads (floats):
 //   no operand is transposed in memory. The weight gradient of the layer pair above, which ran as a
@@ -115,15 +122,12 @@ struct OrderGemmParams {
   int tiles_m, tiles_n;         // of one order
 };
 
-constexpr int kOrderRing = 4;
-
 template <typename T, int WMW, int WNW, int FM, int FN>
 struct OrderTile {
   using B = OrderBlock<T>;
   static constexpr int BM = WMW * FM * B::S, BN = WNW * FN * B::S, BK = 64 / static_cast<int>(sizeof(T));
   static constexpr int kWaves = WMW * WNW, kThreads = kWaves * kWave;
   static constexpr int SA = BM / 16 / kWaves, SB = BN / 16 / kWaves;   // 1 KB DMA segments per wave and chunk
-  static constexpr size_t LDS = static_cast<size_t>(kOrderRing) * (BM + BN) * 64;
   static_assert(SA * 16 * kWaves == BM && SB * 16 * kWaves == BN, "whole DMA segments per wave");
 };
 
@@ -138,7 +142,10 @@ void order_gemm_kernel(OrderGemmParams<T> p) {
   using Tile = OrderTile<T, WMW, WNW, FM, FN>;
   using Blk = OrderBlock<T>;
   constexpr int BM = Tile::BM, BN = Tile::BN, BK = Tile::BK, V = 16 / static_cast<int>(sizeof(T));
-  constexpr int SA = Tile::SA, SB = Tile::SB, R = kOrderRing;
+  constexpr int SA = Tile::SA, SB = Tile::SB;
+  // chunks moved together, sets of them in LDS, buffers
+  constexpr int UNIT = A_COLS && B_COLS ? 1 : 2, SETS = 4 / UNIT, R = UNIT * SETS;
+  static_assert(static_cast<size_t>(R) * (BM + BN) * 64 <= 160 * 1024, "LDS budget");
   constexpr int CPA = A_COLS ? BM / V : 4, CPB = B_COLS ? BN / V : 4;   // 16-byte chunks per tile row
   __shared__ __attribute__((aligned(16))) T As[R][BM * BK];
   __shared__ __attribute__((aligned(16))) T Bs[R][BN * BK];
@@ -197,12 +204,12 @@ void order_gemm_kernel(OrderGemmParams<T> p) {
   }
   const int step_a = (A_COLS ? BK * p.lda : BK) * static_cast<int>(sizeof(T));
   const int step_b = (B_COLS ? BK * p.ldb : BK) * static_cast<int>(sizeof(T));
-  const int per_order = (p.k + BK - 1) / BK;
-  const int chunks = SUM ? per_order * p.orders : per_order;
+  const int per_term = (p.k + UNIT * BK - 1) / (UNIT * BK);   // units
+  const int units = SUM ? per_term * p.orders : per_term;
 
-  // the chunk to issue next: its term of the sum, its position, its buffer. Past the last chunk
-  // every lane is out of range (zeros nobody reads), so each chunk counts the same loads.
-  int is = 0, ik = 0, ibuf = 0, left = p.k;
+  // The unit to issue next: its term of the sum, its position, its buffers. Past the last one every lane
+  // is out of range (zeros nobody reads), so each unit counts the same loads.
+  int is = 0, ip = 0, ibuf = 0, left = p.k;
   BufferRsrc ra, rb;
   auto point = [&]() {   // the operands of term is (of order oa, ob)
     const int term = min(is, p.orders - 1);
@@ -211,30 +218,31 @@ void order_gemm_kernel(OrderGemmParams<T> p) {
     rb = buffer_rsrc(p.b.p[sb] + batch * p.b_bs, p.b_bytes);
   };
   point();
-  auto issue_segment = [&](int s) {   // segment s of the chunk: A's SA, then B's SB
+  auto issue_segment = [&](int i) {   // i / UNIT: the segment, A's SA then B's SB; i % UNIT: the chunk
+    const int s = i / UNIT, half = i % UNIT;
     if (s < SA) {
-      lds_dma16(&As[ibuf][(wave * SA + s) * (1024 / static_cast<int>(sizeof(T)))], ra,
-                ka[s] < left ? va[s] : kBufferOutOfRange);
+      lds_dma16(&As[ibuf + half][(wave * SA + s) * (1024 / static_cast<int>(sizeof(T)))], ra,
+                ka[s] < left - half * BK ? va[s] : kBufferOutOfRange);
       va[s] += step_a;
     } else {
       const int u = s - SA;
-      lds_dma16(&Bs[ibuf][(wave * SB + u) * (1024 / static_cast<int>(sizeof(T)))], rb,
-                kb[u] < left ? vb[u] : kBufferOutOfRange);
+      lds_dma16(&Bs[ibuf + half][(wave * SB + u) * (1024 / static_cast<int>(sizeof(T)))], rb,
+                kb[u] < left - half * BK ? vb[u] : kBufferOutOfRange);
       vb[u] += step_b;
     }
   };
   auto issued = [&]() {
-    ibuf = ibuf + 1 == R ? 0 : ibuf + 1;
-    left -= BK;
-    if (++ik == per_order) {
-      ik = 0;
+    ibuf = ibuf + UNIT == R ? 0 : ibuf + UNIT;
+    left -= UNIT * BK;
+    if (++ip == per_term) {
+      ip = 0;
       ++is;
       left = SUM && is < p.orders ? p.k : 0;
       if constexpr (SUM) {
 #pragma unroll
-        for (int s = 0; s < SA; ++s) va[s] -= per_order * step_a;
+        for (int s = 0; s < SA; ++s) va[s] -= UNIT * per_term * step_a;
 #pragma unroll
-        for (int s = 0; s < SB; ++s) vb[s] -= per_order * step_b;
+        for (int s = 0; s < SB; ++s) vb[s] -= UNIT * per_term * step_b;
         point();
       }
     }
@@ -265,40 +273,50 @@ void order_gemm_kernel(OrderGemmParams<T> p) {
       for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = Blk::mma(fa[set][fm], fb[set][fn], s, acc[fm][fn]);
   };
 
-  for (int i = 0; i < R; ++i) {
+  constexpr int LOADS = UNIT * (SA + SB);   // of a unit
+  for (int i = 0; i < SETS; ++i) {
 #pragma unroll
-    for (int s = 0; s < SA + SB; ++s) issue_segment(s);
+    for (int s = 0; s < LOADS; ++s) issue_segment(s);
     issued();
   }
-  order_wait_barrier<(R - 1) * (SA + SB)>();   // chunk 0 has landed, for every wave
+  order_wait_barrier<(SETS - 1) * LOADS>();   // unit 0 has landed, for every wave
 #pragma unroll
   for (int i = 0; i < FM + FN; ++i) read_operand(0, 0, i);
-  int buf = 1;
-  // Chunk c is in register set c % 2; chunks c + 1 .. c + R - 1 are in flight or landed. The
-  // operand reads of chunk c + 1 and the DMA of chunk c + R are spread between the MFMA rows of
-  // chunk c (fixed by the scheduling barriers), so the MFMAs start right after the barrier.
-  auto step = [&](int set) {
-    order_wait_barrier<(R - 2) * (SA + SB)>();   // chunk c + 1 has landed; chunk c's buffer has been read
+  // One chunk: its MFMAs from register set `set`, the operand reads of the next chunk from `buf`, and in
+  // the last chunk of unit j the DMA of unit j + SETS into the buffers of this one. The reads and the
+  // DMA are spread between the MFMA rows (fixed by the scheduling barriers).
+  auto step = [&](int set, int buf, bool issue) {
 #pragma unroll
     for (int fm = 0; fm < FM; ++fm) {
       multiply_row(set, fm);
 #pragma unroll
       for (int i = fm * (FM + FN) / FM; i < (fm + 1) * (FM + FN) / FM; ++i) read_operand(buf, set ^ 1, i);
+      if (issue) {
 #pragma unroll
-      for (int s = fm * (SA + SB) / FM; s < (fm + 1) * (SA + SB) / FM; ++s) issue_segment(s);
+        for (int s = fm * LOADS / FM; s < (fm + 1) * LOADS / FM; ++s) issue_segment(s);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
-    issued();
-    buf = buf + 1 == R ? 0 : buf + 1;
   };
-  int c = 0;
-  for (; c + 1 < chunks; c += 2) {
-    step(0);
-    step(1);
-  }
-  if (c < chunks) {
-#pragma unroll
-    for (int fm = 0; fm < FM; ++fm) multiply_row(0, fm);
+  int buf = 0;
+  auto last_of_unit = [&](int set) {
+    order_wait_barrier<(SETS - 2) * LOADS>();   // unit j + 1 has landed; every wave has read unit j
+    buf = buf + UNIT == R ? 0 : buf + UNIT;
+    step(set, buf, true);
+    issued();
+  };
+  if constexpr (UNIT == 2) {
+    for (int j = 0; j < units; ++j) {
+      step(0, buf + 1, false);
+      last_of_unit(1);
+    }
+  } else {
+    int j = 0;
+    for (; j + 1 < units; j += 2) {
+      last_of_unit(0);
+      last_of_unit(1);
+    }
+    if (j < units) last_of_unit(0);
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // no DMA outlives the workgroup's LDS
 
@@ -362,8 +380,8 @@ static int launch_order_tile(OrderGemmParams<T> p, int64_t batch, hipStream_t st
 
 // The tile: the one with the least estimated time per chunk of contraction over the launch.
 // * Halves: 256 x 256 (one workgroup of 8 waves a CU) takes 0.80 us a chunk with every CU busy, and
-//   128 x 128 (up to two workgroups of 4 waves a CU) 0.57 us with two and 0.35 with one (from 8192^3
-//   at 809 and 1173 us, and 512 chunks of 256 small tiles at 178 us): four small tiles cost 1.4
+//   128 x 128 (up to two workgroups of 4 waves a CU) 0.49 us with two and 0.34 with one (from 8192^3
+//   at 820 and 1007 us, and 512 chunks of 256 small tiles at 176 us): four small tiles cost 1.2
 //   times a large one where both fill the chip, less where the large ones leave CUs idle.
 // * Floats: 128 x 128, 128 x 64 and 64 x 64 (two, three and five workgroups a CU); MFMA-bound, so the
 //   busiest CU's tiles count, at 137, 133 and 128 TFLOP/s (8192 x 768 x 3072, degree 3).
@@ -375,7 +393,7 @@ static int launch_order_gemm(const OrderGemmParams<T>& p, int64_t batch, hipStre
   if constexpr (sizeof(T) == 2) {
     const int64_t large = tiles(256, 256), small = tiles(128, 128), rest = small % 512;
     const double t_large = 0.80 * static_cast<double>((large + 255) / 256);
-    const double t_small = 0.57 * static_cast<double>(small / 512) + (rest == 0 ? 0.0 : rest <= 256 ? 0.35 : 0.57);
+    const double t_small = 0.49 * static_cast<double>(small / 512) + (rest == 0 ? 0.0 : rest <= 256 ? 0.34 : 0.49);
     if (t_large < t_small) return launch_order_tile<T, 2, 4, 8, 4, A_COLS, B_COLS, SUM>(p, batch, stream);
     return launch_order_tile<T, 2, 2, 4, 4, A_COLS, B_COLS, SUM>(p, batch, stream);
   } else {
