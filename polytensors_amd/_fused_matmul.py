@@ -160,13 +160,13 @@ def matmul(a, b, below_autograd=False, bias=None):
 
 def _kernel_bias(bias, a, b, columns):
     """Whether the kernel of the product of a and b adds this bias: an ordinary vector of its
-    ``columns``, of the operands' dtype and device, that no graph is recorded for, to the kernel's
-    degree."""
+    ``columns``, of the operands' dtype and device, that no graph is recorded for and no function
+    transform follows, to the kernel's degree."""
     if not isinstance(bias, torch.Tensor) or isinstance(bias, PolyTensor) or (torch.is_grad_enabled() and
                                                                               bias.requires_grad):
         return False
     return (bias.dtype == b.dtype and bias.device == b.device and tuple(bias.shape) == (columns,) and
-            bias.is_contiguous() and _degree(a, b) <= _gate.MAX_DEGREE)
+            bias.is_contiguous() and not _gate.transformed(bias) and _degree(a, b) <= _gate.MAX_DEGREE)
 
 
 def linear(x, weight, bias=None):

@@ -67,7 +67,7 @@ def _affine_coeffs(a, input, shape):
 
 def _ordinary_affine(a, input, shape):
     """An ordinary weight or bias without a graph as the kernels take it ([n], contiguous), else None."""
-    if a is None or isinstance(a, PolyTensor) or a.requires_grad:
+    if a is None or isinstance(a, PolyTensor) or a.requires_grad or _gate.transformed(a):
         return None
     coeffs = _affine_coeffs(a, input, shape)
     return coeffs[0] if coeffs else None

@@ -9,6 +9,7 @@ device is never a reason: it raises LibraryMissingError.
 """
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 from ._plain import plain_range_enabled
@@ -107,3 +108,9 @@ def wrapper_grad(*values):
     if _coefficient_autograd_enabled.get() or not torch.is_grad_enabled():
         return False
     return any(isinstance(v, torch.Tensor) and v.requires_grad for v in values)
+
+
+def transformed(t):
+    """Whether a function transform may follow the ordinary tensor t (forward-mode differentiation,
+    vmap): a kernel that takes it as a constant operand would drop its tangent."""
+    return forward_ad._current_level >= 0 or torch._C._functorch.is_functorch_wrapped_tensor(t)

@@ -186,3 +186,23 @@ def test_masks_and_class_weights_that_require_grad_are_refused():
     assert "require grad" in _fused_cross_entropy.why_ineligible(z, y, w)
     with torch.no_grad():
         assert "requires grad" not in (_fused_attention.why_ineligible(x, x, x, mask, 0.0, False, False) or "")
+
+
+def test_transformed_bias_and_weight_are_not_kernel_operands():
+    """A bias or weight with a forward-mode tangent, or under vmap, is no constant of a kernel: it would
+    lose its tangent, or its batch, without an error."""
+    import torch.autograd.forward_ad as forward_ad
+
+    from polytensors_amd import _fused_matmul, _fused_norm
+
+    x, weight, bias = PolyTensor((torch.ones(3, 4), torch.ones(3, 4))), torch.ones(5, 4), torch.ones(5)
+
+    def taken(b):
+        return _fused_matmul._kernel_bias(b, x, weight, 5), _fused_norm._ordinary_affine(b, PolyTensor((bias, bias)), (5,)) is not None
+
+    assert taken(bias) == (True, True)
+    with forward_ad.dual_level():
+        assert taken(forward_ad.make_dual(bias, torch.ones(5))) == (False, False)
+    seen = []
+    torch.func.vmap(lambda b: (seen.append(taken(b)), b)[1])(torch.ones(2, 5))
+    assert seen == [(False, False)]
