@@ -292,8 +292,11 @@ Rows packed_rows(const TensorList& in) {
   for (const Tensor& t : in)
     whole = whole && (reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 || first.scalar_type() == at::kDouble);
   if (whole) return {in, cols};
-  const int64_t unit = cols * static_cast<int64_t>(first.element_size()) >= 512 ? 8 * vec : vec;
-  const int64_t stride = (cols + unit - 1) / unit * unit;
+  auto padded = [&](int64_t unit) { return (cols + unit - 1) / unit * unit; };
+  int64_t stride = padded(vec);
+  if (cols * static_cast<int64_t>(first.element_size()) >= 512 &&
+      first.size(1) * padded(8 * vec) * static_cast<int64_t>(first.element_size()) < int64_t{1} << 30)
+    stride = padded(8 * vec);   // (not where it alone takes a matrix past the kernels' 1 GiB)
   Tensor buffer = at::empty({static_cast<int64_t>(in.size()), first.size(0), first.size(1), stride}, first.options());
   TensorList out = buffer.unbind(0);
   auto from = cptrs(in);

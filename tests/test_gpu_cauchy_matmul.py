@@ -242,3 +242,25 @@ def test_linear_bias(dtype, tol, m, k, n, weight):
         for o in range(degree + 1):
             err = (out.coeffs[o].detach().cpu().to(want[o].dtype) - want[o]).abs().max() / want[o].abs().max()
             assert err <= 2 * tol, (o, err)   # (twice: the separate addition rounds again)
+
+
+# Rows that whole cache lines would pad past the kernels' 1 GiB a matrix, and whole vectors do not: padded to
+# vectors. Products and the gradient of the ordinary operand, on the first and last rows.
+@pytest.mark.parametrize("rows,k", [(1_800_000, 257)])
+def test_padded_rows_stay_below_the_limit(rows, k):
+    n = 8
+    g = torch.Generator(device="cuda").manual_seed(0)
+    X = [torch.randn(rows, k, generator=g, device="cuda", dtype=torch.bfloat16) for _ in range(2)]
+    w = torch.randn(k, n, generator=g, device="cuda", dtype=torch.bfloat16).requires_grad_()
+    cot = [torch.randn(rows, n, generator=g, device="cuda", dtype=torch.bfloat16) for _ in range(2)]
+    with PolyTensor.plain_range(), PolyTensor.coefficient_autograd():
+        y = PolyTensor(tuple(X)) @ w
+    (dw,) = torch.autograd.grad(y.coeffs, [w], cot)
+    for o in range(2):
+        for part in (slice(0, 300), slice(rows - 300, rows)):
+            want = X[o][part].float() @ w.detach().float()
+            assert (y.coeffs[o].detach()[part].float() - want).abs().max() <= 2.0 ** -8 * want.abs().max()
+    want = sum(sum(x[i:i + 65536].T.double() @ c[i:i + 65536].double() for i in range(0, rows, 65536))
+               for x, c in zip(X, cot))
+    # float32 sums of 3.6 million terms of magnitude one, rounded to bfloat16
+    assert (dw.double() - want).abs().max() <= 2.0 ** -7 * want.abs().max()
