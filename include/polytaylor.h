@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define PT_ABI_VERSION 14
+#define PT_ABI_VERSION 15
 #define PT_MAX_DEGREE 8
 /* Largest degree of the elementwise kernels (pt_activation_series_*, pt_series_binary): their
  * register plans are per element, so they run above PT_MAX_DEGREE. */
@@ -484,6 +484,17 @@ int pt_activation_series_fwd(int dtype, int degree, int kind,
 int pt_activation_series_bwd(int dtype, int degree, int kind,
                              const void* const* g, const void* const* saved,
                              void* const* dx, int64_t numel, void* stream);
+
+/*
+ * y(t) = f(x(t)) along a complex direction over a real constant order (complex_planes.hip's evaluation
+ * at degree + 1 real nodes, combined): order 0 f(x_0), order k = 1..degree
+ *   y_k = sum_m (wre_m + i wim_m) f(x_0 + sum_j (Re x_j + nodes_m Im x_j) t^j)_k.
+ * degree: 1..8. x0, y0: `numel` real elements; x, y: `degree` pointers to `numel` interleaved (re, im)
+ * pairs; nodes, wre, wim: degree + 1 values on the host. PT_FLOAT32 and PT_FLOAT64.
+ */
+int pt_complex_activation_fwd(int dtype, int degree, int kind, const void* x0, const void* const* x, void* y0,
+                              void* const* y, const double* nodes, const double* wre, const double* wim,
+                              int64_t numel, void* stream);
 
 /* Operations of pt_series_binary. */
 typedef enum pt_binary {

@@ -266,6 +266,15 @@ def at_stacked_nodes(fn, what, *operands, **kwargs):
     return PolyTensor((y.coeffs[0][0].clone(),) + tuple(planes.unbind(0)))
 
 
+def activation(x, kind):
+    """The series of an activation of a complex-direction series that no autograd records, in one
+    pass: the evaluation of ``at_real_nodes`` with every node inside the kernel."""
+    nodes, weights = nodes_and_weights(x.degree)
+    base, planes = _ops.complex_activation(x.coeffs[0].contiguous(), _planes(x), kind, list(nodes),
+                                           [w.real for w in weights], [w.imag for w in weights])
+    return PolyTensor((base,) + tuple(planes.unbind(0)))
+
+
 def has_complex_base(*values):
     """Whether any operand is complex in its constant term: a series with a complex order 0, or a
     complex ordinary tensor."""

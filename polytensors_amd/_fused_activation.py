@@ -146,6 +146,10 @@ def activation(x, kind):
     if _complex.has_complex_base(x):
         return _complex_base(x, kind)
     if _complex.has_complex(x):
+        # (a graph of the coefficients is recorded by the separate passes' operators)
+        recorded = torch.is_grad_enabled() and any(c.requires_grad for c in x.coeffs)
+        if x.degree <= _gate.MAX_DEGREE and not recorded and not any(map(_gate.transformed, x.coeffs)):
+            return _complex.activation(x, kind)
         return _complex.at_real_nodes_below_autograd(activation, kind, x, kind)
     if _gate.coefficient_graph(x):
         return PolyTensor._wrap(tuple(_ops.activation_series_orders(_coeffs(x, x.degree), kind)))

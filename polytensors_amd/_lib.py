@@ -15,7 +15,7 @@ import torch
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "libpolytaylor.so")
 # the operators' PyTorch registration (csrc/torch_ops.cpp), linked with libpolytaylor.so
 TORCH_LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "libpolytaylor_torch.so")
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 PT_OK, PT_INVALID_ARGUMENT, PT_UNSUPPORTED, PT_DEVICE_ERROR = 0, 1, 2, 3
 REDUCTIONS = {"none": 0, "mean": 1, "sum": 2}
@@ -83,6 +83,8 @@ SIGNATURES = {
     "pt_real_to_complex": (_c_int, [_c_int, _c_int, _c_int, _c_vpp, _c_dblp, _c_dblp, _c_vpp, _c_i64, _c_vp]),
     "pt_activation_series_fwd": (_c_int, [_c_int, _c_int, _c_int, _c_vpp, _c_vpp, _c_i64, _c_vp]),
     "pt_activation_series_bwd": (_c_int, [_c_int, _c_int, _c_int, _c_vpp, _c_vpp, _c_vpp, _c_i64, _c_vp]),
+    "pt_complex_activation_fwd": (_c_int, [_c_int, _c_int, _c_int, _c_vp, _c_vpp, _c_vp, _c_vpp, _c_vp, _c_vp, _c_vp,
+                                           _c_i64, _c_vp]),
     "pt_series_binary": (_c_int, [_c_int, _c_int, _c_int, _c_vpp, _c_vpp, _c_vpp, _c_i64, _c_vp]),
     "pt_rms_norm_series_bwd": (_c_int, [_c_int, _c_int, _c_vpp, _c_vpp, _c_vpp, _c_i64, _c_i64, _c_dbl, _c_vp]),
     "pt_norm_series_bwd_weighted": (_c_int, [_c_int, _c_int, _c_int, _c_vpp, _c_vpp, _c_vp, _c_vpp, _c_i64, _c_i64, _c_dbl,

@@ -40,6 +40,8 @@ SCHEMAS = {
     "complex_at_nodes": "(Tensor base, Tensor[] planes, float[] nodes) -> Tensor",
     "real_to_complex": "(Tensor[] src, int orders, float[] wre, float[] wim) -> Tensor",
     "activation_series": "(Tensor[] x, str kind) -> Tensor",
+    "complex_activation": ("(Tensor base, Tensor[] planes, str kind, float[] nodes, float[] wre, float[] wim) "
+                           "-> (Tensor, Tensor)"),
     "activation_series_backward": "(Tensor[] grad, Tensor[] saved, str kind) -> Tensor",
     "series_binary": "(Tensor[] a, Tensor[] b, str op) -> Tensor",
 }
@@ -213,6 +215,15 @@ complex_at_nodes = _op("complex_at_nodes")
 @torch.library.register_fake(f"{NAMESPACE}::complex_at_nodes")
 def _(base, planes, nodes):
     return base.new_empty((len(planes) + 1, len(nodes), *base.shape))
+
+
+# an activation along a complex direction: order 0 and the stacked complex planes (no autograd: as above)
+complex_activation = _op("complex_activation")
+
+
+@torch.library.register_fake(f"{NAMESPACE}::complex_activation")
+def _(base, planes, kind, nodes, wre, wim):
+    return base.new_empty(base.shape), planes[0].new_empty((len(planes), *base.shape))
 
 
 real_to_complex = _op("real_to_complex")

@@ -703,6 +703,39 @@ TensorList activation_series_orders(const TensorList& x, c10::string_view kind) 
   return activation_series_out(true, x, kind).orders;
 }
 
+// An activation of a complex-direction series: order 0 and the complex planes 1..K, stacked.
+std::tuple<Tensor, Tensor> complex_activation(const Tensor& base, const TensorList& planes, c10::string_view kind,
+                                              at::ArrayRef<double> nodes, at::ArrayRef<double> wre,
+                                              at::ArrayRef<double> wim) {
+  check_abi();
+  TORCH_CHECK_VALUE(!planes.empty(), "complex_activation: planes required");
+  const Tensor& first = planes[0];
+  TORCH_CHECK_VALUE(first.scalar_type() == at::kComplexFloat || first.scalar_type() == at::kComplexDouble,
+                    "complex_activation: complex64 or complex128 planes");
+  const at::ScalarType real = first.scalar_type() == at::kComplexFloat ? at::kFloat : at::kDouble;
+  TORCH_CHECK_VALUE(base.scalar_type() == real && base.sizes() == first.sizes() && base.device() == first.device() &&
+                        base.is_contiguous(),
+                    "complex_activation: the constant order must be real and contiguous, of the planes' shape and device");
+  for (const Tensor& c : planes)
+    TORCH_CHECK_VALUE(c.scalar_type() == first.scalar_type() && c.sizes() == first.sizes() &&
+                          c.device() == first.device() && c.is_contiguous(),
+                      "complex_activation: planes must share dtype, shape and device and be contiguous");
+  TORCH_CHECK_VALUE(nodes.size() == planes.size() + 1 && wre.size() == nodes.size() && wim.size() == nodes.size(),
+                    "complex_activation: one node and weight more than planes");
+  const std::string k(kind);
+  const int code = activation_code(k, false, "complex_activation");
+  c10::DeviceGuard guard(first.device());
+  Tensor y0 = at::empty(base.sizes(), base.options());
+  Tensor out = at::empty(stacked_shape(static_cast<int64_t>(planes.size()), first.sizes()), first.options());
+  auto xs = cptrs(planes);
+  auto ys = slices(out);
+  check_status(pt_complex_activation_fwd(dtype_code(real), static_cast<int>(planes.size()), code, base.data_ptr(), xs.data(),
+                                         y0.data_ptr(), ys.data(), nodes.data(), wre.data(), wim.data(), first.numel(),
+                                         stream_of(first)),
+               "complex_activation(" + k + ")");
+  return {y0, out};
+}
+
 Tensor activation_series_backward(const TensorList& grad, const TensorList& saved, c10::string_view kind) {
   check_abi();
   check_series("activation_series_backward grad", grad);
@@ -772,6 +805,8 @@ TORCH_LIBRARY(polytensors_amd, m) {
   m.def("complex_at_nodes(Tensor base, Tensor[] planes, float[] nodes) -> Tensor");
   m.def("real_to_complex(Tensor[] src, int orders, float[] wre, float[] wim) -> Tensor");
   m.def("activation_series(Tensor[] x, str kind) -> Tensor");
+  m.def("complex_activation(Tensor base, Tensor[] planes, str kind, float[] nodes, float[] wre, float[] wim) "
+        "-> (Tensor, Tensor)");
   m.def("activation_series_backward(Tensor[] grad, Tensor[] saved, str kind) -> Tensor");
   m.def("series_binary(Tensor[] a, Tensor[] b, str op) -> Tensor");
   m.def("norm_series_orders(Tensor[] x, Tensor[] weight, Tensor[] bias, int n, float eps, bool layer) -> Tensor[]");
@@ -793,6 +828,7 @@ TORCH_LIBRARY_IMPL(polytensors_amd, CUDA, m) {
   m.impl("complex_at_nodes", &complex_at_nodes);
   m.impl("real_to_complex", &real_to_complex);
   m.impl("activation_series", &activation_series);
+  m.impl("complex_activation", &complex_activation);
   m.impl("activation_series_backward", &activation_series_backward);
   m.impl("series_binary", &series_binary);
   m.impl("norm_series_orders", &norm_series_orders);

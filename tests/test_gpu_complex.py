@@ -130,6 +130,38 @@ def test_activations(kind, dtype):
     _check(got.coeffs, oracle.activation(_up(X, dtype), kind), dtype)
 
 
+# The fused kernel against the same nodes run one by one: element counts around a vector and a block, planes
+# and base that start at any element (the element path), every kind and degree. Both paths run the same series
+# code; the node's series x_k = Re + lam Im and the combination round (or contract) differently, a few units
+# of the largest node's values times the weights.
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("degree,numel,offset", [(1, 1, 0), (2, 3, 0), (3, 4, 0), (3, 1023, 1), (4, 1026, 0), (5, 1025, 1),
+                                                 (6, 7, 0), (7, 514, 0), (8, 2051, 0)])
+@pytest.mark.parametrize("kind", ["gelu", "gelu_tanh", "tanh", "sigmoid", "silu", "exp", "log", "sin", "cos", "sqrt",
+                                  "rsqrt"])
+def test_activation_nodes_in_one_pass(kind, degree, numel, offset, dtype):
+    from polytensors_amd import _complex, _fused_activation
+
+    g = torch.Generator().manual_seed(degree)
+    draw = lambda: torch.randn(numel + offset, generator=g, dtype=torch.float64)   # noqa: E731
+    base = (draw().abs() + 1 if kind in ("log", "sqrt", "rsqrt") else draw()).to(dtype).cuda()[offset:]
+    wide = torch.complex64 if dtype == torch.float32 else torch.complex128
+    x = PolyTensor((base,) + tuple((0.3 * torch.complex(draw(), draw())).to(wide).cuda()[offset:] for _ in range(degree)))
+    with torch.no_grad(), PolyTensor.plain_range():
+        got = _fused_activation.activation(x, kind)
+        nodes, weights = _complex.nodes_and_weights(degree)
+        at = [_fused_activation.activation(v, kind) for v in _complex._variants(x, [1.0] * len(nodes), nodes)]
+    order0 = at[0].coeffs[0]
+    assert ((got.coeffs[0] - order0).abs() <= 4 * torch.finfo(dtype).eps * order0.abs()).all()
+    for k in range(1, degree + 1):
+        ys = [y.coeffs[k].double() for y in at]
+        want = sum(w * y for w, y in zip(weights, ys))
+        # (the combination is taken element by element)
+        scale = sum(abs(w) * y.abs() for w, y in zip(weights, ys)) + sum(map(abs, weights)) * max(
+            c.abs().max().item() for y in at for c in y.coeffs)
+        assert ((got.coeffs[k].to(torch.complex128) - want).abs() <= 32 * torch.finfo(dtype).eps * scale).all(), k
+
+
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 @pytest.mark.parametrize("layer", [False, True])
 def test_norms(layer, dtype):
