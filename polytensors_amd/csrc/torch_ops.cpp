@@ -284,13 +284,13 @@ struct Rows {
 // MFMAs, does not (1006 -> 973 us there, 57 -> 61 here), and is left to the kernel's element loads.
 // Rows of 512 bytes and more are padded to whole 128-byte cache lines: a tile's row segments of 64 to
 // 256 bytes otherwise straddle lines (4 x 511 x 1023 x 769 bfloat16, degree 4: 85 -> 77 us).
-Rows packed_rows(const TensorList& in) {
+Rows packed_rows(const TensorList& in, bool elements = false) {   // elements: any rows do, nothing is copied
   const Tensor& first = in[0];
   const int64_t cols = first.size(2), rows = first.size(0) * first.size(1);
   const int64_t vec = 16 / static_cast<int64_t>(first.element_size());
-  bool whole = cols % vec == 0 || first.scalar_type() == at::kDouble;
-  for (const Tensor& t : in)
-    whole = whole && (reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 || first.scalar_type() == at::kDouble);
+  bool whole = cols % vec == 0;
+  for (const Tensor& t : in) whole = whole && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  whole = whole || elements;
   if (whole) return {in, cols};
   auto padded = [&](int64_t unit) { return (cols + unit - 1) / unit * unit; };
   int64_t stride = padded(vec);
@@ -331,7 +331,13 @@ SeriesOut cauchy_matmul_out(bool separate, const TensorList& a_in, const TensorL
                     "cauchy_matmul: bias must be a contiguous [n] vector of the operands' dtype and device");
   const int64_t batch = std::max(ba, bb);
   c10::DeviceGuard guard(a_in[0].device());
-  const Rows a = packed_rows(a_in), b = packed_rows(b_in);
+  // float32 products below 2^28 multiply-adds take less time than the copies' launches gain (4 x 16 x 77 x 65
+  // at degree 4: 34 us, 45 with copies; 300 x 301 x 1001 by an ordinary matrix, 3.6e8 at degree 3: 44 and 26)
+  const int64_t terms = a_in.size() > 1 && b_in.size() > 1 ? (degree + 1) * (degree + 2) / 2
+                                                           : static_cast<int64_t>(std::max(a_in.size(), b_in.size()));
+  const bool elements = dtype == at::kDouble ||
+                        (dtype == at::kFloat && static_cast<double>(batch) * m * n * kd * terms < double(1 << 28));
+  const Rows a = packed_rows(a_in, elements), b = packed_rows(b_in, elements);
   SeriesOut out = series_out(separate, degree + 1, {batch, m, n}, a_in[0].options());
   auto as = cptrs(a.matrices), bs = cptrs(b.matrices);
   auto& cs = out.ptrs;

@@ -264,3 +264,20 @@ def test_padded_rows_stay_below_the_limit(rows, k):
                for x, c in zip(X, cot))
     # float32 sums of 3.6 million terms of magnitude one, rounded to bfloat16
     assert (dw.double() - want).abs().max() <= 2.0 ** -7 * want.abs().max()
+
+
+# float32 rows of no whole vectors, either side of the size from which they are copied with padded rows.
+@pytest.mark.parametrize("m,n,k", [(257, 259, 255), (300, 1001, 301)])
+@pytest.mark.parametrize("plain", [True, False])
+def test_float_rows_padded_by_size(m, n, k, plain):
+    degree, tol = 3, 1e-5
+    A, B = _series((m, k), degree, 1, torch.float32), _series((k, n), degree, 2, torch.float32)
+    if plain:
+        B = B[:1]
+    b = B[0].cuda() if plain else PolyTensor(tuple(c.cuda() for c in B))
+    with torch.no_grad(), PolyTensor.plain_range():
+        got = PolyTensor(tuple(c.cuda() for c in A)) @ b
+    up = lambda cs: [c.double() for c in cs]   # noqa: E731
+    want = [c @ up(B)[0] for c in up(A)] if plain else oracle.matmul(up(A), up(B))
+    for o in range(degree + 1):
+        assert (got.coeffs[o].cpu().double() - want[o]).abs().max() <= tol * want[o].abs().max(), o
