@@ -17,16 +17,16 @@
 //   with single chunks of 64-byte rows the tiles ran at 50-57 GB/s a CU whatever the ring's depth (4, 5 or
 //   8 chunks), waves (4 or 8) and order of issue. Two together: 4096 x 1024 x 4096 at degree 3 130 -> 123 us in
 //   256 x 256 tiles and 177 -> 145 in 128 x 128 ones. With both operands along columns rows are longer
-//   than a line as they are, and single chunks, a deeper ring, are faster (the weight gradient below:
-//   190 us, 230 in pairs).
+//   than a line as they are, and single chunks, a deeper ring, are faster (the weight gradient below,
+//   before its contraction was split: 190 us, 230 in pairs).
 // * Operands are read from LDS one chunk ahead into a second register set, so the LDS reads issue
 //   between the MFMAs of the chunk before: one barrier per unit.
 // * Operands may be stored with the contraction along rows (A [m][k], B [n][k]) or along columns
 //   (A [k][m], B [k][n]), the latter read through transpose reads (halves) or element reads (floats):
 //   no operand is transposed in memory. The weight gradient of the layer pair above, which ran as a
 //   full series product of transposed copies (K = 3: ten pairs for the four that the one order of a
-//   weight needs), took 283 us a product and 184 us of transposes, and takes 170 us (810 TFLOP/s:
-//   256 tiles of 128 x 128, one a CU).
+//   weight needs), took 283 us a product and 184 us of transposes, and takes 151 us (910 TFLOP/s:
+//   256 tiles of 128 x 128, one a CU, the contraction in two halves).
 #pragma once
 
 #include <algorithm>
@@ -136,8 +136,8 @@ __device__ __forceinline__ void order_wait_barrier() {   // at most N of this wa
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-template <typename T, int WMW, int WNW, int FM, int FN, bool A_COLS, bool B_COLS, bool SUM, int MIN_WAVES>
-__global__ __launch_bounds__(WMW* WNW* kWave) __attribute__((amdgpu_waves_per_eu(MIN_WAVES)))
+template <typename T, int WMW, int WNW, int FM, int FN, bool A_COLS, bool B_COLS, bool SUM, int SPLIT, int MIN_WAVES>
+__global__ __launch_bounds__(WMW* WNW* kWave* SPLIT) __attribute__((amdgpu_waves_per_eu(MIN_WAVES)))
 void order_gemm_kernel(OrderGemmParams<T> p) {
   using Tile = OrderTile<T, WMW, WNW, FM, FN>;
   using Blk = OrderBlock<T>;
@@ -145,13 +145,16 @@ void order_gemm_kernel(OrderGemmParams<T> p) {
   constexpr int SA = Tile::SA, SB = Tile::SB;
   // chunks moved together, sets of them in LDS, buffers
   constexpr int UNIT = A_COLS && B_COLS ? 1 : 2, SETS = 4 / UNIT, R = UNIT * SETS;
-  static_assert(static_cast<size_t>(R) * (BM + BN) * 64 <= 160 * 1024, "LDS budget");
+  static_assert(static_cast<size_t>(SPLIT) * R * (BM + BN) * 64 <= 160 * 1024, "LDS budget");
   constexpr int CPA = A_COLS ? BM / V : 4, CPB = B_COLS ? BN / V : 4;   // 16-byte chunks per tile row
-  __shared__ __attribute__((aligned(16))) T As[R][BM * BK];
-  __shared__ __attribute__((aligned(16))) T Bs[R][BN * BK];
+  __shared__ __attribute__((aligned(16))) T As[SPLIT * R][BM * BK];
+  __shared__ __attribute__((aligned(16))) T Bs[SPLIT * R][BN * BK];
 
   const int lane = threadIdx.x % kWave;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int wave = wave_id % Tile::kWaves;
+  const int part = SPLIT == 1 ? 0 : wave_id / Tile::kWaves;   // of the contraction
+  const int own = part * R;                                   // its buffers
   const int wm = wave / WNW, wn = wave % WNW;
 
   // Workgroup -> tile: consecutive ids go round robin over the 8 XCDs, so each XCD takes a
@@ -205,11 +208,20 @@ void order_gemm_kernel(OrderGemmParams<T> p) {
   const int step_a = (A_COLS ? BK * p.lda : BK) * static_cast<int>(sizeof(T));
   const int step_b = (B_COLS ? BK * p.ldb : BK) * static_cast<int>(sizeof(T));
   const int per_term = (p.k + UNIT * BK - 1) / (UNIT * BK);   // units
-  const int units = SUM ? per_term * p.orders : per_term;
+  const int units = ((SUM ? per_term * p.orders : per_term) + SPLIT - 1) / SPLIT;   // of a part
 
   // The unit to issue next: its term of the sum, its position, its buffers. Past the last one every lane
   // is out of range (zeros nobody reads), so each unit counts the same loads.
   int is = 0, ip = 0, ibuf = 0, left = p.k;
+  if constexpr (SPLIT > 1) {   // (k > 0)
+    is = part * units / per_term;
+    ip = part * units % per_term;
+    left = is < (SUM ? p.orders : 1) ? p.k - ip * UNIT * BK : 0;
+#pragma unroll
+    for (int s = 0; s < SA; ++s) va[s] += ip * UNIT * step_a;
+#pragma unroll
+    for (int s = 0; s < SB; ++s) vb[s] += ip * UNIT * step_b;
+  }
   BufferRsrc ra, rb;
   auto point = [&]() {   // the operands of term is (of order oa, ob)
     const int term = min(is, p.orders - 1);
@@ -221,12 +233,12 @@ void order_gemm_kernel(OrderGemmParams<T> p) {
   auto issue_segment = [&](int i) {   // i / UNIT: the segment, A's SA then B's SB; i % UNIT: the chunk
     const int s = i / UNIT, half = i % UNIT;
     if (s < SA) {
-      lds_dma16(&As[ibuf + half][(wave * SA + s) * (1024 / static_cast<int>(sizeof(T)))], ra,
+      lds_dma16(&As[own + ibuf + half][(wave * SA + s) * (1024 / static_cast<int>(sizeof(T)))], ra,
                 ka[s] < left - half * BK ? va[s] : kBufferOutOfRange);
       va[s] += step_a;
     } else {
       const int u = s - SA;
-      lds_dma16(&Bs[ibuf + half][(wave * SB + u) * (1024 / static_cast<int>(sizeof(T)))], rb,
+      lds_dma16(&Bs[own + ibuf + half][(wave * SB + u) * (1024 / static_cast<int>(sizeof(T)))], rb,
                 kb[u] < left - half * BK ? vb[u] : kBufferOutOfRange);
       vb[u] += step_b;
     }
@@ -258,12 +270,12 @@ void order_gemm_kernel(OrderGemmParams<T> p) {
   auto read_operand = [&](int buf, int set, int i) {   // operand i of a chunk: B's FN, then A's FM
     if (i < FN) {
       const int at = (wn * FN + i) * Blk::S;
-      if constexpr (B_COLS) fb[set][i] = Blk::template read_cols<BN>(Bs[buf], at, lane);
-      else fb[set][i] = Blk::read_rows(Bs[buf], at, lane);
+      if constexpr (B_COLS) fb[set][i] = Blk::template read_cols<BN>(Bs[own + buf], at, lane);
+      else fb[set][i] = Blk::read_rows(Bs[own + buf], at, lane);
     } else {
       const int at = (wm * FM + i - FN) * Blk::S;
-      if constexpr (A_COLS) fa[set][i - FN] = Blk::template read_cols<BM>(As[buf], at, lane);
-      else fa[set][i - FN] = Blk::read_rows(As[buf], at, lane);
+      if constexpr (A_COLS) fa[set][i - FN] = Blk::template read_cols<BM>(As[own + buf], at, lane);
+      else fa[set][i - FN] = Blk::read_rows(As[own + buf], at, lane);
     }
   };
   auto multiply_row = [&](int set, int fm) {
@@ -320,6 +332,22 @@ void order_gemm_kernel(OrderGemmParams<T> p) {
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // no DMA outlives the workgroup's LDS
 
+  if constexpr (SPLIT == 2) {   // the second part's sums go to the first through LDS (every wave is done with its tiles)
+    static_assert(Blk::ACC == 4 && FM * FN * Tile::kThreads * 16 <= sizeof(As), "sums fit A's buffers");
+    const int at = threadIdx.x % Tile::kThreads;
+    __syncthreads();
+    if (part == 1) {
+#pragma unroll
+      for (int i = 0; i < FM * FN; ++i)
+        reinterpret_cast<floatx4*>(&As[0][0])[i * Tile::kThreads + at] = acc[i / FN][i % FN];
+    }
+    __syncthreads();
+    if (part == 1) return;
+#pragma unroll
+    for (int i = 0; i < FM * FN; ++i)
+      acc[i / FN][i % FN] += reinterpret_cast<const floatx4*>(&As[0][0])[i * Tile::kThreads + at];
+  }
+
   // ---- epilogue: a lane's registers are runs of four columns of one row of C ----
   T* base = p.c.p[order] + batch * p.c_bs;
   const bool add = p.bias != nullptr && order == 0;
@@ -366,14 +394,14 @@ static bool order_gemm_takes(const CauchyArgs& a) {
   return ok;
 }
 
-template <typename T, int WMW, int WNW, int FM, int FN, bool A_COLS, bool B_COLS, bool SUM>
+template <typename T, int WMW, int WNW, int FM, int FN, bool A_COLS, bool B_COLS, bool SUM, int SPLIT = 1>
 static int launch_order_tile(OrderGemmParams<T> p, int64_t batch, hipStream_t stream) {
   using Tile = OrderTile<T, WMW, WNW, FM, FN>;
   p.tiles_m = (p.m + Tile::BM - 1) / Tile::BM;
   p.tiles_n = (p.n + Tile::BN - 1) / Tile::BN;
   const int64_t tiles = static_cast<int64_t>(p.tiles_m) * p.tiles_n * (SUM ? 1 : p.orders) * batch;
-  order_gemm_kernel<T, WMW, WNW, FM, FN, A_COLS, B_COLS, SUM, 2>
-      <<<dim3(static_cast<unsigned>(tiles)), dim3(Tile::kThreads), 0, stream>>>(p);
+  order_gemm_kernel<T, WMW, WNW, FM, FN, A_COLS, B_COLS, SUM, SPLIT, 2>
+      <<<dim3(static_cast<unsigned>(tiles)), dim3(SPLIT * Tile::kThreads), 0, stream>>>(p);
   PT_LAUNCH_CHECK();
   return PT_OK;
 }
@@ -382,7 +410,10 @@ static int launch_order_tile(OrderGemmParams<T> p, int64_t batch, hipStream_t st
 // * Halves: 256 x 256 (one workgroup of 8 waves a CU) takes 0.80 us a chunk with every CU busy, and
 //   128 x 128 (up to two workgroups of 4 waves a CU) 0.49 us with two and 0.34 with one (from 8192^3
 //   at 820 and 1007 us, and 512 chunks of 256 small tiles at 176 us): four small tiles cost 1.2
-//   times a large one where both fill the chip, less where the large ones leave CUs idle.
+//   times a large one where both fill the chip, less where the large ones leave CUs idle. Up to 256
+//   small tiles, one a CU, run as workgroups of 8 waves, each half of which takes half of the contraction:
+//   the chunks of both then arrive at the rate of two tiles a CU. From 8 chunks a half, below which the
+//   sums' way through LDS is not paid for (weight gradients of 4096 rows, 1024 x 4096, degree 3: 190 -> 151 us).
 // * Floats: 128 x 128, 128 x 64 and 64 x 64 (two, three and five workgroups a CU); MFMA-bound, so the
 //   busiest CU's tiles count, at 137, 133 and 128 TFLOP/s (8192 x 768 x 3072, degree 3).
 template <typename T, bool A_COLS, bool B_COLS, bool SUM>
@@ -394,6 +425,8 @@ static int launch_order_gemm(const OrderGemmParams<T>& p, int64_t batch, hipStre
     const int64_t large = tiles(256, 256), small = tiles(128, 128), rest = small % 512;
     const double t_large = 0.80 * static_cast<double>((large + 255) / 256);
     const double t_small = 0.49 * static_cast<double>(small / 512) + (rest == 0 ? 0.0 : rest <= 256 ? 0.34 : 0.49);
+    const int64_t chunks = (p.k + 31) / 32 * (SUM ? p.orders : 1);
+    if (small <= 256 && chunks >= 16) return launch_order_tile<T, 2, 2, 4, 4, A_COLS, B_COLS, SUM, 2>(p, batch, stream);
     if (t_large < t_small) return launch_order_tile<T, 2, 4, 8, 4, A_COLS, B_COLS, SUM>(p, batch, stream);
     return launch_order_tile<T, 2, 2, 4, 4, A_COLS, B_COLS, SUM>(p, batch, stream);
   } else {

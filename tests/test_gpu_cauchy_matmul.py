@@ -281,3 +281,25 @@ def test_float_rows_padded_by_size(m, n, k, plain):
     want = [c @ up(B)[0] for c in up(A)] if plain else oracle.matmul(up(A), up(B))
     for o in range(degree + 1):
         assert (got.coeffs[o].cpu().double() - want[o]).abs().max() <= tol * want[o].abs().max(), o
+
+
+# 16-bit products of few tiles, whose workgroups split the contraction in two: below and from 16 chunks of 32,
+# an odd number of them, halves that end inside a term of a sum, ragged sides. Sums in float32, rounded once.
+@pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -10)])
+@pytest.mark.parametrize("m,n,k,terms", [(1, 8, 480, 1), (3, 130, 512, 1), (130, 65, 520, 2), (257, 129, 1001, 3),
+                                         (64, 264, 168, 3), (128, 128, 33, 9), (40, 40, 2056, 4)])
+def test_split_contraction(dtype, tol, m, n, k, terms):
+    g = torch.Generator().manual_seed(k)
+    draw = lambda *shape: (torch.randn(*shape, generator=g, dtype=torch.float64)).to(dtype)   # noqa: E731
+    A, B = [draw(1, m, k) for _ in range(terms)], [draw(1, k, n) for _ in range(terms)]
+    cu = lambda xs: [x.cuda() for x in xs]   # noqa: E731
+    flip = lambda xs: [x.transpose(1, 2).contiguous() for x in xs]   # noqa: E731
+    want = sum(a.double() @ b.double() for a, b in zip(A, B))
+    for a, b, ta, tb in ((A, B, False, False), (A, flip(B), False, True), (flip(A), B, True, False)):
+        got = _ops.matmul_order_sum(cu(a), cu(b), ta, tb).cpu().double()
+        assert (got - want).abs().max() <= tol * want.abs().max(), (ta, tb)
+    for trans_b in (False, True):
+        got = _ops.cauchy_matmul(cu(A), cu(flip(B[:1]) if trans_b else B[:1]), terms - 1, trans_b).cpu().double()
+        for o in range(terms):
+            want_o = A[o].double() @ B[0].double()
+            assert (got[o] - want_o).abs().max() <= tol * want_o.abs().max(), (o, trans_b)
