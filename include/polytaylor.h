@@ -235,7 +235,7 @@ int pt_cauchy_matmul(int dtype, int degree, const void* const* a, int a_orders,
 
 /*
  * pt_cauchy_matmul of operands with row strides: rows of a lda elements apart, of b ldb (both at
- * least the row length). Where lda (ldb) is a multiple of a 16-byte vector and the rows of a (of b
+ * least the row length and at most 2^31 - 1, else PT_UNSUPPORTED). Where lda (ldb) is a multiple of a 16-byte vector and the rows of a (of b
  * if trans_b) run along k, the values from k to the next multiple of a vector must be zero; b's
  * values past n (not trans_b) take no part. So 16-bit operands of any k and n run with padded rows
  * (pt_pack_rows): here the 16-bit kernels need lda and ldb, not k and n, to be multiples of 8.

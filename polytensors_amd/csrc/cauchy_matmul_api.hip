@@ -95,6 +95,8 @@ int pt_cauchy_matmul_strided(int dtype, int degree, const void* const* a, int a_
              "Cauchy matmul: negative batch stride");
   PT_REQUIRE(lda >= k && ldb >= (trans_b ? k : n), PT_INVALID_ARGUMENT,
              "Cauchy matmul: a row stride below the row length");
+  PT_REQUIRE(lda <= INT32_MAX && ldb <= INT32_MAX, PT_UNSUPPORTED,
+             "Cauchy matmul: a row stride beyond 2^31 - 1 elements");   // (the kernels take 32-bit strides)
   PT_REQUIRE(m <= INT32_MAX && n <= INT32_MAX && k <= INT32_MAX && batch <= 65535 &&
                  (m + 31) / 32 <= 65535,
              PT_UNSUPPORTED, "Cauchy matmul: sizes beyond the launch grid");

@@ -57,6 +57,11 @@ def _vpp(n):
     ("pt_stream_copy", lambda: ((1 << 20) + 4, 1 << 21, 32, 0, 1, None), 1, "aligned"),
     ("pt_stream_read", lambda: (1 << 20, 32, 70000, 1, 1 << 21, None), 1, "blocks"),
     ("pt_stream_read", lambda: (1 << 20, 32, 0, 0, None, None), 1, "out"),
+    # row strides beyond the kernels' 32 bits (float32 and float64 have a kernel for any smaller one)
+    *[("pt_cauchy_matmul_strided",
+       lambda dtype=dtype, lda=lda, ldb=ldb: (dtype, 1, _vpp(2), 2, _vpp(1), 1, _vpp(2), 1, 4, 8, 8, lda, ldb, 0, 0, 0, None,
+                                              None), 2, "row stride")
+      for dtype in (0, 1) for lda, ldb in ((1 << 31, 8), (1 << 32, 8), (8, 1 << 32), ((1 << 32) + 8, 8))],
     # attention masks: a map of heads to masks, additive masks, mask sets
     ("pt_taylor_attention_fwd_ws", lambda: (0, 1, _vpp(2), 2, _vpp(2), 2, _vpp(2), 2, _vpp(2), None, 1, 16, 16, 64,
                                             0, 1 << 20, None, None, (ctypes.c_int64 * 3)(0, 0, 0), 0.125, None, 0,
