@@ -37,6 +37,7 @@
 #pragma once
 
 #include <algorithm>
+#include <type_traits>
 
 #include "cauchy_matmul.h"
 #include "half_mfma.h"
@@ -203,20 +204,26 @@ __global__ __launch_bounds__((CauchyHalfTile<AO, BO, WIDE>::kThreads)) void cauc
   __builtin_amdgcn_s_waitcnt(0);
 
   // ---- epilogue: lane (c, g) holds C[m0 + c][n0 + 4g .. + 3] of each block ----
-#pragma unroll
-  for (int o = 0; o <= K; ++o) {
+  const int row0 = tile_m + FM * 16 * wm + c, col0 = tile_n + FN * 16 * wn + 4 * g;
+  auto store = [&](int o, auto biased) __attribute__((always_inline)) {
     T* base = C.p[o] + batch * static_cast<int64_t>(M) * N;
+    float add[FN][4];
+    if constexpr (decltype(biased)::value) {   // before the stores: between them the loads would wait for the ones issued
+#pragma unroll
+      for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) add[fn][e] = col0 + 16 * fn + e < N ? to_acc(bias[col0 + 16 * fn + e]) : 0.f;
+    }
 #pragma unroll
     for (int fm = 0; fm < FM; ++fm)
 #pragma unroll
       for (int fn = 0; fn < FN; ++fn) {
-        const int row = tile_m + FM * 16 * wm + 16 * fm + c;
-        const int col = tile_n + FN * 16 * wn + 16 * fn + 4 * g;
+        const int row = row0 + 16 * fm, col = col0 + 16 * fn;
         if (row >= M) continue;
         floatx4 v = acc[o][fm][fn];
-        if (o == 0 && bias != nullptr) {
+        if constexpr (decltype(biased)::value) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] += col + e < N ? to_acc(bias[col + e]) : 0.f;
+          for (int e = 0; e < 4; ++e) v[e] += add[fn][e];
         }
         T* p = base + static_cast<int64_t>(row) * N + col;
         const uint32_t w01 = MM::pack2(v[0], v[1]), w23 = MM::pack2(v[2], v[3]);
@@ -231,7 +238,11 @@ __global__ __launch_bounds__((CauchyHalfTile<AO, BO, WIDE>::kThreads)) void cauc
           if (col + 3 < N) q[3] = static_cast<uint16_t>(w23 >> 16);
         }
       }
-  }
+  };
+  if (bias != nullptr) store(0, std::true_type{});
+  else store(0, std::false_type{});
+#pragma unroll
+  for (int o = 1; o <= K; ++o) store(o, std::false_type{});
 }
 
 // Zero orders 1..degree of C (both operands ordinary: only C_0 is a product).

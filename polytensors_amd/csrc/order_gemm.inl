@@ -30,6 +30,7 @@
 #pragma once
 
 #include <algorithm>
+#include <type_traits>
 
 #include "cauchy_matmul.h"
 #include "half_mfma.h"
@@ -350,36 +351,50 @@ void order_gemm_kernel(OrderGemmParams<T> p) {
 
   // ---- epilogue: a lane's registers are runs of four columns of one row of C ----
   T* base = p.c.p[order] + batch * p.c_bs;
-  const bool add = p.bias != nullptr && order == 0;
+  const int row0 = tile_m + wm * FM * Blk::S + lane % Blk::S;
+  const int col0 = tile_n + wn * FN * Blk::S + 4 * (lane / Blk::S);   // of block 0 and its registers 0..3
+  auto store = [&](auto biased) __attribute__((always_inline)) {
+    float add[FN][Blk::ACC];
+    if constexpr (decltype(biased)::value) {   // before the stores: between them the loads would wait for the ones issued
 #pragma unroll
-  for (int fm = 0; fm < FM; ++fm) {
-    const int row = tile_m + (wm * FM + fm) * Blk::S + lane % Blk::S;
-    if (row >= p.m) continue;
+      for (int fn = 0; fn < FN; ++fn)
 #pragma unroll
-    for (int fn = 0; fn < FN; ++fn)
-#pragma unroll
-      for (int q = 0; q < Blk::ACC / 4; ++q) {
-        const int col = tile_n + (wn * FN + fn) * Blk::S + 8 * q + 4 * (lane / Blk::S);
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = acc[fm][fn][4 * q + e];
-        if (add) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] += col + e < p.n ? to_acc(p.bias[col + e]) : 0.f;
+        for (int i = 0; i < Blk::ACC; ++i) {
+          const int col = col0 + fn * Blk::S + 8 * (i / 4) + i % 4;
+          add[fn][i] = col < p.n ? to_acc(p.bias[col]) : 0.f;
         }
-        T* dst = base + static_cast<int64_t>(row) * p.n + col;
-        if (col + 3 < p.n) {
-          Vec<T, 4> w;
+    }
 #pragma unroll
-          for (int e = 0; e < 4; e += 2) vec_put2(w, e, v[e], v[e + 1]);
-          __builtin_memcpy(dst, &w, sizeof(w));   // at any element: one 8- or 16-byte store
-        } else {
+    for (int fm = 0; fm < FM; ++fm) {
+      const int row = row0 + fm * Blk::S;
+      if (row >= p.m) continue;
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (col + e < p.n) dst[e] = from_acc<T>(v[e]);
+      for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+        for (int q = 0; q < Blk::ACC / 4; ++q) {
+          const int col = col0 + fn * Blk::S + 8 * q;
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            v[e] = acc[fm][fn][4 * q + e];
+            if constexpr (decltype(biased)::value) v[e] += add[fn][4 * q + e];
+          }
+          T* dst = base + static_cast<int64_t>(row) * p.n + col;
+          if (col + 3 < p.n) {
+            Vec<T, 4> w;
+#pragma unroll
+            for (int e = 0; e < 4; e += 2) vec_put2(w, e, v[e], v[e + 1]);
+            __builtin_memcpy(dst, &w, sizeof(w));   // at any element: one 8- or 16-byte store
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (col + e < p.n) dst[e] = from_acc<T>(v[e]);
+          }
         }
-      }
-  }
+    }
+  };
+  if (p.bias != nullptr && order == 0) store(std::true_type{});
+  else store(std::false_type{});
 }
 
 // Whether the DMA can read the operands: whole, aligned 16-byte vectors along rows, 32-bit offsets.
