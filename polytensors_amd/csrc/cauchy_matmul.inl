@@ -70,12 +70,26 @@ struct CauchyLds {
   }
 };
 
+// What a product with row strides or a bias takes besides; nothing where rows are as long as the matrices
+// and there is no bias (PLAIN).
+template <typename T, bool PLAIN>
+struct CauchyRows {
+  int lda, ldb;
+  const T* bias;
+};
+template <typename T>
+struct CauchyRows<T, true> {};
+
 template <typename T, int K, int AO, int BO, int BM, int BN, int BK, int WAVES_M, int WAVES_N,
-          int MIN_WAVES, bool TRANS_B, bool VEC>
+          int MIN_WAVES, bool TRANS_B, bool VEC, bool PLAIN>
 __global__ __launch_bounds__(WAVES_M * WAVES_N * kWave) __attribute__((amdgpu_waves_per_eu(MIN_WAVES)))
 void cauchy_matmul_kernel(
-    CPtrs<T> A, CPtrs<T> B, MPtrs<T> C, int M, int N, int Kd, int lda, int ldb, int64_t a_bs, int64_t b_bs,
-    const T* __restrict__ bias) {
+    CPtrs<T> A, CPtrs<T> B, MPtrs<T> C, int M, int N, int Kd, int64_t a_bs, int64_t b_bs, CauchyRows<T, PLAIN> rows) {
+  int lda = Kd, ldb = TRANS_B ? Kd : N;
+  if constexpr (!PLAIN) {
+    lda = rows.lda;
+    ldb = rows.ldb;
+  }
   using MF = Mfma<T>;
   using acc_t = typename MF::acc_t;
   constexpr int THREADS = WAVES_M * WAVES_N * kWave;
@@ -250,33 +264,24 @@ void cauchy_matmul_kernel(
   }
 
   // ---- epilogue: each accumulator register holds one element of C_k ----
-  const int row0 = tile_m + wm * WM, col0 = tile_n + wn * WN + MF::acc_col(lane);
-  // (a path of its own for a bias: its loads and sums between the stores cost a product without one 5-12%
-  // where the contraction is short; 100001 x 33 x 65 float64, degree 3: 140 us, 156 with them)
-  auto store = [&](int o, auto biased) __attribute__((always_inline)) {
+#pragma unroll
+  for (int o = 0; o <= K; ++o) {
     T* c_base = C.p[o] + batch * static_cast<int64_t>(M) * N;
 #pragma unroll
     for (int fm = 0; fm < FM; ++fm)
 #pragma unroll
       for (int fn = 0; fn < FN; ++fn) {
-        const int col = col0 + fn * MF::N;
+        const int col = tile_n + wn * WN + fn * MF::N + MF::acc_col(lane);
         T add = T(0);
-        if constexpr (decltype(biased)::value) add = col < N ? bias[col] : T(0);
+        if constexpr (!PLAIN) add = o == 0 && rows.bias != nullptr && col < N ? rows.bias[col] : T(0);
 #pragma unroll
         for (int r = 0; r < MF::ACC; ++r) {
-          const int row = row0 + fm * MF::M + MF::acc_row(lane, r);
-          if (row < M && col < N) {
-            T v = acc[o][fm][fn][r];
-            if constexpr (decltype(biased)::value) v += add;
-            c_base[static_cast<int64_t>(row) * N + col] = v;
-          }
+          const int row = tile_m + wm * WM + fm * MF::M + MF::acc_row(lane, r);
+          if (row < M && col < N)
+            c_base[static_cast<int64_t>(row) * N + col] = !PLAIN && o == 0 ? acc[o][fm][fn][r] + add : acc[o][fm][fn][r];
         }
       }
-  };
-  if (bias != nullptr) store(0, std::true_type{});
-  else store(0, std::false_type{});
-#pragma unroll
-  for (int o = 1; o <= K; ++o) store(o, std::false_type{});
+  }
 }
 
 // Zero orders 1..degree of C (both operands ordinary: only C_0 is a product).
@@ -317,18 +322,26 @@ static int launch_cauchy_orders(const CauchyArgs& a, const CPtrs<T>& A, const CP
   const dim3 grid((a.n + Tile::BN - 1) / Tile::BN, (a.m + Tile::BM - 1) / Tile::BM, a.batch);
   const dim3 block(Tile::WAVES_M * Tile::WAVES_N * kWave);
   const int M = static_cast<int>(a.m), N = static_cast<int>(a.n), Kd = static_cast<int>(a.k);
-  const int lda = static_cast<int>(a.lda), ldb = static_cast<int>(a.ldb);
-#define PT_CAUCHY_LAUNCH(TB, VV)                                                                   \
+  // Rows as long as the matrices and no bias: an instance of its own. In the other, a bias's loads stand between
+  // the stores: 2048 x 32 x 32 x 32 float64 at degree 3 takes 49 us in this one and 55 in that.
+  const bool plain = a.bias == nullptr && a.lda == a.k && a.ldb == a.width_b();
+#define PT_CAUCHY_LAUNCH(TB, VV, PL)                                                               \
   cauchy_matmul_kernel<T, K, AO, BO, Tile::BM, Tile::BN, Tile::BK, Tile::WAVES_M, Tile::WAVES_N, \
-                       Tile::MIN_WAVES, TB, VV><<<grid, block, 0, a.stream>>>(A, B, C, M, N, Kd, lda, ldb, a.a_bs, a.b_bs, \
-                                                static_cast<const T*>(a.bias))
-  if (a.trans_b) {
-    if (vec) PT_CAUCHY_LAUNCH(true, true);
-    else PT_CAUCHY_LAUNCH(true, false);
-  } else {
-    if (vec) PT_CAUCHY_LAUNCH(false, true);
-    else PT_CAUCHY_LAUNCH(false, false);
-  }
+                       Tile::MIN_WAVES, TB, VV, PL><<<grid, block, 0, a.stream>>>(A, B, C, M, N, Kd, a.a_bs, a.b_bs, rows)
+  auto launch = [&](auto plain_tag) {
+    constexpr bool PL = decltype(plain_tag)::value;
+    CauchyRows<T, PL> rows{};
+    if constexpr (!PL) rows = {static_cast<int>(a.lda), static_cast<int>(a.ldb), static_cast<const T*>(a.bias)};
+    if (a.trans_b) {
+      if (vec) PT_CAUCHY_LAUNCH(true, true, PL);
+      else PT_CAUCHY_LAUNCH(true, false, PL);
+    } else {
+      if (vec) PT_CAUCHY_LAUNCH(false, true, PL);
+      else PT_CAUCHY_LAUNCH(false, false, PL);
+    }
+  };
+  if (plain) launch(std::true_type{});
+  else launch(std::false_type{});
 #undef PT_CAUCHY_LAUNCH
   PT_LAUNCH_CHECK();
   return PT_OK;
@@ -362,7 +375,7 @@ static int launch_cauchy_k(const CauchyArgs& a) {
   if constexpr (sizeof(T) == 4) {
     // float32 with an ordinary operand: order by order, where the DMA can read the operands (the
     // kernel below reads any row length and alignment, at 114 against 137 TFLOP/s: order_gemm.inl)
-    if (!(a_series && b_series) && order_gemm_takes<T>(a)) {
+    if (!(a_series && b_series) && order_gemm_takes<T>(a) && order_gemm_pays<T>(a)) {
       const int orders = std::max(a.a_orders, a.b_orders), st = launch_by_order<T>(a, orders);
       return orders == K + 1 ? st : zero_higher(st);
     }

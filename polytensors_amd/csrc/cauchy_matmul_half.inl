@@ -45,7 +45,8 @@
 
 namespace pt {
 
-// Both operands are series (an ordinary one: order_gemm.inl).
+// Both operands are series, or one is ordinary (AO or BO is 1) and its product is too small, or its
+// contraction too short, for the kernel that runs order by order (order_gemm_pays, order_gemm.inl).
 //
 // Workgroup tile: WMW x WNW waves, each owning FM x FN MFMA blocks of 16 x 16 of every C_k. The
 // narrow tile (64 x 64, 4 waves of 32 x 32) leaves LDS for two workgroups per CU; the wide tile
@@ -277,14 +278,24 @@ static int launch_cauchy_half_tile(const CauchyArgs& a, const CPtrs<T>& A, const
 // operands within 256 (K <= 4), and its rounds over the chip take less time: a round of up to 256
 // wide tiles (one a CU) takes 1.56 times one of up to 512 narrow ones (two a CU; 0.60 with one), from
 // 4096^3 at degree 4: 4 rounds of wide tiles 1.367 ms, 8 of narrow ones 1.750 ms.
-template <typename T, int K, int AO, int BO>
+template <typename T, int K>
 static int launch_cauchy_half_orders(const CauchyArgs& a, const CPtrs<T>& A, const CPtrs<T>& B, const MPtrs<T>& C) {
-  if constexpr (K <= 4 && CauchyHalfTile<AO, BO, true>::LDS <= 160 * 1024) {
+  if constexpr (K <= 4) {
     auto tiles = [&](int64_t side) { return (a.m + side - 1) / side * ((a.n + side - 1) / side) * a.batch; };
     const int64_t rest = tiles(64) % 512;
     const double wide = 1.56 * static_cast<double>((tiles(128) + 255) / 256);
     const double narrow = static_cast<double>(tiles(64) / 512) + (rest == 0 ? 0.0 : rest <= 256 ? 0.6 : 1.0);
-    if (wide < narrow) return launch_cauchy_half_tile<T, K, AO, BO, true>(a, A, B, C);
+    if (wide < narrow) return launch_cauchy_half_tile<T, K, K + 1, K + 1, true>(a, A, B, C);
+  }
+  return launch_cauchy_half_tile<T, K, K + 1, K + 1, false>(a, A, B, C);
+}
+
+// With an ordinary operand, products that order_gemm.inl does not take: the wide tile where both sides span at
+// least two of its tiles (64 x 4096 x 8 x 520 bfloat16, degree 2: 235 us, 380 in narrow ones).
+template <typename T, int K, int AO, int BO>
+static int launch_cauchy_half_one_series(const CauchyArgs& a, const CPtrs<T>& A, const CPtrs<T>& B, const MPtrs<T>& C) {
+  if constexpr (K <= 4) {
+    if (a.m >= 256 && a.n >= 256) return launch_cauchy_half_tile<T, K, AO, BO, true>(a, A, B, C);
   }
   return launch_cauchy_half_tile<T, K, AO, BO, false>(a, A, B, C);
 }
@@ -296,15 +307,40 @@ static int launch_cauchy_half_k(const CauchyArgs& a) {
   for (int o = 0; o < a.a_orders; ++o) A.p[o] = static_cast<const T*>(a.a[o]);
   for (int o = 0; o < a.b_orders; ++o) B.p[o] = static_cast<const T*>(a.b[o]);
   for (int o = 0; o <= K; ++o) C.p[o] = static_cast<T*>(a.c[o]);
-  return launch_cauchy_half_orders<T, K, K + 1, K + 1>(a, A, B, C);
+  if constexpr (K == 0) {
+    return launch_cauchy_half_tile<T, 0, 1, 1, false>(a, A, B, C);
+  } else {
+    if (a.b_orders == 1) return launch_cauchy_half_one_series<T, K, K + 1, 1>(a, A, B, C);
+    if (a.a_orders == 1) return launch_cauchy_half_one_series<T, K, 1, K + 1>(a, A, B, C);
+    return launch_cauchy_half_orders<T, K>(a, A, B, C);
+  }
 }
 
-// A product with an ordinary operand: every order by itself; two ordinary operands give order 0,
-// and zero higher orders.
+template <typename T>
+static int launch_cauchy_half_degree(const CauchyArgs& a, int degree) {
+  switch (degree) {
+    case 0: return launch_cauchy_half_k<T, 0>(a);
+    case 1: return launch_cauchy_half_k<T, 1>(a);
+    case 2: return launch_cauchy_half_k<T, 2>(a);
+    case 3: return launch_cauchy_half_k<T, 3>(a);
+    case 4: return launch_cauchy_half_k<T, 4>(a);
+    case 5: return launch_cauchy_half_k<T, 5>(a);
+    case 6: return launch_cauchy_half_k<T, 6>(a);
+    case 7: return launch_cauchy_half_k<T, 7>(a);
+    case 8: return launch_cauchy_half_k<T, 8>(a);
+    default: break;
+  }
+  pt_host::set_error("Cauchy matmul: degree outside 0..PT_MAX_DEGREE");
+  return PT_UNSUPPORTED;
+}
+
+// A product with an ordinary operand: order by order, or by this file's kernel (order_gemm_pays); two
+// ordinary operands give order 0, and zero higher orders.
 template <typename T>
 static int launch_cauchy_half_ordinary(const CauchyArgs& a) {
   const int orders = std::max(a.a_orders, a.b_orders);
-  const int st = launch_by_order<T>(a, orders);
+  const int st = order_gemm_takes<T>(a) && order_gemm_pays<T>(a) ? launch_by_order<T>(a, orders)
+                                                                 : launch_cauchy_half_degree<T>(a, orders - 1);
   if (st != PT_OK || orders > a.degree) return st;
   MPtrs<T> C{};
   for (int o = 0; o <= a.degree; ++o) C.p[o] = static_cast<T*>(a.c[o]);
@@ -330,26 +366,7 @@ int launch_cauchy_half(const CauchyArgs& a) {
         "to be multiples of 8, 16-byte aligned operands, and each matrix below 1 GiB");
     return PT_UNSUPPORTED;
   }
-  if (a.a_orders == 1 || a.b_orders == 1) {
-    if (!order_gemm_takes<T>(a)) {
-      pt_host::set_error("Cauchy matmul (16-bit): more output tiles than a launch holds");
-      return PT_UNSUPPORTED;
-    }
-    return launch_cauchy_half_ordinary<T>(a);
-  }
-  switch (a.degree) {
-    case 1: return launch_cauchy_half_k<T, 1>(a);
-    case 2: return launch_cauchy_half_k<T, 2>(a);
-    case 3: return launch_cauchy_half_k<T, 3>(a);
-    case 4: return launch_cauchy_half_k<T, 4>(a);
-    case 5: return launch_cauchy_half_k<T, 5>(a);
-    case 6: return launch_cauchy_half_k<T, 6>(a);
-    case 7: return launch_cauchy_half_k<T, 7>(a);
-    case 8: return launch_cauchy_half_k<T, 8>(a);
-    default: break;
-  }
-  pt_host::set_error("Cauchy matmul: degree outside 0..PT_MAX_DEGREE");
-  return PT_UNSUPPORTED;
+  return a.a_orders == 1 || a.b_orders == 1 ? launch_cauchy_half_ordinary<T>(a) : launch_cauchy_half_degree<T>(a, a.degree);
 }
 
 }  // namespace pt

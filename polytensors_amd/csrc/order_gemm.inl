@@ -400,13 +400,23 @@ void order_gemm_kernel(OrderGemmParams<T> p) {
   else store(std::false_type{});
 }
 
-// Whether the DMA can read the operands: whole, aligned 16-byte vectors along rows, 32-bit offsets.
+// Whether a launch holds this many tiles for each order and batch entry: every workgroup has 256 threads
+// at least counted so (the larger tiles and the split ones, of 512, are fewer), and a launch has fewer
+// than 2^32 threads along x.
+template <typename T>
+static bool order_gemm_holds(int64_t m, int64_t n, int64_t count) {
+  constexpr int64_t side = sizeof(T) == 2 ? 128 : 64;   // of the smallest tile
+  return static_cast<double>((m + side - 1) / side) * static_cast<double>((n + side - 1) / side) * static_cast<double>(count) <
+         static_cast<double>(1 << 24);
+}
+
+// Whether the kernel can run the product: whole, aligned 16-byte vectors along rows, 32-bit offsets, one launch.
 template <typename T>
 static bool order_gemm_takes(const CauchyArgs& a) {
   constexpr int64_t V = 16 / static_cast<int64_t>(sizeof(T)), kLimit = (int64_t{1} << 30) / static_cast<int64_t>(sizeof(T));
   bool ok = a.lda % V == 0 && a.ldb % V == 0 && a.a_bs % V == 0 && a.b_bs % V == 0 && a.lda < kLimit && a.ldb < kLimit &&
             a.m * a.lda < kLimit && a.rows_b() * a.ldb < kLimit &&
-            ((a.m + 63) / 64) * ((a.n + 63) / 64) * std::max(a.a_orders, a.b_orders) * a.batch <= INT32_MAX;
+            order_gemm_holds<T>(a.m, a.n, std::max(a.a_orders, a.b_orders) * a.batch);
   for (int o = 0; o < a.a_orders; ++o) ok = ok && pt_host::aligned16(a.a[o]);
   for (int o = 0; o < a.b_orders; ++o) ok = ok && pt_host::aligned16(a.b[o]);
   return ok;
@@ -434,27 +444,76 @@ static int launch_order_tile(OrderGemmParams<T> p, int64_t batch, hipStream_t st
 //   sums' way through LDS is not paid for (weight gradients of 4096 rows, 1024 x 4096, degree 3: 190 -> 151 us).
 // * Floats: 128 x 128, 128 x 64 and 64 x 64 (two, three and five workgroups a CU); MFMA-bound, so the
 //   busiest CU's tiles count, at 137, 133 and 128 TFLOP/s (8192 x 768 x 3072, degree 3).
+static inline bool order_large_tiles(int64_t large, int64_t small) {
+  const int64_t rest = small % 512;
+  return 0.80 * static_cast<double>((large + 255) / 256) <
+         0.49 * static_cast<double>(small / 512) + (rest == 0 ? 0.0 : rest <= 256 ? 0.34 : 0.49);
+}
+
+static inline int order_float_tile(const int64_t (&tiles)[3]) {   // 0: 128 x 128, 1: 128 x 64, 2: 64 x 64
+  constexpr double kArea[3] = {128 * 128, 128 * 64, 64 * 64}, kRate[3] = {137, 133, 128};
+  double cost[3];
+  for (int i = 0; i < 3; ++i) cost[i] = static_cast<double>((tiles[i] + 255) / 256) * kArea[i] / kRate[i];
+  return cost[0] <= cost[1] && cost[0] <= cost[2] ? 0 : cost[1] <= cost[2] ? 1 : 2;
+}
+
 template <typename T, bool A_COLS, bool B_COLS, bool SUM>
 static int launch_order_gemm(const OrderGemmParams<T>& p, int64_t batch, hipStream_t stream) {
   auto tiles = [&](int64_t bm, int64_t bn) {
     return (p.m + bm - 1) / bm * ((p.n + bn - 1) / bn) * (SUM ? 1 : p.orders) * batch;
   };
   if constexpr (sizeof(T) == 2) {
-    const int64_t large = tiles(256, 256), small = tiles(128, 128), rest = small % 512;
-    const double t_large = 0.80 * static_cast<double>((large + 255) / 256);
-    const double t_small = 0.49 * static_cast<double>(small / 512) + (rest == 0 ? 0.0 : rest <= 256 ? 0.34 : 0.49);
-    const int64_t chunks = (p.k + 31) / 32 * (SUM ? p.orders : 1);
+    const int64_t small = tiles(128, 128), chunks = (p.k + 31) / 32 * (SUM ? p.orders : 1);
     if (small <= 256 && chunks >= 16) return launch_order_tile<T, 2, 2, 4, 4, A_COLS, B_COLS, SUM, 2>(p, batch, stream);
-    if (t_large < t_small) return launch_order_tile<T, 2, 4, 8, 4, A_COLS, B_COLS, SUM>(p, batch, stream);
+    if (order_large_tiles(tiles(256, 256), small)) return launch_order_tile<T, 2, 4, 8, 4, A_COLS, B_COLS, SUM>(p, batch, stream);
     return launch_order_tile<T, 2, 2, 4, 4, A_COLS, B_COLS, SUM>(p, batch, stream);
   } else {
-    auto cost = [&](int64_t bm, int64_t bn, double rate) {
-      return static_cast<double>((tiles(bm, bn) + 255) / 256 * bm * bn) / rate;
-    };
-    const double c0 = cost(128, 128, 137), c1 = cost(128, 64, 133), c2 = cost(64, 64, 128);
-    if (c0 <= c1 && c0 <= c2) return launch_order_tile<T, 2, 2, 2, 2, A_COLS, B_COLS, SUM>(p, batch, stream);
-    if (c1 <= c2) return launch_order_tile<T, 2, 2, 2, 1, A_COLS, B_COLS, SUM>(p, batch, stream);
-    return launch_order_tile<T, 2, 2, 1, 1, A_COLS, B_COLS, SUM>(p, batch, stream);
+    const int64_t t[3] = {tiles(128, 128), tiles(128, 64), tiles(64, 64)};
+    switch (order_float_tile(t)) {
+      case 0: return launch_order_tile<T, 2, 2, 2, 2, A_COLS, B_COLS, SUM>(p, batch, stream);
+      case 1: return launch_order_tile<T, 2, 2, 2, 1, A_COLS, B_COLS, SUM>(p, batch, stream);
+      default: return launch_order_tile<T, 2, 2, 1, 1, A_COLS, B_COLS, SUM>(p, batch, stream);
+    }
+  }
+}
+
+// Whether the product runs order by order rather than in the kernels with all orders in a workgroup
+// (cauchy_matmul*.inl): those read an ordinary tile once for all orders and have smaller tiles, this one streams a
+// long contraction faster. The estimated times of both in us, each a fixed part and, for every round of
+// workgroups over the chip, one for the stores and one for every 32 (floats: 16) of the contraction; fitted to 1700
+// shapes (sides 1 to 100000, contractions 8 to 4096, 1 to 16384 matrices, degrees 1 to 8), whose times they
+// give to 15-20%. Order by order where it is 15% less: of those shapes 3% then take over 1.08 times the time of the
+// other kernel, where always running order by order 55% do, up to 7 times: 4096 x 16 x 16 x 16 bfloat16, degree 8,
+// 40 us and 202 order by order; 200000 x 8 x 8, 53 and 129; 2048 x 8 x 2048 float32, degree 3, 17 and 30;
+// 768 x 4096 x 256 bfloat16, degree 8, 104 and 40.
+template <typename T>
+static bool order_gemm_pays(const CauchyArgs& a) {
+  const int64_t orders = std::max(a.a_orders, a.b_orders);
+  const double n1 = static_cast<double>(orders);
+  auto tiles = [&](int64_t bm, int64_t bn) { return (a.m + bm - 1) / bm * ((a.n + bn - 1) / bn) * a.batch; };
+  // rounds of `per` workgroups; `half` of one where the last has at most half of them
+  auto rounds = [](int64_t count, int64_t per, double half) {
+    const int64_t rest = count % per;
+    return static_cast<double>(count / per) + (rest == 0 ? 0.0 : 2 * rest <= per ? half : 1.0);
+  };
+  if constexpr (sizeof(T) == 2) {
+    const double chunks = static_cast<double>((a.k + 31) / 32);
+    const double all = orders <= 5 && a.m >= 256 && a.n >= 256
+        ? 2.5 + rounds(tiles(128, 128), 256, 1.0) * (1.95 * n1 + chunks * (0.065 + 0.25 * n1))
+        : 2.5 + rounds(tiles(64, 64), 512, 0.43) * (0.94 * n1 + chunks * (0.16 + 0.17 * n1));
+    const int64_t small = tiles(128, 128) * orders;
+    double each;   // (the tiles as launch_order_gemm picks them)
+    if (small <= 256 && chunks >= 16) each = 5.2 + 0.20 * chunks;
+    else if (order_large_tiles(tiles(256, 256) * orders, small)) each = 4.9 + rounds(tiles(256, 256) * orders, 256, 1.0) * (8.6 + 0.78 * chunks);
+    else each = 4.9 + rounds(small, 512, 0.24) * (4.2 + 0.35 * chunks);
+    return 1.15 * each <= all;
+  } else {
+    const double chunks = static_cast<double>((a.k + 15) / 16);
+    const double all = 2.4 + rounds(tiles(64, 64), 512, 0.52) * (0.93 * n1 + chunks * (0.26 + 0.53 * n1));
+    const int64_t t[3] = {tiles(128, 128) * orders, tiles(128, 64) * orders, tiles(64, 64) * orders};
+    const int pick = order_float_tile(t);
+    constexpr double kStores[3] = {1.21, 1.81, 0.74}, kChunk[3] = {1.59, 0.49, 0.275};
+    return 1.15 * (3.4 + rounds(t[pick], 256, 1.0) * (kStores[pick] + chunks * kChunk[pick])) <= all;
   }
 }
 
@@ -490,11 +549,11 @@ int launch_order_sum(const OrderSumArgs& a) {
   bool ok = a.lda % V == 0 && a.ldb % V == 0 && a.a_bs % V == 0 && a.b_bs % V == 0 &&
             a.m <= INT32_MAX && a.n <= INT32_MAX && a.k <= INT32_MAX &&
             a.lda < kLimit && a.ldb < kLimit && rows_a * a.lda < kLimit && rows_b * a.ldb < kLimit &&
-            ((a.m + 63) / 64) * ((a.n + 63) / 64) * a.batch <= INT32_MAX;
+            order_gemm_holds<T>(a.m, a.n, a.batch);
   for (int s = 0; s < a.terms; ++s) ok = ok && pt_host::aligned16(a.a[s]) && pt_host::aligned16(a.b[s]);
   if (!ok) {
     pt_host::set_error("matmul order sum: needs 16-byte aligned operands, row and batch strides of whole 16-byte "
-                       "vectors, and each matrix below 1 GiB");
+                       "vectors, and each matrix below 1 GiB, and tiles of one launch");
     return PT_UNSUPPORTED;
   }
   OrderGemmParams<T> p{};

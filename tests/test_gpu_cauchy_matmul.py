@@ -303,3 +303,43 @@ def test_split_contraction(dtype, tol, m, n, k, terms):
         for o in range(terms):
             want_o = A[o].double() @ B[0].double()
             assert (got[o] - want_o).abs().max() <= tol * want_o.abs().max(), (o, trans_b)
+
+
+# Products with an ordinary operand on both sides of the rule that sends them order by order: small matrices in
+# batches, short contractions on large sides (the wide 16-bit tiles to degree 4, the narrow ones past it), both
+# operands ordinary, and long contractions at the edges of the order-by-order tiles. Against float64 of the stored
+# inputs, relative to the largest value: one rounding to the storage type, float32 sums of k terms of magnitude one.
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -11 + 1e-5)])
+@pytest.mark.parametrize("m,k,n,batch,degree", [
+    (16, 16, 16, 300, 8), (1, 8, 300, 40, 1), (65, 24, 33, 17, 5), (300, 8, 264, 2, 4), (257, 40, 513, 1, 6),
+    (70, 16, 64, 1, 0), (129, 1000, 264, 1, 3), (200, 4096, 65, 2, 8), (1, 1024, 640, 1, 2), (520, 513, 260, 3, 1)])
+def test_ordinary_operand_routes(dtype, tol, m, k, n, batch, degree):
+    g = torch.Generator().manual_seed(m + k + n)
+    A = [torch.randn(batch, m, k, generator=g).to(dtype) for _ in range(degree + 1)]
+    B = [(torch.randn(batch, k, n, generator=g) / k ** 0.5).to(dtype) for _ in range(degree + 1)]
+    cu = lambda xs: [x.cuda() for x in xs]   # noqa: E731
+    for a, b in ((A, B[:1]), (A[:1], B), (A[:1], B[:1]), (A, [B[0][:1]])):
+        for trans_b in (False, True):
+            got = _ops.cauchy_matmul(cu(a), cu([x.transpose(1, 2).contiguous() for x in b] if trans_b else b), degree, trans_b)
+            for o in range(degree + 1):
+                if o >= max(len(a), len(b)):
+                    assert not got[o].any()
+                    continue
+                want = a[o if len(a) > 1 else 0].double() @ b[o if len(b) > 1 else 0].double()
+                err = (got[o].cpu().double() - want).abs().max() / want.abs().max()
+                assert err <= tol, (len(a), len(b), trans_b, o, err)
+
+
+# More tiles than a launch along one dimension holds (2^32 threads): one row each of 65535 matrices by a shared one.
+@pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 2.0 ** -8), (torch.float32, 1e-5)])
+def test_many_small_matrices(dtype, tol):
+    batch, k, n, degree = 65535, 8, 4096, 8
+    g = torch.Generator(device="cuda").manual_seed(0)
+    A = [torch.randn(batch, 1, k, generator=g, device="cuda").to(dtype) for _ in range(degree + 1)]
+    b = torch.randn(1, k, n, generator=g, device="cuda").to(dtype)
+    got = _ops.cauchy_matmul(A, [b], degree, False)
+    for o in range(degree + 1):
+        for part in (slice(0, 300), slice(30000, 30300), slice(batch - 300, batch)):
+            want = A[o][part, 0].double() @ b[0].double()
+            err = (got[o][part, 0].double() - want).abs().max() / want.abs().max()
+            assert err <= tol, (o, err)
