@@ -76,20 +76,20 @@ template <typename T, bool PLAIN>
 struct CauchyRows {
   int lda, ldb;
   const T* bias;
+  __device__ __forceinline__ int a(int) const { return lda; }
+  __device__ __forceinline__ int b(int) const { return ldb; }
 };
 template <typename T>
-struct CauchyRows<T, true> {};
+struct CauchyRows<T, true> {
+  __device__ __forceinline__ int a(int width) const { return width; }
+  __device__ __forceinline__ int b(int width) const { return width; }
+};
 
 template <typename T, int K, int AO, int BO, int BM, int BN, int BK, int WAVES_M, int WAVES_N,
           int MIN_WAVES, bool TRANS_B, bool VEC, bool PLAIN>
 __global__ __launch_bounds__(WAVES_M * WAVES_N * kWave) __attribute__((amdgpu_waves_per_eu(MIN_WAVES)))
 void cauchy_matmul_kernel(
     CPtrs<T> A, CPtrs<T> B, MPtrs<T> C, int M, int N, int Kd, int64_t a_bs, int64_t b_bs, CauchyRows<T, PLAIN> rows) {
-  int lda = Kd, ldb = TRANS_B ? Kd : N;
-  if constexpr (!PLAIN) {
-    lda = rows.lda;
-    ldb = rows.ldb;
-  }
   using MF = Mfma<T>;
   using acc_t = typename MF::acc_t;
   constexpr int THREADS = WAVES_M * WAVES_N * kWave;
@@ -134,7 +134,7 @@ void cauchy_matmul_kernel(
       for (int it = 0; it < NA; ++it) {
         const int v = it * THREADS + threadIdx.x;
         const int gr = tile_m + v / (BK / V), gk = k0 + (v % (BK / V)) * V;
-        const T* p = a_base[o] + static_cast<int64_t>(gr) * lda + gk;
+        const T* p = a_base[o] + static_cast<int64_t>(gr) * rows.a(Kd) + gk;
         if constexpr (VEC) {   // a vector that starts inside is whole: lda % V == 0, zeros past Kd
           if (gr < M && gk < Kd) {
             ra[o][it] = load_vec<T, V>(p);
@@ -154,7 +154,7 @@ void cauchy_matmul_kernel(
         const int v = it * THREADS + threadIdx.x;
         if constexpr (TRANS_B) {   // B stored [N][Kd]
           const int gn = tile_n + v / (BK / V), gk = k0 + (v % (BK / V)) * V;
-          const T* p = b_base[o] + static_cast<int64_t>(gn) * ldb + gk;
+          const T* p = b_base[o] + static_cast<int64_t>(gn) * rows.b(Kd) + gk;
           if constexpr (VEC) {
             if (gn < N && gk < Kd) {
               rb[o][it] = load_vec<T, V>(p);
@@ -168,7 +168,7 @@ void cauchy_matmul_kernel(
           }
         } else {                   // B stored [Kd][N]: a vector runs along n
           const int gk = k0 + v / (BN / V), gn = tile_n + (v % (BN / V)) * V;
-          const T* p = b_base[o] + static_cast<int64_t>(gk) * ldb + gn;
+          const T* p = b_base[o] + static_cast<int64_t>(gk) * rows.b(N) + gn;
           if constexpr (VEC) {     // ldb % V == 0 (columns past N are not stored)
             if (gk < Kd && gn < N) {
               rb[o][it] = load_vec<T, V>(p);
