@@ -271,40 +271,41 @@ Tensor cross_entropy_series_backward(const TensorList& z, const Tensor& target, 
 
 // ---- Cauchy-product matmul ---------------------------------------------------
 
-// Matrices as the 16-byte loads of the matmul kernels take them: rows `stride` elements apart.
+// Whether contiguous [batch, rows, cols] matrices have rows of whole 16-byte vectors, at 16-byte aligned places.
+bool whole_rows(const TensorList& in) {
+  const Tensor& first = in[0];
+  bool whole = first.size(2) * static_cast<int64_t>(first.element_size()) % 16 == 0;
+  for (const Tensor& t : in) whole = whole && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  return whole;
+}
+
+// Matrices as a matmul kernel takes them: pointers to the operand's, or to copies of them, and the distance of
+// their rows in elements.
 struct Rows {
-  TensorList matrices;
+  std::vector<const void*> ptrs;
   int64_t stride;
+  Tensor copies;
 };
 
-// Contiguous [batch, rows, cols] matrices with aligned rows: as they are, or, where a row is no whole
-// number of 16-byte vectors or a matrix is not aligned, copied with rows padded by zeros (all orders in
-// one launch). The 16-bit kernels read nothing else; float32 gains by it (4 x 511 x 1023 x 769, degree 4:
-// 704 -> 519 us; 300 x 301 x 1001 by an ordinary matrix, degree 3: 44 -> 26); float64, bound by its
-// MFMAs, does not (1006 -> 973 us there, 57 -> 61 here), and is left to the kernel's element loads.
+Rows own_rows(const TensorList& in) { return {cptrs(in), in[0].size(2), {}}; }
+
+// Copies with rows padded by zeros to whole 16-byte vectors (all orders in one launch).
 // Rows of 512 bytes and more are padded to whole 128-byte cache lines: a tile's row segments of 64 to
 // 256 bytes otherwise straddle lines (4 x 511 x 1023 x 769 bfloat16, degree 4: 85 -> 77 us).
-Rows packed_rows(const TensorList& in, bool elements = false) {   // elements: any rows do, nothing is copied
+Rows packed_rows(const TensorList& in) {
   const Tensor& first = in[0];
-  const int64_t cols = first.size(2), rows = first.size(0) * first.size(1);
-  const int64_t vec = 16 / static_cast<int64_t>(first.element_size());
-  bool whole = cols % vec == 0;
-  for (const Tensor& t : in) whole = whole && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
-  whole = whole || elements;
-  if (whole) return {in, cols};
+  const int64_t cols = first.size(2), rows = first.size(0) * first.size(1), elem = static_cast<int64_t>(first.element_size());
+  const int64_t vec = 16 / elem;
   auto padded = [&](int64_t unit) { return (cols + unit - 1) / unit * unit; };
   int64_t stride = padded(vec);
-  if (cols * static_cast<int64_t>(first.element_size()) >= 512 &&
-      first.size(1) * padded(8 * vec) * static_cast<int64_t>(first.element_size()) < int64_t{1} << 30)
+  if (cols * elem >= 512 && first.size(1) * padded(8 * vec) * elem < int64_t{1} << 30)
     stride = padded(8 * vec);   // (not where it alone takes a matrix past the kernels' 1 GiB)
   Tensor buffer = at::empty({static_cast<int64_t>(in.size()), first.size(0), first.size(1), stride}, first.options());
-  TensorList out = buffer.unbind(0);
-  auto from = cptrs(in);
   auto to = slices(buffer);
-  check_status(pt_pack_rows(static_cast<int>(first.element_size()), static_cast<int>(in.size()), from.data(), to.data(),
-                            rows, cols, stride, stream_of(first)),
+  check_status(pt_pack_rows(static_cast<int>(elem), static_cast<int>(in.size()), cptrs(in).data(), to.data(), rows, cols,
+                            stride, stream_of(first)),
                "pack_rows");
-  return {std::move(out), stride};
+  return {{to.begin(), to.end()}, stride, buffer};
 }
 
 SeriesOut cauchy_matmul_out(bool separate, const TensorList& a_in, const TensorList& b_in, int64_t degree, bool trans_b,
@@ -331,19 +332,28 @@ SeriesOut cauchy_matmul_out(bool separate, const TensorList& a_in, const TensorL
                     "cauchy_matmul: bias must be a contiguous [n] vector of the operands' dtype and device");
   const int64_t batch = std::max(ba, bb);
   c10::DeviceGuard guard(a_in[0].device());
-  // float32 products below 2^28 multiply-adds take less time than the copies' launches gain (4 x 16 x 77 x 65
-  // at degree 4: 34 us, 45 with copies; 300 x 301 x 1001 by an ordinary matrix, 3.6e8 at degree 3: 44 and 26)
-  const int64_t terms = a_in.size() > 1 && b_in.size() > 1 ? (degree + 1) * (degree + 2) / 2
-                                                           : static_cast<int64_t>(std::max(a_in.size(), b_in.size()));
-  const bool elements = dtype == at::kDouble ||
-                        (dtype == at::kFloat && static_cast<double>(batch) * m * n * kd * terms < double(1 << 28));
-  const Rows a = packed_rows(a_in, elements), b = packed_rows(b_in, elements);
+  // Rows of no whole vectors: the 16-bit kernels need copies. float32 products gain by them (4 x 511 x 1023 x 769
+  // at degree 4: 704 -> 519 us; 300 x 301 x 1001 by an ordinary matrix, degree 3: 44 -> 26) from 2^28 multiply-adds
+  // (4 x 16 x 77 x 65, degree 4: 34 us, 45 with copies), over contractions of 128 at least (100001 x 33 x 65, degree
+  // 8: 200 us, 278; 300 x 17 x 16385: 80, 143) and 32 multiply-adds for every element copied (1 x 4097 x 16385,
+  // degree 3: 668, 774; 32 x 5 x 1001 x 1001, degree 8: 522, 805); of 420 products from 2^28 on, 3% of those
+  // copied take over 1.05 times their time without, 32% did by the first line alone. float64, bound by its MFMAs,
+  // does not gain (1006 -> 973 us and 57 -> 61 for the first two).
+  const bool whole_a = whole_rows(a_in), whole_b = whole_rows(b_in);
+  bool copy = dtype != at::kDouble;
+  if (dtype == at::kFloat && !(whole_a && whole_b)) {
+    const int64_t terms = a_in.size() > 1 && b_in.size() > 1 ? (degree + 1) * (degree + 2) / 2
+                                                             : static_cast<int64_t>(std::max(a_in.size(), b_in.size()));
+    const double products = static_cast<double>(batch) * m * n * kd * terms;
+    const double copied = (whole_a ? 0.0 : static_cast<double>(a_in.size()) * ba * m * kd) +
+                          (whole_b ? 0.0 : static_cast<double>(b_in.size()) * bb * n * kd);
+    copy = kd >= 128 && products >= double(1 << 28) && products >= 32 * copied;
+  }
+  const Rows a = whole_a || !copy ? own_rows(a_in) : packed_rows(a_in), b = whole_b || !copy ? own_rows(b_in) : packed_rows(b_in);
   SeriesOut out = series_out(separate, degree + 1, {batch, m, n}, a_in[0].options());
-  auto as = cptrs(a.matrices), bs = cptrs(b.matrices);
-  auto& cs = out.ptrs;
   const int status = pt_cauchy_matmul_strided(
-      dtype_code(dtype), static_cast<int>(degree), as.data(), static_cast<int>(a_in.size()), bs.data(),
-      static_cast<int>(b_in.size()), cs.data(), batch, m, n, kd, a.stride, b.stride, ba == 1 ? 0 : m * a.stride,
+      dtype_code(dtype), static_cast<int>(degree), a.ptrs.data(), static_cast<int>(a_in.size()), b.ptrs.data(),
+      static_cast<int>(b_in.size()), out.ptrs.data(), batch, m, n, kd, a.stride, b.stride, ba == 1 ? 0 : m * a.stride,
       bb == 1 ? 0 : b_in[0].size(1) * b.stride, trans_b ? 1 : 0, bias ? bias->data_ptr() : nullptr,
       stream_of(a_in[0]));
   check_status(status, "cauchy_matmul");
@@ -378,11 +388,10 @@ Tensor matmul_order_sum(const TensorList& a_in, const TensorList& b_in, bool tra
   TORCH_CHECK_VALUE(ba == bb || ba == 1 || bb == 1, "matmul_order_sum: batch dimensions do not broadcast");
   const int64_t batch = std::max(ba, bb);
   c10::DeviceGuard guard(a0.device());
-  const Rows a = packed_rows(a_in), b = packed_rows(b_in);
+  const Rows a = whole_rows(a_in) ? own_rows(a_in) : packed_rows(a_in), b = whole_rows(b_in) ? own_rows(b_in) : packed_rows(b_in);
   Tensor out = at::empty({batch, m, n}, a0.options());
-  auto as = cptrs(a.matrices), bs = cptrs(b.matrices);
   const int status = pt_matmul_order_sum(
-      dtype_code(a0.scalar_type()), static_cast<int>(a_in.size()), as.data(), bs.data(), out.data_ptr(), batch, m, n, k,
+      dtype_code(a0.scalar_type()), static_cast<int>(a_in.size()), a.ptrs.data(), b.ptrs.data(), out.data_ptr(), batch, m, n, k,
       a.stride, b.stride, ba == 1 ? 0 : a0.size(1) * a.stride, bb == 1 ? 0 : b0.size(1) * b.stride, trans_a ? 1 : 0,
       trans_b ? 1 : 0, stream_of(a0));
   check_status(status, "matmul_order_sum");

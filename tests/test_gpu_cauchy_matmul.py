@@ -343,3 +343,16 @@ def test_many_small_matrices(dtype, tol):
             want = A[o][part, 0].double() @ b[0].double()
             err = (got[o][part, 0].double() - want).abs().max() / want.abs().max()
             assert err <= tol, (o, err)
+
+
+# float32 rows of no whole vectors from 2^28 multiply-adds: contractions either side of 128, and few multiply-adds
+# for an element, where they are read as they are.
+@pytest.mark.parametrize("m,n,k", [(520, 1025, 127), (515, 1025, 129), (5, 4097, 4097), (31, 1025, 4097)])
+def test_float_rows_by_contraction_and_reuse(m, n, k):
+    degree, tol = 3, 1e-5
+    A, B = _series((m, k), degree, 1, torch.float32), _series((k, n), degree, 2, torch.float32)
+    with torch.no_grad(), PolyTensor.plain_range():
+        left, right = _poly(A) @ B[0].cuda(), A[0].cuda() @ _poly(B)
+    for o in range(degree + 1):
+        for got, want in ((left, A[o].double() @ B[0].double()), (right, A[0].double() @ B[o].double())):
+            assert (got.coeffs[o].cpu().double() - want).abs().max() <= tol * want.abs().max(), o
