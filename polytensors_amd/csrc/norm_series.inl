@@ -512,11 +512,12 @@ __global__ __launch_bounds__(1024) void norm_series_bwd_reg_kernel(
     }
   }
 
-  if constexpr (WEIGHT) {   // (lanes past the row read column 0: their cotangent is zero)
+  if constexpr (WEIGHT) {   // (zeros past the row, as the cotangent has: another column's value may not be finite)
 #pragma unroll
     for (int ch = 0; ch < CHUNKS; ++ch) {
       const int col = (ch * tpr + tid) * V;
       wv[ch] = load_vec<T, V>(w + (col < n ? col : 0));
+      if (col >= n) wv[ch] = {};
     }
   }
   auto weighted = [&](A v, int ch, int e) { return WEIGHT ? v * vec_get(wv[ch], e) : v; };

@@ -173,6 +173,26 @@ def test_norm_gradient_series_with_an_ordinary_weight(layer, n, dtype):
     _check(x.grad.coeffs, dx, dtype)
 
 
+# A weight that is infinite in the first column (rows whose block has lanes past them): the gradient is not finite
+# where the formula's is not, and no NaN comes in from outside the row.
+@pytest.mark.parametrize("layer", [False, True])
+@pytest.mark.parametrize("n", [8, 72, 1000])
+def test_norm_gradient_with_an_infinite_weight(layer, n):
+    degree = 1
+    x = PolyTensor(tuple(c.float().cuda() for c in _series((3, n), degree, 41)), requires_grad=True)
+    g = [c.float().cuda() for c in _series((3, n), degree, 42)]
+    w = torch.ones(n, device="cuda")
+    w[0] = float("inf")
+    grads = []
+    for weight, cot in ((w, g), (None, [c * w for c in g])):
+        x.grad = None
+        with PolyTensor.plain_range():
+            (F.layer_norm(x, (n,), weight) if layer else F.rms_norm(x, (n,), weight)).backward(PolyTensor(tuple(cot)))
+        grads.append(x.grad.coeffs)
+    for got, want in zip(*grads):
+        torch.testing.assert_close(got, want, rtol=1e-5, atol=0, equal_nan=True)
+
+
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 def test_norm_with_series_weight_gradients(dtype):
     # The weight multiplies as a separate series product (as the reference's
