@@ -66,11 +66,16 @@ def _affine_coeffs(a, input, shape):
 
 
 def _ordinary_affine(a, input, shape):
-    """An ordinary weight or bias without a graph as the kernels take it ([n], contiguous), else None."""
+    """An ordinary weight or bias without a graph as the kernels take it ([n], contiguous, at a 16-byte aligned
+    place: a view into a larger buffer may not be, and would take the whole series to the kernels' element loads;
+    8192 x 4096 bfloat16 RMSNorm and its gradient at degree 4: 807 us, 314 with the weight copied), else None."""
     if a is None or isinstance(a, PolyTensor) or a.requires_grad or _gate.transformed(a):
         return None
     coeffs = _affine_coeffs(a, input, shape)
-    return coeffs[0] if coeffs else None
+    if not coeffs:
+        return None
+    (c,) = coeffs
+    return c if c.storage_offset() * c.element_size() % 16 == 0 else c.clone()
 
 
 def _needs_grad(*values):

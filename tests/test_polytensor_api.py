@@ -206,3 +206,16 @@ def test_transformed_bias_and_weight_are_not_kernel_operands():
     seen = []
     torch.func.vmap(lambda b: (seen.append(taken(b)), b)[1])(torch.ones(2, 5))
     assert seen == [(False, False)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_ordinary_norm_weight_is_handed_over_aligned(dtype):
+    """A norm's weight that is a view at an odd place is copied to where the kernels read vectors."""
+    from polytensors_amd import _fused_norm
+
+    buffer = torch.arange(65, dtype=dtype)
+    x = torch.zeros(2, 64, dtype=dtype)
+    for offset in (0, 1):
+        got = _fused_norm._ordinary_affine(buffer[offset:offset + 64], x, (64,))
+        assert torch.equal(got, buffer[offset:offset + 64])
+        assert got.storage_offset() * got.element_size() % 16 == 0
