@@ -7,9 +7,10 @@ random polynomial (the GPU round trip through the plane kernels is in
 tests/test_gpu_complex.py).
 """
 
+import pytest
 import torch
 
-from polytensors_amd import _complex
+from polytensors_amd import PolyTensor, _complex, _fused_attention
 
 
 def test_weights_evaluate_every_monomial_at_i():
@@ -28,3 +29,34 @@ def test_weights_on_a_random_polynomial():
         nodes, weights = _complex.nodes_and_weights(degree)
         p = lambda z: sum(c * z ** j for j, c in enumerate(coeffs))  # noqa: E731
         assert abs(sum(w * p(x) for w, x in zip(weights, nodes)) - p(1j)) < 1e-12 * sum(abs(c) for c in coeffs) * 2 ** degree
+
+
+def _direction(shape, degree, dtype, complex_=True):
+    """A series of the given shape without its memory (one element, expanded)."""
+    wide = {torch.float32: torch.complex64, torch.float64: torch.complex128}[dtype] if complex_ else dtype
+    return PolyTensor((torch.zeros(1, dtype=dtype).expand(shape),) + (torch.zeros(1, dtype=wide).expand(shape),) * degree)
+
+
+# Both sides of the rule that runs the interpolation nodes of an attention as one batch.
+@pytest.mark.parametrize("heads,L,S,d,degree,dtype,one_launch", [
+    (24, 512, 512, 64, 3, torch.float32, True), (8, 1024, 1024, 128, 3, torch.float32, True),
+    (64, 1024, 1024, 128, 2, torch.float32, False), (256, 256, 256, 128, 1, torch.float32, False),
+    (64, 4, 1000, 128, 1, torch.float32, False), (1, 64, 64, 128, 2, torch.float32, True),
+    (1024, 16, 16, 32, 1, torch.float32, True), (2048, 16, 16, 32, 1, torch.float32, False),
+    (1, 1024, 1024, 128, 3, torch.float64, False), (8, 1024, 1024, 32, 3, torch.float64, True),
+    (24, 512, 512, 128, 1, torch.float64, False), (1, 16, 16, 16, 9, torch.float64, False), (0, 16, 16, 16, 1, torch.float64, False)])
+def test_attention_nodes_in_one_launch(heads, L, S, d, degree, dtype, one_launch):
+    q, k, v = (_direction((heads, n, d), degree, dtype) for n in (L, S, S))
+    assert _fused_attention._stacks_nodes(q, k, v, None, degree) is one_launch
+    assert not _fused_attention._stacks_nodes(q, k, v, torch.zeros(2, L, S, dtype=torch.bool), degree)
+
+
+def test_attention_nodes_in_one_launch_by_kernel():
+    """Shapes that are no longer launch-bound: an ordinary operand or an additive mask takes the other kernel."""
+    q, k, v = (_direction((24, 512, 64), 3, torch.float32) for _ in range(3))
+    stacks = _fused_attention._stacks_nodes
+    assert stacks(q, k, v, torch.ones(512, 512, dtype=torch.bool), 3)
+    q, k, v = (_direction((8, 512, 64), 3, torch.float32) for _ in range(3))   # 64 workgroups
+    assert stacks(q, k, v, None, 3)
+    assert not stacks(q, torch.zeros(8, 512, 64), v, None, 3)
+    assert not stacks(q, k, v, torch.zeros(512, 512), 3)
