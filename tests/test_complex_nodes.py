@@ -10,7 +10,7 @@ tests/test_gpu_complex.py).
 import pytest
 import torch
 
-from polytensors_amd import PolyTensor, _complex, _fused_attention
+from polytensors_amd import PolyTensor, _complex, _fused_activation, _fused_attention
 
 
 def test_weights_evaluate_every_monomial_at_i():
@@ -60,3 +60,10 @@ def test_attention_nodes_in_one_launch_by_kernel():
     assert stacks(q, k, v, None, 3)
     assert not stacks(q, torch.zeros(8, 512, 64), v, None, 3)
     assert not stacks(q, k, v, torch.zeros(512, 512), 3)
+
+
+@pytest.mark.parametrize("degree,numel,dtype,one_pass", [
+    (1, 1 << 21, torch.float64, True), (1, (1 << 21) + 1, torch.float64, False), (2, 1 << 24, torch.float64, True),
+    (1, 1 << 24, torch.float32, True), (9, 4, torch.float32, False)])
+def test_activation_in_one_pass(degree, numel, dtype, one_pass):
+    assert _fused_activation._one_pass(_direction((numel,), degree, dtype)) is one_pass
