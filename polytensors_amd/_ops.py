@@ -481,12 +481,26 @@ def _mm_setup(ctx, inputs, output):
     ctx.n_inputs = len(inputs)
 
 
-def _sums(*operands):
-    """Whether matmul_order_sum takes these matrices: no graph of the gradient is asked for, a type
-    it has, each (row-padded) matrix below 1 GiB."""
+def _sums(m, n, batch, *operands):
+    """Whether matmul_order_sum takes these matrices, for a gradient of [batch, m, n]: no graph of the gradient
+    is asked for, a type it has, each (row-padded) matrix below 1 GiB, its tiles within one launch."""
     if torch.is_grad_enabled() or operands[0].dtype == torch.float64:
         return False
-    return all((x.shape[-2] + 8) * (x.shape[-1] + 8) * x.element_size() < 1 << 30 for x in operands)
+    side = 64 if operands[0].dtype == torch.float32 else 128
+    return (-(-m // side) * -(-n // side) * batch < 1 << 24 and
+            all((x.shape[-2] + 8) * (x.shape[-1] + 8) * x.element_size() < 1 << 30 for x in operands))
+
+
+def _sum_pays(m, n, batch, degree, dtype):
+    """Whether an ordinary left operand's gradient, [batch, m, n], is formed as one sum of products rather than as the
+    coefficient K of a series product. The sum has degree + 1 products for the series' (degree + 1)(degree + 2) / 2,
+    but in 16 bits tiles of 128 a side for 64: it needs enough of them, and well enough filled (4096 x 24 x 32 by 16
+    columns, degree 1: 13 us as a series, 36 as a sum; 16384 x 16 x 136 by 8, degree 3: 203, 389; 20000 x 136 by 96,
+    degree 8: 66, 24; of 172 shapes 41 took over 1.1 times as long as a sum, 1 of those that it is now used for)."""
+    if dtype == torch.float32:
+        return True
+    tiles = lambda side: -(-m // side) * -(-n // side) * batch   # noqa: E731
+    return tiles(128) >= 128 and (degree + 2) * tiles(64) >= 8 * tiles(128)
 
 
 def _mm_backward(ctx, grad):
@@ -497,7 +511,9 @@ def _mm_backward(ctx, grad):
     batch = c[0].shape[0]
     ga = gb = None
     if need_a:   # dA = C (*) B^T
-        if na == 1 and degree > 0 and _sums(c[0], b[0]):   # an ordinary A: coefficient K alone, sum_s C_{K-s} B_s^T
+        size = (a[0].shape[-2], a[0].shape[-1], batch)
+        if na == 1 and degree > 0 and _sum_pays(*size, degree, a[0].dtype) and _sums(*size, c[0], b[0]):
+            # an ordinary A: coefficient K alone, sum_s C_{K-s} B_s^T
             da = matmul_order_sum(c[::-1][:nb], b, False, not trans_b)[None]
         else:
             da = cauchy_matmul(c, b, degree, not trans_b)
@@ -505,7 +521,7 @@ def _mm_backward(ctx, grad):
             da = da.sum(1, keepdim=True)
         ga = _read_back(da, na)
     if need_b:   # dB = A^T (*) C, or its transpose for a [batch, n, k] operand
-        if nb == 1 and _sums(a[0], c[0]):   # an ordinary B: sum_s A_s^T C_{K-s}
+        if nb == 1 and _sums(b[0].shape[-2], b[0].shape[-1], batch, a[0], c[0]):   # an ordinary B: sum_s A_s^T C_{K-s}
             gs = c[::-1][:na]
             db = matmul_order_sum(*((gs, a) if trans_b else (a, gs)), True, False)[None]
         elif trans_b:

@@ -301,6 +301,22 @@ def test_gradient_of_an_ordinary_matrix(dtype, tol, m, k, n, batch, degree):
         assert err <= tol * (2 if batch else 1), (name, err)
 
 
+# The gradient of an ordinary left operand in 16 bits, as a sum of products (enough and filled tiles) and as a series
+# product: batches of both, ragged sides. Tolerance as above.
+@pytest.mark.parametrize("m,k,n,batch,degree", [(130, 130, 24, 40, 3), (128, 128, 40, 130, 1), (24, 16, 32, 150, 2),
+                                                (16, 9, 17, 200, 4)])
+def test_gradient_of_an_ordinary_left_operand(m, k, n, batch, degree):
+    g = torch.Generator().manual_seed(m + n)
+    make = lambda *shape: torch.randn(*shape, generator=g, dtype=torch.float64).to(torch.bfloat16)   # noqa: E731
+    Y, C = [make(batch, k, n) for _ in range(degree + 1)], [make(batch, m, n) for _ in range(degree + 1)]
+    w = make(batch, m, k).cuda().requires_grad_()
+    with PolyTensor.plain_range(), PolyTensor.coefficient_autograd():
+        out = w @ PolyTensor(tuple(c.cuda() for c in Y))
+    (got,) = torch.autograd.grad(out.coeffs, w, [c.cuda() for c in C])
+    want = sum(c.double() @ y.double().transpose(1, 2).contiguous() for c, y in zip(C, Y))
+    assert (got.cpu().double() - want).abs().max() <= 2.0 ** -8 * want.abs().max()
+
+
 # The recorded operations return a tensor per order: cotangents of some orders alone, non-contiguous
 # and misaligned ones, and an order's gradient from another order's output are what torch's autograd of
 # the same series arithmetic gives (the oracle's, differentiated), for each of the four operations.

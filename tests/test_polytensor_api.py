@@ -219,3 +219,23 @@ def test_ordinary_norm_weight_is_handed_over_aligned(dtype):
         got = _fused_norm._ordinary_affine(buffer[offset:offset + 64], x, (64,))
         assert torch.equal(got, buffer[offset:offset + 64])
         assert got.storage_offset() * got.element_size() % 16 == 0
+
+
+def test_gradients_of_ordinary_operands_by_size():
+    """Either side of the rules for the gradient of an ordinary matrix: as one sum of products within a launch's
+    tiles, a type and a size that kernel has; in 16 bits on the left only where its tiles are filled."""
+    from polytensors_amd import _ops
+
+    shape = lambda dtype, *s: torch.zeros(1, dtype=dtype).expand(s)   # noqa: E731
+    with torch.no_grad():
+        for dtype, side in ((torch.bfloat16, 128), (torch.float32, 64)):
+            x = shape(dtype, 65535, 1, 8)
+            assert _ops._sums(1, 255 * side, 65535, x, x)
+            assert not _ops._sums(1, 257 * side, 65535, x, x)
+            assert not _ops._sums(8, 8, 1, x, shape(dtype, 1, 1 << 20, 1 << 10))
+        assert not _ops._sums(8, 8, 1, shape(torch.float64, 1, 8, 8))
+    assert not _ops._sums(8, 8, 1, shape(torch.float32, 1, 8, 8))   # a graph of the gradient
+    pays = lambda *a: _ops._sum_pays(*a, torch.bfloat16)   # noqa: E731
+    assert not pays(128, 128, 127, 8) and pays(128, 128, 128, 8)
+    assert not pays(24, 16, 4096, 1) and not pays(16, 8, 16384, 3) and pays(72, 8, 16384, 8)
+    assert _ops._sum_pays(24, 16, 4096, 1, torch.float32)
