@@ -479,41 +479,43 @@ static int launch_order_gemm(const OrderGemmParams<T>& p, int64_t batch, hipStre
 
 // Whether the product runs order by order rather than in the kernels with all orders in a workgroup
 // (cauchy_matmul*.inl): those read an ordinary tile once for all orders and have smaller tiles, this one streams a
-// long contraction faster. The estimated times of both in us, each a fixed part and, for every round of
-// workgroups over the chip, one for the stores and one for every 32 (floats: 16) of the contraction; fitted to 1700
-// shapes (sides 1 to 100000, contractions 8 to 4096, 1 to 16384 matrices, degrees 1 to 8), whose times they
-// give to 15-20%. Order by order where it is 15% less: of those shapes 3% then take over 1.08 times the time of the
-// other kernel, where always running order by order 55% do, up to 7 times: 4096 x 16 x 16 x 16 bfloat16, degree 8,
-// 40 us and 202 order by order; 200000 x 8 x 8, 53 and 129; 2048 x 8 x 2048 float32, degree 3, 17 and 30;
-// 768 x 4096 x 256 bfloat16, degree 8, 104 and 40.
+// long contraction faster. The estimated times of both in us: a fixed part, and for every round of workgroups
+// over the chip one for the stores and one for every 32 (floats: 16) of the contraction; fitted to 2400 products
+// (sides 1 to 100000, contractions 8 to 4096, 1 to 16384 matrices, degrees 1 to 8; 1e4 to 1e12 multiply-adds),
+// whose times they give to 7-9% (floats) and 13-20%. Order by order where it is 10% less (floats 5%): then 2% of
+// the products take over 1.08 times what the other kernel takes; always order by order 45% do, up to 8 times (4096
+// x 16 x 16 x 16 bfloat16, degree 8: 40 us and 202; 200000 x 8 x 8, 53 and 129; 2048 x 8 x 2048 float32, degree 3, 17
+// and 30; the other way 768 x 4096 x 256 bfloat16, degree 8, 104 and 40; 8192 x 768 x 3072 float32, 1350 and 1150).
 template <typename T>
 static bool order_gemm_pays(const CauchyArgs& a) {
   const int64_t orders = std::max(a.a_orders, a.b_orders);
   const double n1 = static_cast<double>(orders);
   auto tiles = [&](int64_t bm, int64_t bn) { return (a.m + bm - 1) / bm * ((a.n + bn - 1) / bn) * a.batch; };
-  // rounds of `per` workgroups; `half` of one where the last has at most half of them
-  auto rounds = [](int64_t count, int64_t per, double half) {
-    const int64_t rest = count % per;
-    return static_cast<double>(count / per) + (rest == 0 ? 0.0 : 2 * rest <= per ? half : 1.0);
+  auto whole_rounds = [](int64_t count) { return static_cast<double>((count + 255) / 256); };
+  // rounds of 512 workgroups; `half` of one where the last has at most half of them
+  auto rounds = [](int64_t count, double half) {
+    const int64_t rest = count % 512;
+    return static_cast<double>(count / 512) + (rest == 0 ? 0.0 : rest <= 256 ? half : 1.0);
   };
   if constexpr (sizeof(T) == 2) {
     const double chunks = static_cast<double>((a.k + 31) / 32);
     const double all = orders <= 5 && a.m >= 256 && a.n >= 256
-        ? 2.5 + rounds(tiles(128, 128), 256, 1.0) * (1.95 * n1 + chunks * (0.065 + 0.25 * n1))
-        : 2.5 + rounds(tiles(64, 64), 512, 0.43) * (0.94 * n1 + chunks * (0.16 + 0.17 * n1));
-    const int64_t small = tiles(128, 128) * orders;
+        ? 2.4 + whole_rounds(tiles(128, 128)) * (2.0 * n1 + chunks * (0.075 + 0.23 * n1))
+        : 2.4 + rounds(tiles(64, 64), 0.44) * (0.94 * n1 + chunks * (0.17 + 0.17 * n1));
+    const int64_t small = tiles(128, 128) * orders, large = tiles(256, 256) * orders;
     double each;   // (the tiles as launch_order_gemm picks them)
-    if (small <= 256 && chunks >= 16) each = 5.2 + 0.20 * chunks;
-    else if (order_large_tiles(tiles(256, 256) * orders, small)) each = 4.9 + rounds(tiles(256, 256) * orders, 256, 1.0) * (8.6 + 0.78 * chunks);
-    else each = 4.9 + rounds(small, 512, 0.24) * (4.2 + 0.35 * chunks);
-    return 1.15 * each <= all;
+    if (small <= 256 && chunks >= 16) each = 6.2 + 0.20 * chunks;
+    else if (order_large_tiles(large, small)) each = 3.7 + whole_rounds(large) * (9.8 + 0.77 * chunks);
+    else each = 3.7 + rounds(small, 0.46) * (3.9 + 0.47 * chunks);
+    return 1.10 * each <= all;
   } else {
     const double chunks = static_cast<double>((a.k + 15) / 16);
-    const double all = 2.4 + rounds(tiles(64, 64), 512, 0.52) * (0.93 * n1 + chunks * (0.26 + 0.53 * n1));
+    const double all = 2.3 + rounds(tiles(64, 64), 0.56) * (0.97 * n1 + chunks * (0.125 + 0.53 * n1));
     const int64_t t[3] = {tiles(128, 128) * orders, tiles(128, 64) * orders, tiles(64, 64) * orders};
     const int pick = order_float_tile(t);
-    constexpr double kStores[3] = {1.21, 1.81, 0.74}, kChunk[3] = {1.59, 0.49, 0.275};
-    return 1.15 * (3.4 + rounds(t[pick], 256, 1.0) * (kStores[pick] + chunks * kChunk[pick])) <= all;
+    constexpr double kStores[3] = {3.6, 1.54, 0.76}, kOne[3] = {1.05, 0.59, 0.30}, kMany[3] = {0.96, 0.51, 0.27};
+    const double q = whole_rounds(t[pick]);   // tiles of the busiest CU
+    return 1.05 * (3.2 + q * kStores[pick] + chunks * (q == 1.0 ? kOne[pick] : q * kMany[pick])) <= all;
   }
 }
 
