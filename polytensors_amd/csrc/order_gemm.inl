@@ -482,7 +482,7 @@ static int launch_order_gemm(const OrderGemmParams<T>& p, int64_t batch, hipStre
 // long contraction faster. The estimated times of both in us: a fixed part, and for every round of workgroups
 // over the chip one for the stores and one for every 32 (floats: 16) of the contraction; fitted to 2400 products
 // (sides 1 to 100000, contractions 8 to 4096, 1 to 16384 matrices, degrees 1 to 8; 1e4 to 1e12 multiply-adds),
-// whose times they give to 7-9% (floats) and 13-20%. Order by order where it is 10% less (floats 5%): then 2% of
+// whose times they give to 7-9% (floats) and 13-20%. Order by order where it is less (halves: by 10%): then 2% of
 // the products take over 1.08 times what the other kernel takes; always order by order 45% do, up to 8 times (4096
 // x 16 x 16 x 16 bfloat16, degree 8: 40 us and 202; 200000 x 8 x 8, 53 and 129; 2048 x 8 x 2048 float32, degree 3, 17
 // and 30; the other way 768 x 4096 x 256 bfloat16, degree 8, 104 and 40; 8192 x 768 x 3072 float32, 1350 and 1150).
@@ -515,7 +515,7 @@ static bool order_gemm_pays(const CauchyArgs& a) {
     const int pick = order_float_tile(t);
     constexpr double kStores[3] = {3.6, 1.54, 0.76}, kOne[3] = {1.05, 0.59, 0.30}, kMany[3] = {0.96, 0.51, 0.27};
     const double q = whole_rounds(t[pick]);   // tiles of the busiest CU
-    return 1.05 * (3.2 + q * kStores[pick] + chunks * (q == 1.0 ? kOne[pick] : q * kMany[pick])) <= all;
+    return 3.2 + q * kStores[pick] + chunks * (q == 1.0 ? kOne[pick] : q * kMany[pick]) <= all;
   }
 }
 
