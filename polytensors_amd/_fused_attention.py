@@ -223,39 +223,45 @@ def _composed(query, key, value, attn_mask, is_causal, scale):
     return (e / e.sum(-1, keepdim=True)) @ value
 
 
-def _stacks_nodes(query, key, value, attn_mask, degree):
+def _stacks_nodes(query, key, value, attn_mask, is_causal, degree):
     """Whether a complex direction's interpolation nodes run in one launch, as a batch, rather than one after
-    another. A batch repeats order 0 for every node; it gains where a node's launch alone leaves the chip idle. Of 1230
-    shapes (1 to 1024 heads, 1 to 1024 queries, 16 to 4096 keys, degrees 1 to 4) none takes over 1.02 times as long in
-    the batch where this is true, 163 do where it is not.
+    another. A batch repeats order 0 for every node; it gains where a node's launch alone leaves the chip idle. Of 1380
+    shapes (1 to 1024 heads, 1 to 1024 queries, 16 to 4096 keys, degrees 1 to 4) none takes over 1.04 times as long in
+    the batch where this is true, 180 do where it is not.
 
     * Launch-bound: below 3e8 multiply-adds, 32 MB of operands and 2048 workgroups (a head of 64 x 64 at degree 2: 217 and 108 us).
-    * A workgroup takes a head and 64 queries. Below 256, one a CU, the float32 kernel for series over whole 16-key
-      blocks leaves CUs idle (24 heads of 512, d 64, causal, degree 3: 680 and 337 us; 64 heads of 1024, d 128,
-      causal, degree 2, 1024 workgroups: 2940 and 3181). The other kernel shares few workgroups' keys out over the
-      chip by itself, below 128 (1 head of 1024, d 128, float64, degree 3: 915 and 1554 us), and is then in need of
-      the batch from there on, past degree 1 (8 heads of 1024, d 32, causal, float64, degree 3: 2560 and 740).
+    * A workgroup takes a head and 64 queries. Below 512, two a CU, the float32 kernel for series over whole 16-key
+      blocks leaves CUs idle (24 heads of 512, d 64, causal, degree 3: 680 and 337 us), from there on with small heads of
+      some length (96 of 1024, d 16, causal, degree 3: 1513 and 1288; 64, d 64: 3304 and 3081), not with large or short
+      ones (64 of 1024, d 128, causal, degree 2: 2940 and 3181; 1800 of 64, d 32, degree 2: 336 and 357). The other kernel shares few workgroups' keys out over the chip by itself, below 128 (1 head of 1024, d
+      128, float64, degree 3: 915 and 1554 us), and needs the batch from there on, past degree 1 (8 heads of 1024,
+      d 32, causal, float64, degree 3: 2560 and 740).
     """
-    if degree > _gate.MAX_DEGREE or (attn_mask is not None and attn_mask.numel() != query.shape[-2] * key.shape[-2]):
+    q, k = (x.coeffs[0] if isinstance(x, PolyTensor) else x for x in (query, key))   # (a wrapper's attributes cost a call each)
+    *lead, L, d = q.shape
+    S = k.shape[-2]
+    if degree > _gate.MAX_DEGREE or (attn_mask is not None and attn_mask.numel() != L * S):
         return False   # (past the kernel's degree; a mask per head would be repeated for every node)
-    heads, L, S, d = math.prod(query.shape[:-2]), query.shape[-2], key.shape[-2], query.shape[-1]
-    products = 2 * heads * L * S * d * (degree + 1) * (degree + 2) // 2
-    size = query.element_size() * heads * (L + 2 * S) * d * (degree + 1)
+    heads = math.prod(lead)
     workgroups = heads * -(-L // 64)
     if not 0 < workgroups < 2048:
         return False
+    products = 2 * heads * L * S * d * (degree + 1) * (degree + 2) // 2
+    size = q.element_size() * heads * (L + 2 * S) * d * (degree + 1)
     if products < 3e8 and size < 32e6:
         return True
-    pipelined = (query.dtype == torch.float32 and S % 16 == 0 and all(isinstance(x, PolyTensor) for x in (query, key, value))
-                 and (attn_mask is None or attn_mask.dtype == torch.bool))
-    return workgroups < 256 and (pipelined or (degree >= 2 and workgroups >= 128))
+    if (q.dtype == torch.float32 and S % 16 == 0 and all(isinstance(x, PolyTensor) for x in (query, key, value))
+            and (attn_mask is None or attn_mask.dtype == torch.bool)):
+        return workgroups < 512 or (d <= 32 and degree >= 2 and L >= 256) or (d <= 64 and degree >= 3 and L >= 512 and
+                                                                              bool(is_causal))
+    return degree >= 2 and 128 <= workgroups < 256
 
 
 def attention_checked(query, key, value, attn_mask=None, is_causal=False, scale=None):
     """``attention`` for a call whose eligibility (including dropout and GQA) the caller checked."""
     if _complex.has_complex(query, key, value):
         degree = next(x.degree for x in (query, key, value) if isinstance(x, PolyTensor))
-        if (_stacks_nodes(query, key, value, attn_mask, degree) and not _needs_grad(query, key, value)
+        if (_stacks_nodes(query, key, value, attn_mask, is_causal, degree) and not _needs_grad(query, key, value)
                 and not _gate.coefficient_graph(query, key, value)):
             return _complex.at_stacked_nodes(attention, "scaled_dot_product_attention", query, key, value,
                                              attn_mask=attn_mask, is_causal=is_causal, scale=scale)

@@ -40,26 +40,29 @@ def _direction(shape, degree, dtype, complex_=True):
 # Both sides of the rule that runs the interpolation nodes of an attention as one batch.
 @pytest.mark.parametrize("heads,L,S,d,degree,dtype,one_launch", [
     (24, 512, 512, 64, 3, torch.float32, True), (8, 1024, 1024, 128, 3, torch.float32, True),
-    (64, 1024, 1024, 128, 2, torch.float32, False), (256, 256, 256, 128, 1, torch.float32, False),
+    (64, 1024, 1024, 128, 2, torch.float32, False), (24, 1024, 1024, 128, 1, torch.float32, True),
+    (64, 512, 512, 64, 2, torch.float32, False), (64, 1024, 1024, 32, 2, torch.float32, True), (1800, 64, 64, 32, 2, torch.float32, False), (256, 256, 256, 128, 1, torch.float32, False),
     (64, 4, 1000, 128, 1, torch.float32, False), (1, 64, 64, 128, 2, torch.float32, True),
     (1024, 16, 16, 32, 1, torch.float32, True), (2048, 16, 16, 32, 1, torch.float32, False),
     (1, 1024, 1024, 128, 3, torch.float64, False), (8, 1024, 1024, 32, 3, torch.float64, True),
     (24, 512, 512, 128, 1, torch.float64, False), (1, 16, 16, 16, 9, torch.float64, False), (0, 16, 16, 16, 1, torch.float64, False)])
 def test_attention_nodes_in_one_launch(heads, L, S, d, degree, dtype, one_launch):
     q, k, v = (_direction((heads, n, d), degree, dtype) for n in (L, S, S))
-    assert _fused_attention._stacks_nodes(q, k, v, None, degree) is one_launch
-    assert not _fused_attention._stacks_nodes(q, k, v, torch.zeros(2, L, S, dtype=torch.bool), degree)
+    assert _fused_attention._stacks_nodes(q, k, v, None, False, degree) is one_launch
+    assert not _fused_attention._stacks_nodes(q, k, v, torch.zeros(2, L, S, dtype=torch.bool), False, degree)
 
 
 def test_attention_nodes_in_one_launch_by_kernel():
     """Shapes that are no longer launch-bound: an ordinary operand or an additive mask takes the other kernel."""
     q, k, v = (_direction((24, 512, 64), 3, torch.float32) for _ in range(3))
     stacks = _fused_attention._stacks_nodes
-    assert stacks(q, k, v, torch.ones(512, 512, dtype=torch.bool), 3)
+    assert stacks(q, k, v, torch.ones(512, 512, dtype=torch.bool), False, 3)
     q, k, v = (_direction((8, 512, 64), 3, torch.float32) for _ in range(3))   # 64 workgroups
-    assert stacks(q, k, v, None, 3)
-    assert not stacks(q, torch.zeros(8, 512, 64), v, None, 3)
-    assert not stacks(q, k, v, torch.zeros(512, 512), 3)
+    assert stacks(q, k, v, None, False, 3)
+    assert not stacks(q, torch.zeros(8, 512, 64), v, None, False, 3)
+    assert not stacks(q, k, v, torch.zeros(512, 512), False, 3)
+    q, k, v = (_direction((64, 1024, 64), 3, torch.float32) for _ in range(3))   # 1024 workgroups
+    assert stacks(q, k, v, None, True, 3) and not stacks(q, k, v, None, False, 3)
 
 
 @pytest.mark.parametrize("degree,numel,dtype,one_pass", [
