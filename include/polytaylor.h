@@ -224,8 +224,7 @@ size_t pt_cross_entropy_series_noalloc_max_bytes(void);
  * operands, fp32 accumulation, each output element rounded once; needs k and, unless trans_b, n
  * to be multiples of 8, 16-byte aligned operands, batch strides that are multiples of 8 and each
  * matrix below 1 GiB, else PT_UNSUPPORTED). Any alignment of c is accepted: 16-bit outputs are
- * written 8 bytes at a time where n is a multiple of 4 and every c[o] is 8-byte aligned, else one
- * element at a time).
+ * written 8 bytes at a time at any element, the last columns of a row one element at a time.
  */
 int pt_cauchy_matmul(int dtype, int degree, const void* const* a, int a_orders,
                      const void* const* b, int b_orders, void* const* c,
@@ -235,10 +234,12 @@ int pt_cauchy_matmul(int dtype, int degree, const void* const* a, int a_orders,
 
 /*
  * pt_cauchy_matmul of operands with row strides: rows of a lda elements apart, of b ldb (both at
- * least the row length and at most 2^31 - 1, else PT_UNSUPPORTED). Where lda (ldb) is a multiple of a 16-byte vector and the rows of a (of b
- * if trans_b) run along k, the values from k to the next multiple of a vector must be zero; b's
- * values past n (not trans_b) take no part. So 16-bit operands of any k and n run with padded rows
- * (pt_pack_rows): here the 16-bit kernels need lda and ldb, not k and n, to be multiples of 8.
+ * least the row length and at most 2^31 - 1, else PT_UNSUPPORTED). Where lda (ldb) is a multiple of
+ * a 16-byte vector and the rows of a (of b if trans_b) run along k, the values from k to the next
+ * multiple of a vector must be zero; b's values past n (not trans_b) take no part, but are read, as
+ * every row, the last one too, is to the next multiple of a vector. So 16-bit operands of any k and
+ * n run with padded rows (pt_pack_rows): here the 16-bit kernels need lda and ldb, not k and n, to
+ * be multiples of 8.
  * bias: null, or n values of `dtype` (any alignment) added to every row of C_0 before it is rounded
  *       (the bias of a linear layer, an ordinary tensor, adds to the constant order:
  *       /root/reference/src/polytensors/_range_ops.py:109-132).
@@ -267,7 +268,8 @@ int pt_pack_rows(int elem_bytes, int count, const void* const* src, void* const*
  * c: [batch, m, n] contiguous.
  * dtype: PT_FLOAT32, PT_BFLOAT16 or PT_FLOAT16 (fp32 accumulation, each element rounded once).
  * Rows are read in 16-byte vectors: operands 16-byte aligned, row and batch strides multiples of 16
- * bytes, each matrix (its rows times the row stride) below 1 GiB, else PT_UNSUPPORTED. The values of a
+ * bytes, each matrix (its rows times the row stride) below 1 GiB, and less than 2^24 tiles (of 128 x 128 elements
+ * of c, float32 64 x 64) in all, else PT_UNSUPPORTED. The values of a
  * row from its length to the next multiple of a vector are zeros where it runs along k, and take no
  * part where it runs along m or n. trans_a needs trans_b = 0.
  */

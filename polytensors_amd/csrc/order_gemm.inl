@@ -1,12 +1,13 @@
 // Products of a series with an ordinary matrix, C_o = A_o B (or A B_o), o = 0..K, as one matrix
 // product in which the orders are further rows (columns) of C; and the sum of products of two series,
 // C = sum_s op(A_s) op(B_s) (the gradient of an ordinary operand), in which the orders lengthen the
-// contraction. float32, and bfloat16 / float16 with float32 accumulation. An ordinary operand mixes no orders, so the k-diagonals share nothing as
-// they do in the series-by-series kernels (cauchy_matmul*.inl, which ran these products before):
-// what bounds it is how fast one tile's contraction streams from memory to the MFMAs. With K = 3,
-// the forward products and the input gradients of a 1024 -> 4096 -> 1024 bfloat16 layer pair on 4096
-// rows took 232 and 222 us each (600 TFLOP/s) and take 137 and 129 (1000-1070); 8192 rows of float32,
-// 768 -> 3072, 1356 us (114 TFLOP/s) and 1281 (121).
+// contraction. float32, and bfloat16 / float16 with float32 accumulation. An ordinary operand mixes no orders, so the
+// k-diagonals share nothing as they do in the series-by-series kernels (cauchy_matmul*.inl, which run the products
+// that are not worth it here, order_gemm_pays): what bounds it is how fast one tile's contraction streams from memory
+// to the MFMAs. With K = 3, the forward products and the input gradients of a 1024 -> 4096 -> 1024 bfloat16 layer
+// pair on 4096 rows took 232 and 222 us each (600 TFLOP/s) there and take 139-144 in a training step (950-990, MFMA
+// busy 46%; a forward product launched alone 123 us); 8192 rows of float32 with a bias, 768 -> 3072, 1410 us a call
+// among others and 1149 (134.5 TFLOP/s, MFMA busy 85%).
 //
 // * Chunks of 64 bytes of contraction (32 halves, 16 floats) are moved into LDS by LDS DMA
 //   (half_mfma.h) into four buffers, two chunks at a time where an operand's rows run along the
