@@ -225,9 +225,9 @@ def _composed(query, key, value, attn_mask, is_causal, scale):
 
 def _stacks_nodes(query, key, value, attn_mask, is_causal, degree):
     """Whether a complex direction's interpolation nodes run in one launch, as a batch, rather than one after
-    another. A batch repeats order 0 for every node; it gains where a node's launch alone leaves the chip idle. Of 1380
-    shapes (1 to 1024 heads, 1 to 1024 queries, 16 to 4096 keys, degrees 1 to 4) none takes over 1.04 times as long in
-    the batch where this is true, 180 do where it is not.
+    another. A batch repeats order 0 for every node; it gains where a node's launch alone leaves the chip idle. Of 2090
+    shapes (1 to 1024 heads, 1 to 1024 queries, 16 to 4096 keys, degrees 1 to 5) none takes over 1.04 times as long in
+    the batch where this is true; 314 take less than 0.93 times where it is not.
 
     * Launch-bound: below 3e8 multiply-adds, 32 MB of operands and 2048 workgroups (a head of 64 x 64 at degree 2: 217 and 108 us).
     * A workgroup takes a head and 64 queries. Below 512, two a CU, the float32 kernel for series over whole 16-key
@@ -236,6 +236,11 @@ def _stacks_nodes(query, key, value, attn_mask, is_causal, degree):
       ones (64 of 1024, d 128, causal, degree 2: 2940 and 3181; 1800 of 64, d 32, degree 2: 336 and 357). The other kernel shares few workgroups' keys out over the chip by itself, below 128 (1 head of 1024, d
       128, float64, degree 3: 915 and 1554 us), and needs the batch from there on, past degree 1 (8 heads of 1024,
       d 32, causal, float64, degree 3: 2560 and 740).
+    * Under the causal rule that kernel's parts of the keys lie partly past the diagonal, and the batch gains on either
+      side of that range as well with heads of up to 64 (16 of 361, d 64, float64, degree 2: 355 and 294), but not
+      where it comes to 128 to 255 workgroups itself, whole rows of keys on half the chip (8 of 512, degree 1: 155 and
+      245); from 256 workgroups
+      on, heads of some length alone (48 of 361, degree 2: 807 and 663).
     """
     q, k = (x.coeffs[0] if isinstance(x, PolyTensor) else x for x in (query, key))   # (a wrapper's attributes cost a call each)
     *lead, L, d = q.shape
@@ -254,6 +259,8 @@ def _stacks_nodes(query, key, value, attn_mask, is_causal, degree):
             and (attn_mask is None or attn_mask.dtype == torch.bool)):
         return workgroups < 512 or (d <= 32 and degree >= 2 and L >= 256) or (d <= 64 and degree >= 3 and L >= 512 and
                                                                               bool(is_causal))
+    if is_causal and attn_mask is None and L == S and d <= 64:
+        return not 128 <= workgroups * (degree + 1) < 256 and (workgroups < 256 or (workgroups < 512 and L >= 256))
     return degree >= 2 and 128 <= workgroups < 256
 
 

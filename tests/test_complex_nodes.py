@@ -65,6 +65,19 @@ def test_attention_nodes_in_one_launch_by_kernel():
     assert stacks(q, k, v, None, True, 3) and not stacks(q, k, v, None, False, 3)
 
 
+# Causal calls of the kernel that shares few workgroups' keys out over the chip: the batch's own workgroups count too.
+@pytest.mark.parametrize("heads,T,d,degree,one_launch", [
+    (16, 361, 64, 2, True), (8, 361, 64, 2, False), (8, 512, 64, 1, False), (16, 512, 64, 1, True),
+    (48, 512, 64, 2, True), (64, 512, 64, 2, False), (1, 1024, 128, 3, False)])
+def test_causal_attention_nodes_in_one_launch(heads, T, d, degree, one_launch):
+    q, k, v = (_direction((heads, T, d), degree, torch.float64) for _ in range(3))
+    assert _fused_attention._stacks_nodes(q, k, v, None, True, degree) is one_launch
+    # a mask beside the causal rule becomes one mask: the rule of masked calls
+    keep = torch.ones(T, T, dtype=torch.bool)
+    assert (_fused_attention._stacks_nodes(q, k, v, keep, True, degree)
+            is _fused_attention._stacks_nodes(q, k, v, keep, False, degree))
+
+
 @pytest.mark.parametrize("degree,numel,dtype,one_pass", [
     (1, 1 << 21, torch.float64, True), (1, (1 << 21) + 1, torch.float64, False), (2, 1 << 24, torch.float64, True),
     (1, 1 << 24, torch.float32, True), (9, 4, torch.float32, False)])
